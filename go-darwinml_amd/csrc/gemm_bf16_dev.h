@@ -74,6 +74,9 @@ struct GemmParams {
   void* c_g[4];
   // Slices of 2 GiB or more (the BIG instantiations): their byte extents.
   int64_t a_extent64, b_extent64;
+  // Register-staged cores: leading k-tiles whose chunks are whole 16-byte loads
+  // (gemm_fast_ktiles).
+  int k_fast;
 };
 constexpr int kGemmMaxGroups = 4;
 
@@ -84,6 +87,21 @@ constexpr int kGemmMaxGroups = 4;
 __host__ __device__ inline bool gemm_rows_fit(int64_t s_mn, int64_t s_k, int64_t es) {
   const int64_t s = s_mn > s_k ? s_mn : s_k;
   return s >= 0 && (s * 256 + 256) * es < (int64_t{1} << 31);
+}
+
+// k-tiles (of BK steps) that a register-staged core may load as whole 16-byte chunks
+// without a bounds check, from one operand: CE elements a chunk, MN rows or columns,
+// k stride s_k.  K-contiguous operands: every whole tile.  MN-contiguous ones read
+// whole chunks past the last column of a k-row, which stay inside the operand's
+// slice (its last element is (K - 1) s_k + MN - 1) for all but the last k-rows.
+__host__ __device__ inline int gemm_fast_ktiles(bool k_contig, int64_t MN, int64_t K, int64_t s_k, int BK, int CE) {
+  const int64_t whole = K / BK;
+  const int64_t over = (MN + CE - 1) / CE * CE - MN;  // elements read past a k-row's end
+  if (k_contig || over == 0) return static_cast<int>(whole);
+  if (s_k <= 0) return 0;
+  // k-row r is readable when r s_k + MN + over <= (K - 1) s_k + MN.
+  const int64_t rows = K - (over + s_k - 1) / s_k;
+  return rows <= 0 ? 0 : static_cast<int>(rows / BK < whole ? rows / BK : whole);
 }
 
 #if !defined(__HIPCC_RTC__)
@@ -134,9 +152,49 @@ inline GemmSplit gemm_k_split(int64_t batch, int64_t M, int64_t N, int64_t K, in
   }
   return r;
 }
+// Grids of at most this many 128 x 128 tiles run 64 x 64 tiles of the register-staged
+// core instead (any layout): four times the workgroups, each with four k-tiles of
+// loads in flight.  Graph-replayed, us, 128 x 128 DMA core / 64 x 64: bf16 [256,512,256]
+// 5.8 / 4.3, [512,512,512] 8.0 / 5.4, [1024,1024,1024] 12.6 / 8.1, [1024,2048,1024] (128
+// tiles) 12.8 / 11.3, but 14.2 / 14.8 at 144 tiles and 14.6 / 18.8 at 256; fp32, bound
+// by a CU's MFMA rate, [256,512,256] 20.9 / 8.2, [1024,1024,256] 21.8 / 9.4,
+// [1536,2048,512] (192 tiles) 40.2 / 32.4, 270 / 277 at 224 tiles.
+inline bool gemm_small_tiles(int64_t batch, int64_t M, int64_t N, int es) {
+  return batch * ((M + 127) / 128) * ((N + 127) / 128) <= (es == 4 ? 192 : 128);
+}
+// Whether a product that gemm_k_split would split runs as its split: not where the
+// 64 x 64 tiles, unsplit, are modelled at less than 0.8 of the split's cost.  Their
+// cost: one round of 256 tiles ~2.4 us + 4.6 ns a contraction step (fp32 3 + 20.9),
+// two rounds ~4 + 8.3 (4 + 37); measured, us, split / 64 x 64 tiles: bf16 [256,4096,2048]
+// 20.9 / 12.2, [1024,1024,2048] 21.1 / 12.3, [256,4096,4096] 23.4 / 21.4, and the split
+// kept at [128,4096,4096] 17.6 / 20.4, [512,512,4096] 15.6 / 20.0, [1024,2048,4096]
+// 31.8 / 32.8; fp32 [256,4096,1024] 35.5 / 25.4.  At most 64 rows (decoding, weights
+// from HBM): always the split, whose ranges keep more loads in flight.
+inline bool gemm_uses_split(int64_t batch, int64_t M, int64_t N, int64_t K, int es) {
+  const GemmSplit sp = gemm_k_split(batch, M, N, K, es);
+  if (sp.s <= 1) return false;
+  if (M <= 64 || !gemm_small_tiles(batch, M, N, es)) return true;
+  const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
+  const double k = static_cast<double>(K);
+  const double c64 = es == 4 ? (t64 <= 256 ? 3.0 + 0.0209 * k : 4.0 + 0.037 * k)
+                             : (t64 <= 256 ? 2.4 + 0.0046 * k : 4.0 + 0.0083 * k);
+  const double step_us = es == 4 ? 0.065 : 0.0146;
+  const double split_us = 4.0 + static_cast<double>(sp.kc) * step_us + static_cast<double>(sp.s) * M * N * 8 / 3e6;
+  return c64 >= 0.8 * split_us;
+}
 // Workspace bytes of a split (0 for s = 1): s fp32 partial products [M, N].
 inline int64_t gemm_split_bytes(const GemmSplit& sp, int64_t M, int64_t N) {
   return sp.s > 1 ? static_cast<int64_t>(sp.s) * M * N * 4 : 0;
+}
+// Operand majorness for the register-staged cores, which take any element alignment.
+inline int rs_majorness(int64_t s_mn, int64_t s_k, int64_t MN, int64_t K) {
+  if (s_k == 1 || K == 1) return 1;
+  return s_mn == 1 || MN == 1 ? 0 : -1;
+}
+inline bool rs_fits(const GemmParams& p, int es) {
+  return p.K > 0 && p.sa_m >= 0 && p.sa_k >= 0 && p.sb_n >= 0 && p.sb_k >= 0 && p.sa_b >= 0 && p.sb_b >= 0 &&
+         gemm_rows_fit(p.sa_m, p.sa_k, es) && gemm_rows_fit(p.sb_n, p.sb_k, es) &&
+         rs_majorness(p.sa_m, p.sa_k, p.M, p.K) >= 0 && rs_majorness(p.sb_n, p.sb_k, p.N, p.K) >= 0;
 }
 #endif
 
@@ -196,6 +254,13 @@ __device__ __forceinline__ int swz_k(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 // by 16 lanes of a transpose read, and the 4 x 64 bytes read by 32 lanes, land
 // in distinct bank groups.
 __device__ __forceinline__ int swz_n(int k) { return (0xCA60u >> ((k & 3) * 4)) & 15u; }
+// The same for a tile of R columns: a row of R = 64 is 8 chunks, two k-rows to a
+// 256-byte bank period, so the odd pairs of k-rows swap their halves.
+template <int R>
+__device__ __forceinline__ int swz_mn(int k) {
+  if constexpr (R >= 128) return swz_n(k);
+  else return ((k >> 1) & 1) << 2;
+}
 // Variant for 16x16x32 fragments, whose transpose reads cover k-rows k..k+3 and
 // k+8..k+11 of the same 16 columns in one half-wave: bit 3 of k also flips bit 1 of
 // the slot, so those 8 row pieces (2 chunks each) fill all 16 slots of a 256-byte
@@ -397,7 +462,7 @@ template <int R>
 __device__ __forceinline__ bf16x8_t frag_mn(const uint16_t* lds, int nbase, int s, int lane) {
   const int kl = 16 * s + 8 * (lane >> 5) + ((lane & 15) >> 2);
   const int nl = nbase + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  const uint16_t* p0 = lds + kl * R + (((nl >> 3) ^ swz_n(kl)) * 8) + (nl & 7);
+  const uint16_t* p0 = lds + kl * R + (((nl >> 3) ^ swz_mn<R>(kl)) * 8) + (nl & 7);
   const uint16_t* p1 = p0 + 4 * R;  // k + 4 keeps k & 3, hence the swizzle
   bf16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((GHIP_LDS bf16x4_t*)(p0));
   bf16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((GHIP_LDS bf16x4_t*)(p1));
@@ -714,6 +779,216 @@ __device__ __forceinline__ void gemm_bf16_body(const GemmParams& p, const Epi& e
   tile_epilogue<BM, BN, WM, WN, NB>(p, epi, smem, acc, bb, m0, n0, mn_full, lane, wm, wn);
 }
 
+
+// ---------------------------------------------------------------------------
+// Register-staged tiles: global -> VGPR -> LDS, for operands that the LDS DMA
+// cannot address (rows, columns or strides that are not whole 16-byte chunks) and
+// for grids of few tiles.  A chunk is one 16-byte load at element alignment
+// (ES bytes; gfx950 global loads need no more), so odd sizes move as many bytes per
+// instruction as aligned ones; only the k-tiles past GemmParams::k_fast read element
+// by element, with zeros beyond K.  Rows / columns past the operand's end re-read
+// valid ones: they only reach outputs that are never stored.
+// R rows x BK = 128 / ES k per tile, 256 threads.
+// ---------------------------------------------------------------------------
+typedef uint32_t u32x4_a2_t __attribute__((ext_vector_type(4), aligned(2), may_alias));
+typedef uint32_t u32x4_a4_t __attribute__((ext_vector_type(4), aligned(4), may_alias));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4), may_alias));
+template <int ES>
+struct RsElem {
+  using E = uint32_t;
+  using V = u32x4_a4_t;
+};
+template <>
+struct RsElem<2> {
+  using E = uint16_t;
+  using V = u32x4_a2_t;
+};
+
+template <int ES, int R, bool KC>
+struct RsTile {
+  using E = typename RsElem<ES>::E;
+  static constexpr int CE = 16 / ES, BK = 128 / ES;
+  static constexpr int NC = R / 32;                 // chunks per thread
+  static constexpr int CPR = KC ? 8 : R / CE;       // chunks per LDS row
+  static_assert(R % 32 == 0 && 256 % CPR == 0, "even share of chunks");
+  uint32_t voff[NC];  // byte offset of the thread's chunks from the tile's base
+  int valid;          // MN tiles: columns of the thread's chunk column inside the operand
+  int64_t s_k;
+
+  __device__ __forceinline__ static int lds_row(int i, int t) { return (i * 256 + t) / CPR; }
+  __device__ __forceinline__ void init(int t, int64_t mn_left, int64_t s_mn, int64_t sk) {
+    s_k = sk;
+    valid = 0;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int r = lds_row(i, t), c = t % CPR;
+      if constexpr (KC) {
+        const int64_t row = r < mn_left ? r : mn_left - 1;
+        voff[i] = static_cast<uint32_t>((row * s_mn + c * CE) * ES);
+      } else {
+        const int64_t left = mn_left - c * CE;
+        valid = left >= CE ? CE : left > 0 ? static_cast<int>(left) : 0;
+        voff[i] = static_cast<uint32_t>((r * sk + (left > 0 ? c * CE : 0)) * ES);
+      }
+    }
+  }
+  // Tile kt from `base` (the operand at the tile's first row / column, k = 0).
+  __device__ __forceinline__ void load(const E* base, int kt, u32x4_t (&v)[NC]) const {
+    const char* src = reinterpret_cast<const char*>(base + static_cast<int64_t>(kt) * BK * (KC ? 1 : s_k));
+#pragma unroll
+    for (int i = 0; i < NC; ++i) v[i] = *reinterpret_cast<const typename RsElem<ES>::V*>(src + voff[i]);
+  }
+  // A tile with steps past K or whole chunks past the slice's end: element loads, each
+  // from a valid element (no exec-masked load, so all are in flight at once), zeroed
+  // where the tile's element lies outside the operand.
+  __device__ __forceinline__ void load_edge(const E* base, int kt, int64_t K, int t, u32x4_t (&v)[NC]) const {
+    const E* src = base + static_cast<int64_t>(kt) * BK * (KC ? 1 : s_k);
+    const int64_t left = K - static_cast<int64_t>(kt) * BK;
+    const int k_left = static_cast<int>(left < BK ? left : BK);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int c = t % CPR, kr = lds_row(i, t);
+      // Row start (K-contiguous) or valid k-row of the tile, and the chunk's valid length.
+      const E* q = KC ? src + (voff[i] / ES - c * CE) : src + (kr < k_left ? voff[i] / ES : 0);
+      const int n = KC ? k_left - c * CE : (kr < k_left ? valid : 0);
+      E e[CE];
+#pragma unroll
+      for (int j = 0; j < CE; ++j) e[j] = q[j < n ? (KC ? c * CE : 0) + j : 0];
+      uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int j = 0; j < CE; ++j) w[j * ES / 4] |= (j < n ? static_cast<uint32_t>(e[j]) : 0u) << (j * ES % 4 * 8);
+      v[i] = u32x4_t{w[0], w[1], w[2], w[3]};
+    }
+  }
+  // LDS layouts of OperandTile (16-bit) and TileF32 (fp32).
+  __device__ __forceinline__ void store(E* lds, int t, const u32x4_t (&v)[NC]) const {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int r = lds_row(i, t), c = t % CPR;
+      const int slot = KC ? (ES == 2 ? c ^ swz_k(r) : c ^ (r & 7)) : (ES == 2 ? c ^ swz_mn<R>(r) : c);
+      *reinterpret_cast<u32x4_t*>(lds + (r * CPR + slot) * CE) = v[i];
+    }
+  }
+};
+
+// The k loop of a register-staged core: the KF whole tiles with PD of them in flight
+// in registers ahead of two LDS stages, one barrier a tile, then the edge tiles (one
+// or two) as they come; compute(stage) runs a staged tile's MFMAs.
+template <int PD, class TA, class TB, class E, class F>
+__device__ __forceinline__ void rs_main_loop(const TA& ta, const TB& tb, const E* A, const E* B, int64_t K, int KT,
+                                             int KF, E* sa, E* sb, int sa_elems, int sb_elems, F compute) {
+  static_assert(PD % 2 == 0, "a tile's LDS stage is the parity of its register set");
+  const int t = threadIdx.x;
+  u32x4_t va[PD][TA::NC], vb[PD][TB::NC];
+  auto load = [&](int kt, int d) {
+    ta.load(A, kt, va[d]);
+    tb.load(B, kt, vb[d]);
+  };
+  auto store = [&](int st, int d) {
+    ta.store(sa + st * sa_elems, t, va[d]);
+    tb.store(sb + st * sb_elems, t, vb[d]);
+  };
+  if (KF > 0) {
+#pragma unroll
+    for (int d = 0; d < PD; ++d)
+      if (d < KF) load(d, d);
+    store(0, 0);
+    if (PD < KF) load(PD, 0);
+    __syncthreads();
+    // Tile kt + u lives in stage u & 1 and came through register set u.
+    int kt = 0;
+    for (; kt + 2 * PD < KF; kt += PD) {
+#pragma unroll
+      for (int u = 0; u < PD; ++u) {
+        store((u & 1) ^ 1, (u + 1) % PD);
+        load(kt + u + 1 + PD, (u + 1) % PD);
+        compute(u & 1);
+        __syncthreads();
+      }
+    }
+    for (; kt < KF; kt += PD) {
+#pragma unroll
+      for (int u = 0; u < PD; ++u) {
+        if (kt + u >= KF) break;
+        if (kt + u + 1 < KF) store((u & 1) ^ 1, (u + 1) % PD);
+        if (kt + u + 1 + PD < KF) load(kt + u + 1 + PD, (u + 1) % PD);
+        compute(u & 1);
+        __syncthreads();
+      }
+    }
+  }
+  for (int kt = KF; kt < KT; ++kt) {
+    const int st = kt & 1;
+    ta.load_edge(A, kt, K, t, va[0]);
+    tb.load_edge(B, kt, K, t, vb[0]);
+    store(st, 0);
+    __syncthreads();
+    compute(st);
+  }
+}
+
+// 16-bit operands, one BM x BN tile per workgroup of 2 x 2 waves; same MFMA and k
+// order per accumulator as the other cores (the same bits).  p.a / p.b at any element
+// alignment, non-negative strides, rows within gemm_rows_fit.  Bound by the latency of
+// a tile's loads where the grid is small (hence four k-tiles in flight for 64 x 64
+// tiles), else by the extra VGPR round trip: [2048,2048,2048] 26 us against the DMA
+// core's 27-30.  [1000,1531] . [1531,776] with bias and GELU in the epilogue: 181 us
+// on the scalar kernel that such operands took before, 15.2 here.
+template <int BM, int BN, bool A_K, bool B_K, class Epi, bool F16 = false>
+__device__ __forceinline__ void gemm_bf16_body_rs(const GemmParams& p, const Epi& epi) {
+  constexpr int WM = 2, WN = 2;
+  constexpr int TM = BM / WM, TN = BN / WN;
+  constexpr int FM = TM / 32, FN = TN / 32;
+  constexpr int PD = BM * BN <= 64 * 64 ? 4 : 2;
+  using TA = RsTile<2, BM, A_K>;
+  using TB = RsTile<2, BN, B_K>;
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[2 * (BM + BN) * kBK];
+  uint16_t* sa = smem;
+  uint16_t* sb = smem + 2 * BM * kBK;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  int64_t bb;
+  int tm, tn;
+  map_tile(blockIdx.x, p.batch * p.tiles_m * p.tiles_n, p.tiles_m, p.tiles_n, bb, tm, tn);
+  const int64_t m0 = static_cast<int64_t>(tm) * BM, n0 = static_cast<int64_t>(tn) * BN;
+  const uint16_t* A = static_cast<const uint16_t*>(p.a) + bb * p.sa_b + m0 * p.sa_m;
+  const uint16_t* B = static_cast<const uint16_t*>(p.b) + bb * p.sb_b + n0 * p.sb_n;
+  TA ta;
+  TB tb;
+  ta.init(threadIdx.x, p.M - m0, p.sa_m, p.sa_k);
+  tb.init(threadIdx.x, p.N - n0, p.sb_n, p.sb_k);
+
+  f32x16_t acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  auto compute = [&](int st) {
+    const uint16_t* As = sa + st * BM * kBK;
+    const uint16_t* Bs = sb + st * BN * kBK;
+#pragma unroll
+    for (int s = 0; s < kBK / 16; ++s) {
+      bf16x8_t fa[FM], fb[FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+        fa[i] = A_K ? frag_kc(As, wm * TM + i * 32, s, lane) : frag_mn<BM>(As, wm * TM + i * 32, s, lane);
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+        fb[j] = B_K ? frag_kc(Bs, wn * TN + j * 32, s, lane) : frag_mn<BN>(Bs, wn * TN + j * 32, s, lane);
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = mma16<F16>(fb[j], fa[i], acc[i][j]);
+    }
+  };
+  rs_main_loop<PD>(ta, tb, A, B, p.K, static_cast<int>((p.K + kBK - 1) / kBK), p.k_fast, sa, sb, BM * kBK, BN * kBK,
+                   compute);
+  tile_epilogue<BM, BN, WM, WN, 1>(p, epi, smem, acc, bb, m0, n0, m0 + BM <= p.M && n0 + BN <= p.N, lane, wm, wn);
+}
 
 // 4-wave core for both operands MN-contiguous (A [K, M], B [K, N] in memory, e.g.
 // a weight gradient X^T . dY): one 256 x 256 tile per workgroup of 2 x 2 waves, each

@@ -39,9 +39,11 @@ struct StoreEpi16 {
   __device__ __forceinline__ void store(int64_t bb, int64_t m, int64_t n, const Stage* v, const Stage*,
                                         const Pre&) const {
     uint16_t* dst = reinterpret_cast<uint16_t*>(c + bb * sc_b + m * sc_m + n);
-    if (vec && (FULL || n + 7 < N)) {
-      *reinterpret_cast<uint4*>(dst) = make_uint4(v[0] | (uint32_t(v[1]) << 16), v[2] | (uint32_t(v[3]) << 16),
-                                                 v[4] | (uint32_t(v[5]) << 16), v[6] | (uint32_t(v[7]) << 16));
+    if (FULL || n + 7 < N) {
+      const u32x4_t w = {v[0] | (uint32_t(v[1]) << 16), v[2] | (uint32_t(v[3]) << 16), v[4] | (uint32_t(v[5]) << 16),
+                         v[6] | (uint32_t(v[7]) << 16)};
+      if (vec) *reinterpret_cast<u32x4_t*>(dst) = w;
+      else *reinterpret_cast<u32x4_a2_t*>(dst) = w;  // one store at element alignment
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
@@ -67,8 +69,10 @@ struct StoreEpi<float> {
   __device__ __forceinline__ void store(int64_t bb, int64_t m, int64_t n, const Stage* v, const Stage*,
                                         const Pre&) const {
     float* dst = c + bb * sc_b + m * sc_m + n;
-    if (vec && (FULL || n + 3 < N)) {
-      *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+    if (FULL || n + 3 < N) {
+      const u32x4_t w = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+      if (vec) *reinterpret_cast<u32x4_t*>(dst) = w;
+      else *reinterpret_cast<u32x4_a4_t*>(dst) = w;  // one store at element alignment
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -86,6 +90,13 @@ __device__ __forceinline__ StoreEpi<OutT> store_epi(const GemmParams& p) {
   e.N = p.N;
   e.vec = p.vec_c;
   return e;
+}
+
+// Register-staged core (any element alignment).
+template <int BM, int BN, bool A_K, bool B_K, typename InT, typename OutT>
+__global__ __launch_bounds__(256, 2) void gemm_bf16_rs_kernel(GemmParams p) {
+  const StoreEpi<OutT> epi = store_epi<OutT>(p);
+  gemm_bf16_body_rs<BM, BN, A_K, B_K, StoreEpi<OutT>, __is_same(InT, f16_t)>(p, epi);
 }
 
 // 16-bit inputs: bf16, or f16 (InT = f16_t selects the f16 MFMA).
@@ -214,6 +225,79 @@ __device__ __forceinline__ float f4_at(const float4& v, int e) {
   return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w;
 }
 
+// One 32-deep k-tile's MFMAs from its LDS tiles.
+template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, int FM, int FN>
+__device__ __forceinline__ void f32_tile_mma(const float* As, const float* Bs, int wm, int wn, int lane,
+                                             f32x16_t (&acc)[FM][FN]) {
+  constexpr int TM = BM / WM, TN = BN / WN;
+#pragma unroll
+  for (int g = 0; g < kBK32 / 8; ++g) {
+    float4 a4[FM], b4[FN];
+    if constexpr (A_K) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) a4[i] = frag_f32_kc(As, wm * TM + i * 32, g, lane);
+    }
+    if constexpr (B_K) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) b4[j] = frag_f32_kc(Bs, wn * TN + j * 32, g, lane);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float af[FM], bf[FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+        af[i] = A_K ? f4_at(a4[i], e) : frag_f32_mn<BM>(As, wm * TM + i * 32, g, e, lane);
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+        bf[j] = B_K ? f4_at(b4[j], e) : frag_f32_mn<BN>(Bs, wn * TN + j * 32, g, e, lane);
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bf[j], af[i], acc[i][j], 0, 0, 0);
+    }
+  }
+}
+
+// Output of an fp32 core.
+template <int BM, int BN, int WM, int WN, typename OutT, int FM, int FN>
+__device__ __forceinline__ void f32_tile_store(const GemmParams& p, int64_t bb, int64_t m0, int64_t n0, int wm, int wn,
+                                               int lane, const f32x16_t (&acc)[FM][FN]) {
+  constexpr int TM = BM / WM, TN = BN / WN;
+  // acc[i][j]: lane l, value v -> row m = l % 32 of block i, columns
+  // n = (v / 4) * 8 + (l / 32) * 4 + v % 4 of block j.
+  OutT* C = static_cast<OutT*>(p.c) + bb * p.sc_b;
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int64_t m = m0 + wm * TM + i * 32 + (lane & 31);
+    if (m >= p.M) continue;
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t n = n0 + wn * TN + j * 32 + q * 8 + (lane >> 5) * 4;
+        if (n >= p.N) continue;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][q * 4 + e];
+        OutT* dst = C + m * p.sc_m + n;
+        if (p.vec_c && n + 3 < p.N) {
+          if constexpr (sizeof(OutT) == 2)
+            *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+          else
+            *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+        } else if (sizeof(OutT) == 4 && n + 3 < p.N) {  // one store at element alignment
+          *reinterpret_cast<u32x4_a4_t*>(dst) = u32x4_t{__float_as_uint(v[0]), __float_as_uint(v[1]),
+                                                         __float_as_uint(v[2]), __float_as_uint(v[3])};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < p.N) store_out<OutT>(dst + e, v[e]);
+        }
+      }
+  }
+}
+
 template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, typename OutT, bool BIG = false>
 __global__ __launch_bounds__(WM* WN * 64, (WM * WN == 4 ? 2 : 1)) void gemm_f32_kernel(GemmParams p) {
   constexpr int NW = WM * WN;
@@ -266,35 +350,7 @@ __global__ __launch_bounds__(WM* WN * 64, (WM * WN == 4 ? 2 : 1)) void gemm_f32_
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
   auto compute = [&](int st) {
-    const float* As = &smem[st][0];
-    const float* Bs = &smem[st][SA];
-#pragma unroll
-    for (int g = 0; g < kBK32 / 8; ++g) {
-      float4 a4[FM], b4[FN];
-      if constexpr (A_K) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i) a4[i] = frag_f32_kc(As, wm * TM + i * 32, g, lane);
-      }
-      if constexpr (B_K) {
-#pragma unroll
-        for (int j = 0; j < FN; ++j) b4[j] = frag_f32_kc(Bs, wn * TN + j * 32, g, lane);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float af[FM], bf[FN];
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-          af[i] = A_K ? f4_at(a4[i], e) : frag_f32_mn<BM>(As, wm * TM + i * 32, g, e, lane);
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          bf[j] = B_K ? f4_at(b4[j], e) : frag_f32_mn<BN>(Bs, wn * TN + j * 32, g, e, lane);
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bf[j], af[i], acc[i][j], 0, 0, 0);
-      }
-    }
+    f32_tile_mma<BM, BN, WM, WN, A_K, B_K>(&smem[st][0], &smem[st][SA], wm, wn, lane, acc);
   };
 
   // Prologue: tiles 0 and 1 in flight, wait for tile 0.
@@ -315,35 +371,48 @@ __global__ __launch_bounds__(WM* WN * 64, (WM * WN == 4 ? 2 : 1)) void gemm_f32_
     if (kt + 2 < KT) issue(kt + 2, st);
   }
 
-  // acc[i][j]: lane l, value v -> row m = l % 32 of block i, columns
-  // n = (v / 4) * 8 + (l / 32) * 4 + v % 4 of block j.
-  OutT* C = static_cast<OutT*>(p.c) + bb * p.sc_b;
+  f32_tile_store<BM, BN, WM, WN, OutT>(p, bb, m0, n0, wm, wn, lane, acc);
+}
+
+// Register-staged fp32 core (RsTile, rs_main_loop): any element alignment, 64 x 64
+// or 128 x 128 tiles of 2 x 2 waves; same MFMA and k order as gemm_f32_kernel (the
+// same bits).
+template <int BM, int BN, bool A_K, bool B_K, typename OutT>
+__global__ __launch_bounds__(256, 2) void gemm_f32_rs_kernel(GemmParams p) {
+  constexpr int WM = 2, WN = 2;
+  constexpr int FM = BM / 64, FN = BN / 64;
+  constexpr int PD = BM * BN <= 64 * 64 ? 4 : 2;
+  using TA = RsTile<4, BM, A_K>;
+  using TB = RsTile<4, BN, B_K>;
+  __shared__ __attribute__((aligned(1024))) float smem[2 * (BM + BN) * kBK32];
+  float* sa = smem;
+  float* sb = smem + 2 * BM * kBK32;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  int64_t bb;
+  int tm, tn;
+  map_tile(blockIdx.x, p.batch * p.tiles_m * p.tiles_n, p.tiles_m, p.tiles_n, bb, tm, tn);
+  const int64_t m0 = static_cast<int64_t>(tm) * BM, n0 = static_cast<int64_t>(tn) * BN;
+  const uint32_t* A = static_cast<const uint32_t*>(p.a) + bb * p.sa_b + m0 * p.sa_m;
+  const uint32_t* B = static_cast<const uint32_t*>(p.b) + bb * p.sb_b + n0 * p.sb_n;
+  TA ta;
+  TB tb;
+  ta.init(threadIdx.x, p.M - m0, p.sa_m, p.sa_k);
+  tb.init(threadIdx.x, p.N - n0, p.sb_n, p.sb_k);
+  f32x16_t acc[FM][FN];
 #pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    const int64_t m = m0 + wm * TM + i * 32 + (lane & 31);
-    if (m >= p.M) continue;
+  for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int64_t n = n0 + wn * TN + j * 32 + q * 8 + (lane >> 5) * 4;
-        if (n >= p.N) continue;
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][q * 4 + e];
-        OutT* dst = C + m * p.sc_m + n;
-        if (p.vec_c && n + 3 < p.N) {
-          if constexpr (sizeof(OutT) == 2)
-            *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-          else
-            *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < p.N) store_out<OutT>(dst + e, v[e]);
-        }
-      }
-  }
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  auto compute = [&](int st) {
+    f32_tile_mma<BM, BN, WM, WN, A_K, B_K>(sa + st * BM * kBK32, sb + st * BN * kBK32, wm, wn, lane, acc);
+  };
+  rs_main_loop<PD>(ta, tb, A, B, p.K, static_cast<int>((p.K + kBK32 - 1) / kBK32), p.k_fast,
+                   reinterpret_cast<uint32_t*>(sa), reinterpret_cast<uint32_t*>(sb), BM * kBK32, BN * kBK32, compute);
+  f32_tile_store<BM, BN, WM, WN, OutT>(p, bb, m0, n0, wm, wn, lane, acc);
 }
 
 // The 256 x 256 cores (grids of >= 128 tiles).  BIG: the 64-bit-records
@@ -372,6 +441,41 @@ hipError_t launch_f32(GemmParams p, bool a_k, bool b_k, hipStream_t s) {
   return hipGetLastError();
 }
 
+// T x T tiles of a register-staged core (instantiated in k_gemm_rs.hip).
+template <int T, typename InT, typename OutT>
+hipError_t launch_rs_tile(GemmParams p, hipStream_t s) {
+  constexpr int ES = sizeof(InT), BK = 128 / ES, CE = 16 / ES;
+  const bool a_k = rs_majorness(p.sa_m, p.sa_k, p.M, p.K) == 1, b_k = rs_majorness(p.sb_n, p.sb_k, p.N, p.K) == 1;
+  const int fa = gemm_fast_ktiles(a_k, p.M, p.K, p.sa_k, BK, CE), fb = gemm_fast_ktiles(b_k, p.N, p.K, p.sb_k, BK, CE);
+  p.k_fast = fa < fb ? fa : fb;
+  p.tiles_m = static_cast<int>((p.M + T - 1) / T);
+  p.tiles_n = static_cast<int>((p.N + T - 1) / T);
+  const dim3 grid(static_cast<unsigned>(p.batch * p.tiles_m * p.tiles_n)), block(256);
+  if constexpr (ES == 4) {
+    if (a_k && b_k) hipLaunchKernelGGL((gemm_f32_rs_kernel<T, T, true, true, OutT>), grid, block, 0, s, p);
+    else if (a_k) hipLaunchKernelGGL((gemm_f32_rs_kernel<T, T, true, false, OutT>), grid, block, 0, s, p);
+    else if (b_k) hipLaunchKernelGGL((gemm_f32_rs_kernel<T, T, false, true, OutT>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((gemm_f32_rs_kernel<T, T, false, false, OutT>), grid, block, 0, s, p);
+  } else {
+    if (a_k && b_k) hipLaunchKernelGGL((gemm_bf16_rs_kernel<T, T, true, true, InT, OutT>), grid, block, 0, s, p);
+    else if (a_k) hipLaunchKernelGGL((gemm_bf16_rs_kernel<T, T, true, false, InT, OutT>), grid, block, 0, s, p);
+    else if (b_k) hipLaunchKernelGGL((gemm_bf16_rs_kernel<T, T, false, true, InT, OutT>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((gemm_bf16_rs_kernel<T, T, false, false, InT, OutT>), grid, block, 0, s, p);
+  }
+  return hipGetLastError();
+}
+extern template hipError_t launch_rs_tile<64, bf16_t, bf16_t>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<64, bf16_t, float>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<64, f16_t, f16_t>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<64, f16_t, float>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<64, float, float>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<64, float, bf16_t>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<128, bf16_t, bf16_t>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<128, bf16_t, float>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<128, f16_t, f16_t>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<128, f16_t, float>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<128, float, float>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<128, float, bf16_t>(GemmParams, hipStream_t);
 extern template hipError_t launch_bf16_4w<true, bf16_t, bf16_t>(GemmParams, bool, bool, hipStream_t);
 extern template hipError_t launch_bf16_4w<true, bf16_t, float>(GemmParams, bool, bool, hipStream_t);
 extern template hipError_t launch_bf16_4w<true, f16_t, f16_t>(GemmParams, bool, bool, hipStream_t);

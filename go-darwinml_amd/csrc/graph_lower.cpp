@@ -1799,7 +1799,7 @@ struct Lowerer {
     const int64_t M = d.M, N_ = d.N, K = d.K, sam = d.sam, sak = d.sak, sbk = d.sbk, sbn = d.sbn;
     // Products that split their contraction run one after another, sharing one
     // workspace in the arena.
-    const int64_t ws_bytes = ghip_gemm_workspace_bytes(dt, odt, 1, M, N_, K);
+    const int64_t ws_bytes = split_ws_bytes(dt, odt, 1, M, N_, K);
     const View wsv = gemm_workspace_view(ws_bytes, &wr);
     add_step(fmt("gemm_grouped %s G=%d M=%lld N=%lld K=%lld (products sharing a; a strides m=%lld k=%lld, b strides "
                  "k=%lld n=%lld%s)",
@@ -1839,7 +1839,7 @@ struct Lowerer {
     const int dt = N[n.in[0]].shape.dtype, odt = n.shape.dtype;
     const int64_t scb = M * N_, scm = N_;
     std::vector<int> wr{y.slot};
-    const int64_t ws_bytes = ghip_gemm_workspace_bytes(dt, odt, B, M, N_, K);
+    const int64_t ws_bytes = split_ws_bytes(dt, odt, B, M, N_, K);
     const View wsv = gemm_workspace_view(ws_bytes, &wr);
     add_step(fmt("gemm_batched %s B=%lld M=%lld N=%lld K=%lld (%s; a strides b=%lld m=%lld k=%lld, b strides b=%lld k=%lld n=%lld%s)",
                  dtype_name(dt), (long long)B, (long long)M, (long long)N_, (long long)K, d.how.c_str(), (long long)sab,
@@ -1863,6 +1863,11 @@ struct Lowerer {
     const View w = fresh(wss);
     wr->push_back(w.slot);
     return w;
+  }
+  // Workspace bytes of a GEMM step (0 unless it runs as its contraction split).
+  static int64_t split_ws_bytes(int dt, int odt, int64_t B, int64_t M, int64_t N_, int64_t K) {
+    return gemm_uses_split(B, M, N_, K, dt == GHIP_DTYPE_FLOAT32 ? 4 : 2)
+               ? ghip_gemm_workspace_bytes(dt, odt, B, M, N_, K) : 0;
   }
   static std::string split_note(int64_t ws_bytes, int64_t B, int64_t M, int64_t N_, int64_t K, int dt) {
     if (ws_bytes <= 0) return "";
@@ -2704,7 +2709,7 @@ bool Lowerer::emit_split_partials(int o, const Shape& os, const std::set<int>& i
   if (!plan_dot(o, false, &d)) return false;
   if (d.B != 1 || d.M <= 0 || d.N <= 0 || d.K <= 0) return false;
   const int64_t wsb = ghip_gemm_workspace_bytes(dt, odt, 1, d.M, d.N, d.K);
-  if (wsb <= 0 || d.sam < 0 || d.sak < 0 || d.sbk < 0 || d.sbn < 0) return false;
+  if (wsb <= 0 || !gemm_uses_split(1, d.M, d.N, d.K, 2) || d.sam < 0 || d.sak < 0 || d.sbk < 0 || d.sbn < 0) return false;
   if (mfma_majorness(d.lv.offset, 0, d.sam, d.sak, d.M, d.K, 1) < 0 ||
       mfma_majorness(d.rv.offset, 0, d.sbn, d.sbk, d.N, d.K, 1) < 0)
     return false;
@@ -2773,20 +2778,28 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   // A product the stand-alone GEMM step would run with its contraction split stays
   // unfused (the split's fp32 partials are summed by a kernel of their own, which
   // the generated epilogue kernel does not reproduce).
-  if (ghip_gemm_workspace_bytes(GHIP_DTYPE_BFLOAT16, N[dots[0]].shape.dtype, d.B, d.M, d.N, d.K) > 0) return View{};
+  if (gemm_uses_split(d.B, d.M, d.N, d.K, 2)) return View{};
   // The bf16 MFMA path's operand conditions, decided here because the fused
   // kernel has no generic fallback.
   if (d.B > 65535 || d.M == 0 || d.N == 0 || d.K == 0) return View{};
   if (d.sab < 0 || d.sam < 0 || d.sak < 0 || d.sbb < 0 || d.sbk < 0 || d.sbn < 0) return View{};
-  const int ma = mfma_majorness(d.lv.offset, d.sab, d.sam, d.sak, d.M, d.K, d.B);
+  int ma = mfma_majorness(d.lv.offset, d.sab, d.sam, d.sak, d.M, d.K, d.B);
   int mb = mfma_majorness(d.rv.offset, d.sbb, d.sbn, d.sbk, d.N, d.K, d.B);
   if (NB == 2 && mfma_majorness(dp[1].rv.offset, d.sbb, d.sbn, d.sbk, d.N, d.K, d.B) != mb) mb = -1;
+  // One product that the LDS DMA cannot address, or of few tiles: the register-staged
+  // core, as the stand-alone product (the same bits).
+  const bool dma_ok = ma >= 0 && mb >= 0;
+  const bool rs = NB == 1 && (!dma_ok || gemm_small_tiles(d.B, d.M, d.N, 2));
+  if (rs) {
+    ma = rs_majorness(d.sam, d.sak, d.M, d.K);
+    mb = rs_majorness(d.sbn, d.sbk, d.N, d.K);
+  }
   if (ma < 0 || mb < 0) return View{};
   const int64_t ea = ((d.M - 1) * d.sam + (d.K - 1) * d.sak + 1) * 2;
   const int64_t eb = ((d.N - 1) * d.sbn + (d.K - 1) * d.sbk + 1) * 2;
   if (!gemm_rows_fit(d.sam, d.sak, 2) || !gemm_rows_fit(d.sbn, d.sbk, 2)) return View{};
   // Operand slices of 2 GiB or more: the cores' 64-bit-records form (BIG).
-  const bool big = ea >= (int64_t{1} << 31) || eb >= (int64_t{1} << 31);
+  const bool big = !rs && (ea >= (int64_t{1} << 31) || eb >= (int64_t{1} << 31));
   const char* big_arg = big ? ", true" : "";
 
   // Extra operands: each must fold to one stride per (batch, m, n) group of the
@@ -2798,7 +2811,8 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
     View view;
     int dt;
     int64_t sb, sm, sn;
-    bool vin;  // 4-element vector loads: unit n stride, rows and base 4-element aligned
+    bool vin;  // vector loads of a chunk: unit n stride
+    bool al;   // its rows and base are whole chunks (else loaded at element alignment)
   };
   std::vector<In> ins;
   std::map<int, std::string> expr;
@@ -2830,11 +2844,12 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
       const int off = os.rank() - s.rank();
       for (int i = 0; i < s.rank(); ++i)
         if (s.dims[i] != 1) eff.strides[off + i] = w.strides[i];
-      In in{w, s.dtype, 0, 0, 0, false};
+      In in{w, s.dtype, 0, 0, 0, false, false};
       int64_t sz;
       if (!merge(os, eff, gb, &sz, &in.sb) || !merge(os, eff, gm, &sz, &in.sm) || !merge(os, eff, gn, &sz, &in.sn))
         return View{};
-      in.vin = in.sn == 1 && (in.sm % CH == 0 || d.M == 1) && (in.sb % CH == 0 || d.B == 1) && w.offset % CH == 0;
+      in.vin = in.sn == 1;
+      in.al = (in.sm % CH == 0 || d.M == 1) && (in.sb % CH == 0 || d.B == 1) && w.offset % CH == 0;
       const int k = static_cast<int>(ins.size());
       const std::string ks = std::to_string(k);
       body << "      const " << ctype(s.dtype) << " in" << ks << " = " << load_expr(s.dtype, "pr.x" + ks + "[e]") << ";\n";
@@ -2881,7 +2896,9 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   // leaves half the CUs or more idle).
   bool eight_km = false, eight_x = false, four_km = false;
   const int64_t t4 = d.B * ((d.M + 255) / 256) * ((d.N + 256 / NB - 1) / (256 / NB));
-  if (ma && !mb && d.M >= 256 && d.N >= 256 / NB && (NB == 2 || !heavy_epilogue) && (NB == 2 ? t4 >= 128 : t4 > 128)) {
+  if (rs) {
+    if (gemm_small_tiles(d.B, d.M, d.N, 2)) BM = BN = 64;
+  } else if (ma && !mb && d.M >= 256 && d.N >= 256 / NB && (NB == 2 || !heavy_epilogue) && (NB == 2 ? t4 >= 128 : t4 > 128)) {
     BM = 256, BN = 256 / NB, WM = 2, WN = 2, four_km = true;
   } else if (NB == 1) {
     if (d.M >= 256 && d.N >= 256 && t256 > 128 && ma && !mb) BM = 256, BN = 256, WM = 2, WN = 4, eight_km = true;
@@ -2916,7 +2933,8 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
         << "] + m * a.s_m[" << ks << "] + n * a.s_n[" << ks << "];\n";
     if (ins[k].vin)
       src << "      if (FULL || n + " << CH - 1 << " < a.N) {\n"
-          << "        struct __attribute__((aligned(" << vbytes << "))) V { " << T << " x[" << CHs << "]; };\n"
+          << "        struct __attribute__((" << (ins[k].al ? fmt("aligned(%d)", vbytes) : "packed") << ")) V { " << T
+          << " x[" << CHs << "]; };\n"
           << "        const V w = *(const V*)src;\n"
           << "#pragma unroll\n        for (int e = 0; e < " << CHs << "; ++e) pr.x" << ks << "[e] = w.x[e];\n"
           << "      } else {\n";
@@ -2935,10 +2953,11 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
       << body.str()
       << "      r[e] = " << expr[v] << ";\n    }\n"
       << "    " << stype(odt) << "* o = (" << stype(odt) << "*)a.out + bb * a.so_b + m * a.so_m + n;\n";
-  if (vec) {
+  {
     const int obytes = std::min(CH * dtype_size(odt), 16);
     src << "    if (FULL || n + " << CH - 1 << " < a.N) {\n"
-        << "      struct __attribute__((aligned(" << obytes << "))) V { " << stype(odt) << " x[" << CHs << "]; } w;\n"
+        << "      struct __attribute__((" << (vec ? fmt("aligned(%d)", obytes) : "packed") << ")) V { " << stype(odt)
+        << " x[" << CHs << "]; } w;\n"
         << "#pragma unroll\n      for (int e = 0; e < " << CHs << "; ++e) w.x[e] = " << store_expr(odt, "r[e]") << ";\n"
         << "      *(V*)o = w;\n      return;\n    }\n";
   }
@@ -2946,7 +2965,10 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
       << ";\n  }\n};\n}  // namespace ghip\n";
   src << "extern \"C\" __global__ void __launch_bounds__(" << nt << ", 1) gemm_epilogue(ghip::GemmParams p, ghip::EpiArgs a) {\n"
       << "  const ghip::GenEpi epi{a};\n";
-  if (four_km)
+  if (rs)
+    src << "  ghip::gemm_bf16_body_rs<" << BM << ", " << BN << ", " << (ma ? "true" : "false") << ", "
+        << (mb ? "true" : "false") << ", ghip::GenEpi>(p, epi);\n}\n";
+  else if (four_km)
     src << "  ghip::gemm_bf16_body4km<ghip::GenEpi, false, " << NB << big_arg << ">(p, epi);\n}\n";
   else if (eight_km)
     src << "  ghip::gemm_bf16_body8km<ghip::GenEpi, false, " << NB << big_arg << ">(p, epi);\n}\n";
@@ -2975,6 +2997,10 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   gp.b_extent = big ? 0u : static_cast<uint32_t>(eb);
   gp.a_extent64 = ea;
   gp.b_extent64 = eb;
+  if (rs) {
+    const int fa = gemm_fast_ktiles(ma == 1, d.M, d.K, d.sak, 64, 8), fb = gemm_fast_ktiles(mb == 1, d.N, d.K, d.sbk, 64, 8);
+    gp.k_fast = std::min(fa, fb);
+  }
   const int64_t blocks = d.B * gp.tiles_m * gp.tiles_n;
   const int64_t so_b = d.M * d.N, so_m = d.N;
   const View lv = d.lv, rv0 = d.rv, rv1 = dp[NB - 1].rv;
@@ -2983,7 +3009,7 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   for (auto& in : ins) rd.push_back(in.view.slot);
   std::ostringstream desc;
   // core: waves and k-depth of the main loop (km32: A in 64-deep, B in 32-deep stages)
-  const char* core = four_km ? "4w-km32" : eight_km ? "8w-km32" : eight_x ? "8w-k64" : four_wave ? "4w-mn32" : "small";
+  const char* core = four_km ? "4w-km32" : eight_km ? "8w-km32" : eight_x ? "8w-k64" : four_wave ? "4w-mn32" : rs ? "staged" : "small";
   desc << fmt("gemm_batched+epilogue bf16 B=%lld M=%lld N=%lld K=%lld dots=%d tile=%dx%d waves=%d core=%s (%s) ops=%zu "
               "inputs=%zu [",
               (long long)d.B, (long long)d.M, (long long)d.N, (long long)d.K, NB, BM, BN * NB, WM * WN, core,
@@ -3000,7 +3026,7 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
     p.b = st.ptr(rv0, GHIP_DTYPE_BFLOAT16);
     p.b1 = st.ptr(rv1, GHIP_DTYPE_BFLOAT16);
     p.c = st.ptr(y, odt);
-    if ((reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b) | reinterpret_cast<uintptr_t>(p.b1)) & 15u)
+    if (!rs && (reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b) | reinterpret_cast<uintptr_t>(p.b1)) & 15u)
       return set_error(e, GHIP_ERR_STATE, "fused GEMM epilogue: operand base not 16-byte aligned");
     EpiArgs a{};
     for (size_t k = 0; k < ins.size(); ++k) {
@@ -3011,7 +3037,7 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
       a.s_n[k] = ins[k].sn;
       a.vin[k] = ins[k].vin;
       const int va = std::min(CH * es, 16);
-      if (ins[k].vin && reinterpret_cast<uintptr_t>(a.in[k]) % va != 0)
+      if (ins[k].vin && ins[k].al && reinterpret_cast<uintptr_t>(a.in[k]) % va != 0)
         return set_error(e, GHIP_ERR_STATE, "fused GEMM epilogue: operand %zu not %d-byte aligned", k, va);
     }
     a.out = p.c;

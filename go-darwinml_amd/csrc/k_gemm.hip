@@ -6,11 +6,13 @@
 // 128 256 x 256 tiles run the 256 x 256 cores (A K- / B N-contiguous: the 4-wave
 // 16x16x32 core; B K-contiguous: the 8-wave 64-deep 16x16x32 core; both
 // MN-contiguous: the 4-wave 32-deep core); smaller grids the 4-wave 128 x 128
-// 32x32x16 core, two workgroups per CU.
-// fp32 path: v_mfma_f32_32x32x2f32 over LDS-DMA tiles (below).
-// Anything the vector paths cannot address (odd strides, unaligned bases,
-// negative strides, a row stride of 4M elements (bf16) / 2M (fp32) or more) runs
-// a generic LDS-tiled kernel.  Operand slices may exceed 4 GiB: each tile's
+// 32x32x16 core, two workgroups per CU; grids of few tiles the register-staged core's
+// 64 x 64 tiles (gemm_small_tiles).
+// fp32 path: v_mfma_f32_32x32x2f32 over LDS-DMA tiles, or register-staged tiles.
+// Operands that the LDS DMA cannot address (unaligned bases, rows or strides that
+// are not whole 16-byte chunks) run the register-staged cores (RsTile); neither unit
+// stride, negative strides or a row stride of 4M elements (bf16) / 2M (fp32) or
+// more run a generic LDS-tiled kernel.  Operand slices may exceed 4 GiB: each tile's
 // buffer descriptors are based at the tile (gemm_rows_fit, left_bytes).
 #include "gemm_kernels.h"
 
@@ -155,6 +157,12 @@ static int64_t slice_bytes(int64_t rows, int64_t s_row, int64_t K, int64_t s_k, 
   return ((rows - 1) * s_row + (K - 1) * s_k + 1) * es;
 }
 
+template <typename InT, typename OutT>
+static hipError_t launch_rs(const GemmParams& p, hipStream_t s) {
+  return gemm_small_tiles(p.batch, p.M, p.N, sizeof(InT)) ? launch_rs_tile<64, InT, OutT>(p, s)
+                                                          : launch_rs_tile<128, InT, OutT>(p, s);
+}
+
 // Workspace of a split contraction (16-byte aligned, large enough: checked by the
 // entry points); ptr null: no split.
 struct GemmWs {
@@ -233,7 +241,7 @@ static hipError_t dispatch_bf16(GemmParams p, hipStream_t s, GemmWs ws = {}) {
   const bool big_ok = p.M >= 256 && p.N >= 256 && t256 >= 128;
   if (ma < 0 || mb < 0 || !nonneg || !gemm_rows_fit(p.sa_m, p.sa_k, 2) || !gemm_rows_fit(p.sb_n, p.sb_k, 2) ||
       (big && !big_ok))
-    return launch_generic<InT, OutT>(p, s);
+    return rs_fits(p, 2) ? launch_rs<InT, OutT>(p, s) : launch_generic<InT, OutT>(p, s);
   p.a_extent = big ? 0u : static_cast<uint32_t>(ea);
   p.b_extent = big ? 0u : static_cast<uint32_t>(eb);
   p.a_extent64 = ea;
@@ -243,10 +251,11 @@ static hipError_t dispatch_bf16(GemmParams p, hipStream_t s, GemmWs ws = {}) {
             (reinterpret_cast<uintptr_t>(p.c) % 16 == 0);
   if (big) return launch_bf16_4w<true, InT, OutT>(p, ma, mb, s);
   // Few tiles and a long contraction, with a workspace: the contraction split.
-  if (ws.ptr) {
+  if (ws.ptr && gemm_uses_split(p.batch, p.M, p.N, p.K, 2)) {
     const GemmSplit sp = gemm_k_split(p.batch, p.M, p.N, p.K, 2);
-    if (sp.s > 1 && gemm_split_bytes(sp, p.M, p.N) <= ws.bytes) return launch_split<InT, OutT>(p, ma, mb, sp, ws.ptr, s);
+    if (gemm_split_bytes(sp, p.M, p.N) <= ws.bytes) return launch_split<InT, OutT>(p, ma, mb, sp, ws.ptr, s);
   }
+  if (p.K > 0 && gemm_small_tiles(p.batch, p.M, p.N, 2)) return launch_rs_tile<64, InT, OutT>(p, s);
   // Grids of more than 128 256 x 256 tiles: the 256 x 256 cores (one workgroup per
   // CU).  Up to 128 such tiles they would leave half the 256 CUs or more idle, and
   // the 128 x 128 core (two workgroups per CU, so up to 512 tiles in one round) is
@@ -274,7 +283,7 @@ static hipError_t dispatch_grouped(GemmParams p, int G, const void* const* b, vo
   ok = ok && ea < (int64_t{1} << 31) && eb < (int64_t{1} << 31) && p.M >= 256 && p.N >= 256 && G * tiles >= 128;
   // Products the stand-alone entry splits (given the workspace) run as that split,
   // one after another in the same workspace, so each keeps the stand-alone bits.
-  if (ws.ptr && gemm_k_split(1, p.M, p.N, p.K, 2).s > 1) ok = false;
+  if (ws.ptr && gemm_uses_split(1, p.M, p.N, p.K, 2)) ok = false;
   if (!ok) {
     for (int g = 0; g < G; ++g) {
       GemmParams q = p;
@@ -320,7 +329,7 @@ static hipError_t dispatch_f32(GemmParams p, hipStream_t s, GemmWs ws = {}) {
   const bool big = ea >= (int64_t{1} << 31) || eb >= (int64_t{1} << 31);
   if (ma < 0 || mb < 0 || !nonneg || !gemm_rows_fit(p.sa_m, p.sa_k, 4) || !gemm_rows_fit(p.sb_n, p.sb_k, 4) ||
       (big && !grid256))
-    return launch_generic<float, OutT>(p, s);
+    return rs_fits(p, 4) ? launch_rs<float, OutT>(p, s) : launch_generic<float, OutT>(p, s);
   p.a_extent = big ? 0u : static_cast<uint32_t>(ea);
   p.b_extent = big ? 0u : static_cast<uint32_t>(eb);
   p.a_extent64 = ea;
@@ -329,10 +338,11 @@ static hipError_t dispatch_f32(GemmParams p, hipStream_t s, GemmWs ws = {}) {
             (reinterpret_cast<uintptr_t>(p.c) % (4 * sizeof(OutT)) == 0);
   if (big) return launch_f32<256, 256, 2, 4, OutT, true>(p, ma, mb, s);
   // Few tiles and a long contraction, with a workspace: the contraction split.
-  if (ws.ptr) {
+  if (ws.ptr && gemm_uses_split(p.batch, p.M, p.N, p.K, 4)) {
     const GemmSplit sp = gemm_k_split(p.batch, p.M, p.N, p.K, 4);
-    if (sp.s > 1 && gemm_split_bytes(sp, p.M, p.N) <= ws.bytes) return launch_split<float, OutT>(p, ma, mb, sp, ws.ptr, s);
+    if (gemm_split_bytes(sp, p.M, p.N) <= ws.bytes) return launch_split<float, OutT>(p, ma, mb, sp, ws.ptr, s);
   }
+  if (p.K > 0 && gemm_small_tiles(p.batch, p.M, p.N, 4)) return launch_rs_tile<64, float, OutT>(p, s);
   // The 8-wave 256 x 256 fp32 core only from one full round of its tiles: below
   // that the 4-wave 128 x 128 core (two workgroups per CU) is faster, 1.9x at 128
   // tiles of 256 x 256 ([2048,4096,4096]), 1.3x at 144 and 192, even at 256.
