@@ -18,8 +18,10 @@
 //     67% of the 8 TB/s HBM peak;
 //   * WPR > 1 combines the per-wave partial sums through LDS (one barrier per
 //     reduction);
-//   * anything else (unaligned rows, n not a multiple of the vector width, or
-//     rows beyond the register budget) takes a generic multi-pass kernel.
+//   * rows of any width and element alignment take the same kernels with their first
+//     and last vectors read element by element (UA);
+//   * rows beyond the register budget (and unaligned attention scores) take a generic
+//     multi-pass kernel.
 // Statistics are fp32 for fp32, bf16 and f16 I/O.
 #include <stdarg.h>
 
@@ -99,10 +101,43 @@ __device__ __forceinline__ uint4 pack(const float* f, f16_t) {
                     pack_f16x2(f[6], f[7]));
 }
 
+// 16 bytes at element alignment (rows that start inside a 16-byte block).
+typedef unsigned u32x4_un __attribute__((ext_vector_type(4), aligned(2), may_alias));
+__device__ __forceinline__ uint4 ld_un(const void* p) {
+  const u32x4_un v = *static_cast<const u32x4_un*>(p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void st_un(void* p, uint4 v) {
+  *static_cast<u32x4_un*>(p) = u32x4_un{v.x, v.y, v.z, v.w};
+}
+// Elements lo .. hi - 1 (lo < hi) of a 16-byte vector at p, `pad` bits in the others.
+template <typename T>
+__device__ __forceinline__ uint4 ld_part(const T* p, int lo, int hi, uint32_t pad) {
+  constexpr int VEC = Elem<T>::kVec, ES = sizeof(T);
+  using E = std::conditional_t<ES == 4, uint32_t, uint16_t>;
+  uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) {
+    // Every load is of a valid element, so none is conditional.
+    const E e = *reinterpret_cast<const E*>(p + (j < lo ? lo : j >= hi ? hi - 1 : j));
+    w[j * ES / 4] |= (j >= lo && j < hi ? static_cast<uint32_t>(e) : pad) << (j * ES % 4 * 8);
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+template <typename T>
+__device__ __forceinline__ void st_part(T* p, int lo, int hi, const float* f) {
+#pragma unroll
+  for (int j = 0; j < Elem<T>::kVec; ++j)
+    if (j >= lo && j < hi) Elem<T>::store1(p + j, f[j]);
+}
+__device__ __forceinline__ uint32_t neg_inf_bits(float) { return 0xff800000u; }
+__device__ __forceinline__ uint32_t neg_inf_bits(bf16_t) { return 0xff80u; }
+__device__ __forceinline__ uint32_t neg_inf_bits(f16_t) { return 0xfc00u; }
+
 // Sum / max over the WPR waves of a row (slot: which LDS pair to use, so two
 // back-to-back reductions need no extra barrier).
-template <int WPR>
-__device__ __forceinline__ float row_reduce_sum(float v, float (*lds)[4], int slot) {
+template <int WPR, int W>
+__device__ __forceinline__ float row_reduce_sum(float v, float (*lds)[W], int slot) {
   v = wave_sum(v);
   if constexpr (WPR == 1) {
     return v;
@@ -117,8 +152,8 @@ __device__ __forceinline__ float row_reduce_sum(float v, float (*lds)[4], int sl
     return t;
   }
 }
-template <int WPR>
-__device__ __forceinline__ float row_reduce_max(float v, float (*lds)[4], int slot) {
+template <int WPR, int W>
+__device__ __forceinline__ float row_reduce_max(float v, float (*lds)[W], int slot) {
   v = wave_max(v);
   if constexpr (WPR == 1) {
     return v;
@@ -136,10 +171,14 @@ __device__ __forceinline__ float row_reduce_max(float v, float (*lds)[4], int sl
 
 // Row statistics of RMSNorm (mean 0, rstd = 1/sqrt(mean(x^2) + eps)) or
 // LayerNorm (mean, rstd = 1/sqrt(var + eps)) from the row values of the calling
-// lanes: xget(i, f) gives vector i as fp32 (live[i]: vector i lies on the row).
-template <typename T, int OP, int NV, int WPR, typename XG>
-__device__ __forceinline__ void norm_stats(XG xget, const bool (&live)[NV], int64_t n, float eps, float (*lds)[4],
-                                           float& mean, float& rstd) {
+// lanes: xget(i, f) gives vector i as fp32 (live[i]: vector i lies on the row), zeros
+// outside the row; ok(i, j): element j of a live vector i lies on the row.
+struct WholeVectors {
+  __device__ __forceinline__ bool operator()(int, int) const { return true; }
+};
+template <typename T, int OP, int NV, int WPR, int W, typename XG, typename OK = WholeVectors>
+__device__ __forceinline__ void norm_stats(XG xget, const bool (&live)[NV], int64_t n, float eps, float (*lds)[W],
+                                           float& mean, float& rstd, OK ok = OK{}) {
   // Contraction only within one expression (s += x * x is one fma; a product is
   // never fused into a later statement's sum): otherwise the backend may fuse
   // either product of x0*x0 + x1*x1, and the two norm kernels (which must give
@@ -160,9 +199,11 @@ __device__ __forceinline__ void norm_stats(XG xget, const bool (&live)[NV], int6
       if (!live[i]) continue;
       float f[VEC];
       xget(i, f);
-      cnt += VEC;
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) sw += f[j];
+      for (int j = 0; j < VEC; ++j) {
+        cnt += ok(i, j) ? 1.f : 0.f;
+        sw += f[j];
+      }
     }
     cnt = wave_sum(cnt);
     sw = wave_sum(sw);
@@ -175,7 +216,7 @@ __device__ __forceinline__ void norm_stats(XG xget, const bool (&live)[NV], int6
       xget(i, f);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
-        const float d = f[j] - mw;
+        const float d = ok(i, j) ? f[j] - mw : 0.f;
         qw += d * d;
       }
     }
@@ -220,7 +261,7 @@ __device__ __forceinline__ void norm_stats(XG xget, const bool (&live)[NV], int6
       xget(i, f);
 #pragma unroll
         for (int j = 0; j < VEC; ++j) {
-          const float d = f[j] - mean;
+          const float d = ok(i, j) ? f[j] - mean : 0.f;
           q += d * d;
         }
       }
@@ -233,15 +274,20 @@ __device__ __forceinline__ void norm_stats(XG xget, const bool (&live)[NV], int6
 // Store pass of the norms: y = (x - mean) * rstd [* gamma] [+ beta], one copy per
 // (gamma, beta) presence (tested per element, the uniform pointer checks became a
 // select per value); gfetch / bfetch(i, c0, out) supply vector i of gamma / beta.
-template <typename T, int NV, int LANES, typename XG, typename HG, typename HB, typename GF, typename BF>
+struct StoreNt {  // whole aligned vectors
+  template <typename T>
+  __device__ __forceinline__ void operator()(int, T* y, const float* f) const { st_nt(y, pack(f, T{})); }
+};
+template <typename T, int NV, int LANES, typename XG, typename HG, typename HB, typename GF, typename BF,
+          typename ST = StoreNt>
 __device__ __forceinline__ void norm_store(XG xget, const bool (&live)[NV], float mean, float rstd, T* yr, int l, HG,
-                                           HB, GF gfetch, BF bfetch) {
+                                           HB, GF gfetch, BF bfetch, int64_t off = 0, ST st = ST{}) {
 #pragma clang fp contract(on)
   constexpr int VEC = Elem<T>::kVec;
   constexpr bool G = HG::value, B = HB::value;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int64_t c0 = (static_cast<int64_t>(i) * LANES + l) * VEC;
+    const int64_t c0 = (static_cast<int64_t>(i) * LANES + l) * VEC - off;
     if (!live[i]) continue;
     float x[VEC], f[VEC], gv[VEC], bv[VEC];
     xget(i, x);
@@ -255,20 +301,28 @@ __device__ __forceinline__ void norm_store(XG xget, const bool (&live)[NV], floa
       else if constexpr (B) f[j] = t + bv[j];
       else f[j] = t;
     }
-    st_nt(yr + c0, pack(f, T{}));
+    st(i, yr + c0, f);
   }
 }
 
 // One row per WPR waves; a 256-thread workgroup handles 4 / WPR rows (row group
-// `blk`).  NV packed 16-byte vectors per lane.
-template <typename T, int OP, int NV, int WPR>
-__device__ __forceinline__ void rows_reg_group(const RowParams& p, int64_t blk, float (*lds)[4]) {
+// `blk`), a wider one (WPR > 4) one row.  NV packed 16-byte vectors per lane.
+//
+// UA: rows of any width and element alignment.  The row's vectors are the 16-byte
+// blocks of memory it covers (vector v starts `off` elements before a multiple of VEC
+// from the row's first element), so every whole one is an aligned load; the first and
+// last may hold elements outside the row (lo / hi bound the valid ones), which are
+// read and written one by one and stand in as -inf (softmax) or zero (norms).  Bound by
+// HBM like the aligned rows; such rows took the several-pass scalar kernel before:
+// fp32 log-softmax [2048, 32003] 248 us (2.1 TB/s), here 100 (5.2 TB/s).
+template <typename T, int OP, int NV, int WPR, bool UA, int W>
+__device__ __forceinline__ void rows_reg_group(const RowParams& p, int64_t blk, float (*lds)[W]) {
   constexpr int VEC = Elem<T>::kVec;
   constexpr int LANES = kWave * WPR;
-  constexpr int ROWS_PER_BLOCK = 4 / WPR;
+  constexpr int ROWS_PER_BLOCK = WPR > 4 ? 1 : 4 / WPR;
 
-  const int sub = threadIdx.x / LANES;  // row slot within the block
-  const int l = threadIdx.x % LANES;    // lane index within the row
+  const int sub = ROWS_PER_BLOCK == 1 ? 0 : threadIdx.x / LANES;  // row slot within the block
+  const int l = ROWS_PER_BLOCK == 1 ? threadIdx.x : threadIdx.x % LANES;  // lane index within the row
   const int64_t row = blk * ROWS_PER_BLOCK + sub;
   // With WPR > 1 every wave of a row slot shares the row, and the grid covers
   // whole blocks only when rows % ROWS_PER_BLOCK == 0; the early exit is taken
@@ -281,14 +335,65 @@ __device__ __forceinline__ void rows_reg_group(const RowParams& p, int64_t blk, 
   const T* xr = static_cast<const T*>(p.x) + (row_ok ? row : 0) * n;
   T* yr = static_cast<T*>(p.y) + (row_ok ? row : 0) * n;
 
+  const int off = UA ? static_cast<int>(reinterpret_cast<uintptr_t>(xr) / sizeof(T) % VEC) : 0;
   uint4 v[NV];
-  bool live[NV];
+  bool live[NV];   // vector i holds elements of the row
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int64_t c0 = (static_cast<int64_t>(i) * LANES + l) * VEC;
+    const int64_t c0 = (static_cast<int64_t>(i) * LANES + l) * VEC - off;
     live[i] = row_ok && c0 < n;
   }
-
+  // UA: the partly covered vectors are the first (lane 0, elements head .. VEC - 1 or
+  // the row's end) and the last (element tail - 1 its last one); a row inside one
+  // vector is all head.  Each is handled by code of its own outside the loops over i.
+  const int last = UA ? static_cast<int>((off + n - 1) / VEC) : 0;
+  const int tail = UA ? static_cast<int>(off + n - static_cast<int64_t>(last) * VEC) : VEC;
+  const bool is_head = UA && row_ok && l == 0 && (off > 0 || (last == 0 && tail < VEC));
+  const bool is_tail = UA && row_ok && tail < VEC && last > 0 && l == last % LANES;
+  const int i_tail = last / LANES, head_end = last == 0 ? tail : VEC;
+  // Vector i of this lane in the row at q (a 32-bit lane offset from a per-row base).
+  auto vec_at = [&](auto* q, int i) {
+    using P = decltype(q);
+    using C = std::conditional_t<std::is_const_v<std::remove_pointer_t<P>>, const char, char>;
+    return reinterpret_cast<P>(reinterpret_cast<C*>(q - off + i * LANES * VEC) + static_cast<uint32_t>(l) * 16u);
+  };
+  // Keeps the compiler from carrying the widened values of 16-bit vectors between the
+  // passes (twice the registers: half the waves, or spills in the 1024-thread form).
+  auto repack = [&]() {
+    if constexpr (UA && (VEC == 8 || NV > 8)) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(v[i].x), "+v"(v[i].y), "+v"(v[i].z), "+v"(v[i].w));
+    }
+  };
+  auto whole = [&](int i) { return !(UA && ((i == 0 && is_head) || (is_tail && i == i_tail))); };
+  // The row's vectors from q (x, gamma or beta); pad stands outside the row.
+  auto load_edges = [&](const T* q, uint32_t pad, auto set) {
+    if constexpr (UA) {
+      if (is_head) set(0, ld_part(q - off, off, head_end, pad));
+      if (is_tail) {
+        const uint4 w = ld_part(q - off + static_cast<int64_t>(last) * VEC, 0, tail, pad);
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+          if (i == i_tail) set(i, w);
+      }
+    }
+  };
+  float f_tail[VEC];
+  auto store = [&](int i, T* dst, const float* f) {
+    if constexpr (UA) {
+      if (whole(i)) st_un(dst, pack(f, T{}));
+      if (i == 0 && is_head) st_part(dst, off, head_end, f);
+      if (is_tail && i == i_tail)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) f_tail[j] = f[j];
+    } else {
+      st_nt(dst, pack(f, T{}));
+    }
+  };
+  auto store_tail = [&]() {
+    if constexpr (UA)
+      if (is_tail) st_part(yr - off + static_cast<int64_t>(last) * VEC, 0, tail, f_tail);
+  };
   if constexpr (OP == kSoftmax || OP == kLogSoftmax || OP == kMaskedSoftmax) {
     const int64_t qrow = (OP == kMaskedSoftmax) ? ((row_ok ? row : 0) % p.sq) : 0;
     int64_t moff = 0;
@@ -323,8 +428,9 @@ __device__ __forceinline__ void rows_reg_group(const RowParams& p, int64_t blk, 
     for (int i = 0; i < NV; ++i) {
       const int64_t c0 = (static_cast<int64_t>(i) * LANES + l) * VEC;
       const bool skip = (OP == kMaskedSoftmax) && p.causal && c0 > qrow;
-      if (live[i] && !skip) v[i] = ld_nt(xr + c0);
+      if (live[i] && !skip && whole(i)) v[i] = ld_nt(vec_at(xr, i));
     }
+    load_edges(xr, neg_inf_bits(T{}), [&](int i, uint4 w) { v[i] = w; });
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -334,6 +440,7 @@ __device__ __forceinline__ void rows_reg_group(const RowParams& p, int64_t blk, 
       for (int j = 0; j < VEC; ++j) mx = fmaxf(mx, f[j]);
     }
     mx = row_reduce_max<WPR>(mx, lds, 0);
+    repack();
     // fp32 softmax keeps each exp in the register its input came from (a
     // vector holds 4 fp32 either way), so the store pass only scales.
     constexpr bool kKeepExp = OP != kLogSoftmax && Elem<T>::kVec == 4;
@@ -351,12 +458,13 @@ __device__ __forceinline__ void rows_reg_group(const RowParams& p, int64_t blk, 
                                                __float_as_uint(f[3]));
     }
     s = row_reduce_sum<WPR>(s, lds, 1);
+    repack();
     const float shift = mx + logf(s);
     const float inv = 1.0f / s;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       if (!live[i]) continue;
-      const int64_t c0 = (static_cast<int64_t>(i) * LANES + l) * VEC;
+      const int64_t c0 = (static_cast<int64_t>(i) * LANES + l) * VEC - off;
       float f[VEC];
       if constexpr (kKeepExp) {
         f[0] = __uint_as_float(v[i].x) * inv;
@@ -369,21 +477,22 @@ __device__ __forceinline__ void rows_reg_group(const RowParams& p, int64_t blk, 
         for (int j = 0; j < VEC; ++j)
           f[j] = (OP == kLogSoftmax) ? f[j] - shift : fast_exp(f[j] - mx) * inv;
       }
-      st_nt(yr + c0, pack(f, T{}));
+      store(i, vec_at(yr, i), f);
     }
+    store_tail();
   } else {
     // RMSNorm / LayerNorm.
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int64_t c0 = (static_cast<int64_t>(i) * LANES + l) * VEC;
-      v[i] = live[i] ? ld_nt(xr + c0) : make_uint4(0, 0, 0, 0);
+      v[i] = live[i] && whole(i) ? ld_nt(vec_at(xr, i)) : make_uint4(0, 0, 0, 0);
     }
+    load_edges(xr, 0u, [&](int i, uint4 w) { v[i] = w; });
     // RMSNorm fp32: gamma is fetched with x, so its (L2) latency overlaps the
     // loads of x instead of following the statistics ([8192, 4096]: +3.5..5%).
     // For 16-bit data and for LayerNorm (gamma and beta) the extra registers cost
     // more than the overlap gains (measured -1..2%); beyond 4 vectors per lane
     // they would halve the waves in flight.
-    constexpr bool kEarlyParams = Elem<T>::kVec == 4 && OP == kRmsNorm && NV <= 4;
+    constexpr bool kEarlyParams = !UA && Elem<T>::kVec == 4 && OP == kRmsNorm && NV <= 4;
     uint4 gr[kEarlyParams ? NV : 1];
 #pragma unroll
     for (int i = 0; i < NV && kEarlyParams; ++i) {
@@ -395,20 +504,46 @@ __device__ __forceinline__ void rows_reg_group(const RowParams& p, int64_t blk, 
     // mask per 16-bit value), which needs half the registers of an fp32 copy.
     float mean, rstd;
     auto xget = [&](int i, float* f) { unpack(v[i], f, T{}); };
-    norm_stats<T, OP, NV, WPR>(xget, live, n, p.eps, lds, mean, rstd);
+    if constexpr (UA)
+      norm_stats<T, OP, NV, WPR>(xget, live, n, p.eps, lds, mean, rstd,
+                                 [&](int i, int j) {
+                                   const int c = (i * LANES + l) * VEC - off + j;
+                                   return c >= 0 && c < static_cast<int>(n);
+                                 });
+    else norm_stats<T, OP, NV, WPR>(xget, live, n, p.eps, lds, mean, rstd);
+    repack();
     const T* g = static_cast<const T*>(p.gamma);
     const T* b = static_cast<const T*>(p.beta);
+    // gamma / beta at the vector's columns; those of the partly covered vectors (a lane
+    // holds at most one head and one tail) are read before the store pass.
+    uint4 ge[2], be[2];
+    auto edges = [&](const T* q, uint4 (&e)[2]) {
+      if constexpr (UA) {
+        if (q && is_head) e[0] = ld_part(q - off, off, head_end, 0u);
+        if (q && is_tail) e[1] = ld_part(q - off + static_cast<int64_t>(last) * VEC, 0, tail, 0u);
+      }
+    };
+    edges(g, ge);
+    edges(b, be);
+    auto fetch = [&](const T* q, const uint4 (&e)[2], int i, int64_t c0, float* w) {
+      if constexpr (UA) unpack(whole(i) ? ld_un(q + c0) : i == 0 && is_head ? e[0] : e[1], w, T{});
+      else load_vec(q + c0, w);
+    };
     auto gfetch = [&](int i, int64_t c0, float* gv) {
       if constexpr (kEarlyParams) unpack(gr[i], gv, T{});
-      else load_vec(g + c0, gv);
+      else fetch(g, ge, i, c0, gv);
     };
-    auto bfetch = [&](int i, int64_t c0, float* bv) { load_vec(b + c0, bv); };
+    auto bfetch = [&](int i, int64_t c0, float* bv) { fetch(b, be, i, c0, bv); };
     using yes = std::true_type;
     using no = std::false_type;
-    if (g && b) norm_store<T, NV, LANES>(xget, live, mean, rstd, yr, l, yes{}, yes{}, gfetch, bfetch);
-    else if (g) norm_store<T, NV, LANES>(xget, live, mean, rstd, yr, l, yes{}, no{}, gfetch, bfetch);
-    else if (b) norm_store<T, NV, LANES>(xget, live, mean, rstd, yr, l, no{}, yes{}, gfetch, bfetch);
-    else norm_store<T, NV, LANES>(xget, live, mean, rstd, yr, l, no{}, no{}, gfetch, bfetch);
+    auto put = [&](auto hg, auto hb) {
+      norm_store<T, NV, LANES>(xget, live, mean, rstd, yr, l, hg, hb, gfetch, bfetch, off, store);
+    };
+    if (g && b) put(yes{}, yes{});
+    else if (g) put(yes{}, no{});
+    else if (b) put(no{}, yes{});
+    else put(no{}, no{});
+    store_tail();
   }
 }
 
@@ -416,16 +551,16 @@ __device__ __forceinline__ void rows_reg_group(const RowParams& p, int64_t blk, 
 // own, preloaded into SGPRs like rows_norm_stream_kernel's: the row's loads are
 // addressed without waiting for a kernel-argument fetch (at the config's 6 us per
 // launch, that fetch is a visible part of the kernel).
-template <typename T, int OP, int NV, int WPR>
-__global__ __launch_bounds__(256) void rows_reg_kernel(const void* x, void* y, int64_t rows, int64_t n,
-                                                       RowParams p) {
-  __shared__ float lds[3][4];
+template <typename T, int OP, int NV, int WPR, bool UA = false>
+__global__ __launch_bounds__(WPR > 4 ? WPR * 64 : 256) void rows_reg_kernel(const void* x, void* y, int64_t rows,
+                                                                            int64_t n, RowParams p) {
+  __shared__ float lds[3][WPR > 4 ? WPR : 4];
   RowParams q = p;
   q.x = x;
   q.y = y;
   q.rows = rows;
   q.n = n;
-  rows_reg_group<T, OP, NV, WPR>(q, blockIdx.x, lds);
+  rows_reg_group<T, OP, NV, WPR, UA>(q, blockIdx.x, lds);
 }
 
 // Streaming RMSNorm / LayerNorm for rows that exactly fill NV vectors of every
@@ -634,12 +769,12 @@ static int device_cus() {
   return c;
 }
 
-template <typename T, int OP, int NV, int WPR>
+template <typename T, int OP, int NV, int WPR, bool UA = false>
 static hipError_t launch_reg(const RowParams& p, hipStream_t s) {
-  const int rows_per_block = 4 / WPR;
+  const int rows_per_block = WPR > 4 ? 1 : 4 / WPR;
   const int64_t groups = (p.rows + rows_per_block - 1) / rows_per_block;
-  hipLaunchKernelGGL((rows_reg_kernel<T, OP, NV, WPR>), dim3(static_cast<unsigned>(groups)), dim3(256), 0, s, p.x, p.y,
-                     p.rows, p.n, p);
+  hipLaunchKernelGGL((rows_reg_kernel<T, OP, NV, WPR, UA>), dim3(static_cast<unsigned>(groups)),
+                     dim3(WPR > 4 ? WPR * 64 : 256), 0, s, p.x, p.y, p.rows, p.n, p);
   return hipGetLastError();
 }
 
@@ -716,6 +851,30 @@ static hipError_t launch_rows(const RowParams& p, hipStream_t s) {
     if (vecs <= 256 * 4) return go(I4{}, I4{});
     if (vecs <= 256 * 8) return go(I8{}, I4{});
     if (vecs <= 256 * 16) return go(I16{}, I4{});
+  }
+  // Rows of any width and alignment, and wide softmax rows (sixteen waves a row), held
+  // whole in registers too (x read from HBM once).  vecs: blocks of 16 bytes the row may
+  // touch.  Norms stop at four vectors a lane: wider ones are not met.
+  if constexpr (OP != kMaskedSoftmax) {
+    const int64_t vecs = (p.n + 2 * VEC - 2) / VEC;
+    auto go = [&](auto nv, auto wpr) { return launch_reg<T, OP, decltype(nv)::value, decltype(wpr)::value, true>(p, s); };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I4 = std::integral_constant<int, 4>;
+    using I8 = std::integral_constant<int, 8>;
+    using I16 = std::integral_constant<int, 16>;
+    if (vecs <= 64 * 1) return go(I1{}, I1{});
+    if (vecs <= 64 * 2) return go(I2{}, I1{});
+    if (vecs <= 64 * 4) return go(I4{}, I1{});
+    if (vecs <= 128 * 4) return go(I4{}, I2{});
+    if (vecs <= 256 * 4) return go(I4{}, I4{});
+    if (vecs <= 256 * 8) return go(I8{}, I4{});
+    if (vecs <= 1024 * 4) return go(I4{}, I16{});
+    if constexpr (OP == kSoftmax || OP == kLogSoftmax) {
+      if (vecs <= 1024 * 8) return go(I8{}, I16{});
+      if constexpr (VEC == 4)
+        if (vecs <= 1024 * 16) return go(I16{}, I16{});
+    }
   }
   hipLaunchKernelGGL((rows_generic_kernel<T, OP>), dim3(static_cast<unsigned>(p.rows)),
                      dim3(256), 0, s, p);
