@@ -2515,6 +2515,9 @@ View Lowerer::emit_cluster(int root, int v) {
   }
   const Shape& os = N[v].shape;
   std::set<int> inset(mem.begin(), mem.end());
+  const int64_t total = os.size();
+  const int rank = os.rank();
+  const int64_t inner = rank ? os.dims[rank - 1] : 1;
   // Inputs: operands outside the cluster (scalar constants become literals;
   // Iota operands of the cluster's shape are computed from the index).
   struct In {
@@ -2523,17 +2526,20 @@ View Lowerer::emit_cluster(int root, int v) {
     std::vector<int64_t> eff;  // effective strides over os.dims
     bool linear;
     bool partial = false;      // a split Dot's fp32 partials, read at i + j * size
+    int splits = 0;
   };
   std::vector<In> ins;
   int n_partial = 0;
-  std::map<int, std::string> expr;  // value -> C expression
+  std::map<int, std::string> expr;  // value -> C expression of element i + e
   std::ostringstream body;
   bool need_idx = false;
   std::vector<std::string> idx_names;
-  for (int d = 0; d < os.rank(); ++d) idx_names.push_back("d" + std::to_string(d));
+  for (int d = 0; d < rank; ++d) idx_names.push_back("d" + std::to_string(d));
+  // Coordinates of element e of the thread's vector: the last one steps with e.
   auto iota_expr = [&](int u) {
     need_idx = true;
-    return "((" + ctype(N[u].shape.dtype) + ")" + idx_names[N[u].i0] + ")";
+    const int ax = static_cast<int>(N[u].i0);
+    return "((" + ctype(N[u].shape.dtype) + ")(" + idx_names[ax] + (ax == rank - 1 ? " + e" : "") + "))";
   };
   for (int u : mem) {
     for (int o : N[u].in) {
@@ -2547,6 +2553,8 @@ View Lowerer::emit_cluster(int root, int v) {
         expr[o] = iota_expr(o);
         continue;
       }
+      const std::string ks = std::to_string(ins.size());
+      expr[o] = "in" + ks;
       // A DotGeneral read only here whose contraction splits: its fp32 partials
       // come from a GEMM step of their own and are summed here, in range order,
       // then rounded to the Dot's dtype: the value the stand-alone sum kernel
@@ -2554,17 +2562,11 @@ View Lowerer::emit_cluster(int root, int v) {
       View pw;
       int ps = 0;
       if (fuse_epilogues && emit_split_partials(o, os, inset, &pw, &ps)) {
-        const int k = static_cast<int>(ins.size());
         In in{o, pw, contiguous_strides(os.dims), true};
         in.partial = true;
-        const std::string pk = "((const float*)p_in" + std::to_string(k) + ")";
-        const std::string acc = "acc" + std::to_string(k);
-        body << "    float " << acc << " = " << pk << "[i];\n";
-        body << "    for (int j = 1; j < " << ps << "; ++j) " << acc << " += " << pk << "[i + (long long)j * "
-             << os.size() << "LL];\n";
-        body << "    const " << ctype(N[o].shape.dtype) << " in" << k << " = " << round_expr(N[o].shape.dtype, acc)
-             << ";\n";
-        expr[o] = "in" + std::to_string(k);
+        in.splits = ps;
+        body << "      const " << ctype(N[o].shape.dtype) << " in" << ks << " = "
+             << round_expr(N[o].shape.dtype, "x" + ks + "[e]") << ";\n";
         ins.push_back(in);
         ++n_partial;
         continue;
@@ -2575,39 +2577,39 @@ View Lowerer::emit_cluster(int root, int v) {
       In in{o, w, {}, true};
       // right-aligned implicit broadcast to os.dims
       const Shape& s = N[o].shape;
-      const int off = os.rank() - s.rank();
-      in.eff.assign(os.rank(), 0);
+      const int off = rank - s.rank();
+      in.eff.assign(rank, 0);
       for (int d = 0; d < s.rank(); ++d)
         if (s.dims[d] != 1) in.eff[off + d] = w.strides[d];
       auto cs = contiguous_strides(os.dims);
-      for (int d = 0; d < os.rank(); ++d)
+      for (int d = 0; d < rank; ++d)
         if (os.dims[d] != 1 && in.eff[d] != cs[d]) in.linear = false;
       if (!in.linear) need_idx = true;
-      const int k = static_cast<int>(ins.size());
-      std::string off_e = "i";
-      if (!in.linear) {
-        off_e = "0";
-        for (int d = 0; d < os.rank(); ++d)
-          if (in.eff[d] != 0 && os.dims[d] != 1) off_e += " + " + idx_names[d] + " * " + std::to_string(in.eff[d]) + "LL";
-      }
-      body << "    const " << ctype(s.dtype) << " in" << k << " = "
-           << load_expr(s.dtype, "((const " + stype(s.dtype) + "*)p_in" + std::to_string(k) + ")[" + off_e + "]") << ";\n";
-      expr[o] = "in" + std::to_string(k);
+      body << "      const " << ctype(s.dtype) << " in" << ks << " = " << load_expr(s.dtype, "x" + ks + "[e]") << ";\n";
       ins.push_back(in);
     }
     if (failed) return bad();
     if (N[u].kind == Kind::Iota) {
       const std::string name = "v" + std::to_string(u);
-      body << "    const " << ctype(N[u].shape.dtype) << " " << name << " = " << round_expr(N[u].shape.dtype, iota_expr(u)) << ";\n";
+      body << "      const " << ctype(N[u].shape.dtype) << " " << name << " = " << round_expr(N[u].shape.dtype, iota_expr(u)) << ";\n";
       expr[u] = name;
     } else {
-      body << member_stmt(u, expr, "v" + std::to_string(u));
+      body << "  " << member_stmt(u, expr, "v" + std::to_string(u));
     }
   }
+  // V consecutive elements a thread: 16 bytes of the output where the cluster still
+  // fills the chip (256 CUs x 256 threads), fewer below that, where more threads hide
+  // the loads' latency better than wider loads.  A vector stays inside a row of the
+  // last axis when coordinates are needed.  Bound by HBM; bf16 [4096, 8192], two
+  // inputs: 41 us (4.9 TB/s) with an element a thread, 31 (6.5 TB/s) with eight.
+  int V = std::max(1, 16 / dtype_size(os.dtype));
+  while (V > 1 && (total / V < 65536 || (need_idx && inner % V != 0))) V /= 2;
+  const std::string Vs = std::to_string(V);
   // Slots every read of which is at the output's own element index (linear,
   // offset 0, same element size): the output may overwrite them in place (a
   // donated input), so those operands and the output are not declared
-  // __restrict__: with donation they are one buffer.
+  // __restrict__: with donation they are one buffer.  (A thread's loads of its
+  // vector all precede its store.)
   std::vector<int> inplace;
   for (auto& in : ins) {
     bool ok = !in.partial;
@@ -2618,28 +2620,75 @@ View Lowerer::emit_cluster(int root, int v) {
     if (ok && std::find(inplace.begin(), inplace.end(), in.view.slot) == inplace.end()) inplace.push_back(in.view.slot);
   }
   auto may_alias = [&](const View& w) { return std::find(inplace.begin(), inplace.end(), w.slot) != inplace.end(); };
+  const std::string I = total < (int64_t{1} << 31) ? "unsigned" : "long long";  // coordinate arithmetic
   std::ostringstream src;
   src << kRtcPrelude << R"(extern "C" __global__ void __launch_bounds__(256) fused(
 )";
   for (size_t k = 0; k < ins.size(); ++k)
     src << "    const void* " << (may_alias(ins[k].view) ? "" : "__restrict__ ") << "p_in" << k << ",\n";
   src << "    void* " << (inplace.empty() ? "__restrict__ " : "") << "p_out, long long n) {\n";
-  src << "  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {\n";
+  src << "  for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * " << V << "; i < n; i += (long long)gridDim.x * "
+      << 256 * V << ") {\n";
+  if (V > 1 && total % V != 0) src << "    const bool whole = i + " << V << " <= n;\n";
   if (need_idx) {
-    src << "    long long q = i;\n";
-    for (int d = os.rank() - 1; d >= 0; --d) {
-      src << "    const long long " << idx_names[d] << " = q % " << os.dims[d] << "LL;";
-      if (d > 0) src << " q /= " << os.dims[d] << "LL;";
+    src << "    " << I << " q = (" << I << ")i;\n";
+    for (int d = rank - 1; d >= 0; --d) {
+      src << "    const long long " << idx_names[d] << " = (long long)(q % (" << I << ")" << os.dims[d] << "LL);";
+      if (d > 0) src << " q /= (" << I << ")" << os.dims[d] << "LL;";
       src << "\n";
     }
   }
-  src << body.str();
-  src << "    ((" << stype(os.dtype) << "*)p_out)[i] = " << store_expr(os.dtype, expr[v]) << ";\n  }\n}\n";
+  // x<k>[V]: the stored elements of input k (an input that repeats along the last
+  // axis: the same element V times).
+  for (size_t k = 0; k < ins.size(); ++k) {
+    const In& in = ins[k];
+    const std::string ks = std::to_string(k);
+    const std::string T = in.partial ? "float" : stype(N[in.value].shape.dtype);
+    std::string off_e = "i";
+    if (!in.linear) {
+      off_e = "0";
+      for (int d = 0; d < rank; ++d)
+        if (in.eff[d] != 0 && os.dims[d] != 1) off_e += " + " + idx_names[d] + " * " + std::to_string(in.eff[d]) + "LL";
+    }
+    const int64_t last = rank && inner != 1 ? in.eff[rank - 1] : 0;
+    src << "    " << T << " x" << ks << "[" << V << "];\n    {\n      const " << T << "* src = (const " << T << "*)p_in" << ks
+        << " + (" << off_e << ");\n";
+    if (V > 1 && (in.linear || last == 1)) {
+      // One vector load at element alignment (any view offset or caller's base; gfx950
+      // needs no more for 16 bytes).
+      src << "      struct __attribute__((packed)) W { " << T << " x[" << V << "]; };\n";
+      if (total % V != 0) src << "      if (whole) {\n";
+      src << "      const W w = *(const W*)src;\n#pragma unroll\n      for (int e = 0; e < " << V << "; ++e) x" << ks << "[e] = w.x[e];\n";
+      if (in.partial)
+        src << "#pragma unroll\n      for (int j = 1; j < " << in.splits << "; ++j) {\n        const W u = *(const W*)(src + (long long)j * "
+            << total << "LL);\n#pragma unroll\n        for (int e = 0; e < " << V << "; ++e) x" << ks << "[e] += u.x[e];\n      }\n";
+      if (total % V != 0) {
+        src << "      } else {\n#pragma unroll\n        for (int e = 0; e < " << V << "; ++e) {\n          const " << T
+            << "* p = src + (i + e < n ? e : 0);\n          x" << ks << "[e] = *p;\n";
+        if (in.partial)
+          src << "          for (int j = 1; j < " << in.splits << "; ++j) x" << ks << "[e] += p[(long long)j * " << total << "LL];\n";
+        src << "        }\n      }\n";
+      }
+    } else {
+      src << "#pragma unroll\n      for (int e = 0; e < " << V << "; ++e) x" << ks << "[e] = src[" << (last == 0 ? std::string("0") : "e * " + std::to_string(last) + "LL")
+          << "];\n";
+      if (in.partial)
+        src << "      for (int j = 1; j < " << in.splits << "; ++j) x" << ks << "[0] += src[(long long)j * " << total << "LL];\n";
+    }
+    src << "    }\n";
+  }
+  src << "    struct __attribute__((packed)) O { " << stype(os.dtype) << " x[" << V
+      << "]; } r;\n#pragma unroll\n    for (int e = 0; e < " << V << "; ++e) {\n"
+      << body.str() << "      r.x[e] = " << store_expr(os.dtype, expr[v]) << ";\n    }\n    " << stype(os.dtype) << "* dst = ("
+      << stype(os.dtype) << "*)p_out + i;\n";
+  if (V > 1 && total % V != 0)
+    src << "    if (!whole) {\n#pragma unroll\n      for (int e = 0; e < " << V << "; ++e)\n        if (i + e < n) dst[e] = r.x[e];\n"
+        << "    } else\n";
+  src << "    *(O*)dst = r;\n  }\n}\n";
   const std::string code = src.str();
   RtcKernel kern;
   if (rtc_get(be, code, "fused", &kern, err) != GHIP_OK) return bad();
   View y = fresh(os);
-  const int64_t total = os.size();
   std::vector<int> rd;
   std::vector<View> in_views;
   std::vector<int> in_dt;
@@ -2668,7 +2717,7 @@ View Lowerer::emit_cluster(int root, int v) {
     for (size_t k = 0; k < ptrs.size(); ++k) args.push_back(&ptrs[k]);
     args.push_back(&outp);
     args.push_back(&nn);
-    int64_t g = (total + 255) / 256;
+    int64_t g = ((total + V - 1) / V + 255) / 256;
     if (g > 16384) g = 16384;
     hipError_t h = hipModuleLaunchKernel(kern.func, static_cast<unsigned>(g), 1, 1, 256, 1, 1, 0, st.stream, args.data(), nullptr);
     if (h != hipSuccess) return check_hip(h, e, "generated elementwise kernel launch");
