@@ -236,14 +236,6 @@ struct CopyDesc {
 };
 int launch_strided_copy(int elem_bytes, const void* src, void* dst, const CopyDesc& d,
                         hipStream_t s, GHipError* err);
-// out[o] = reduce over r of src[o-offset + r-offset]; out is contiguous over odims.
-struct ReduceDesc {
-  int orank = 0, rrank = 0;
-  int64_t odims[kMaxRank], ost[kMaxRank];
-  int64_t rdims[kMaxRank], rst[kMaxRank];
-};
-int launch_reduce(int dtype, int op, const void* src, const ReduceDesc& d, void* dst,
-                  hipStream_t s, GHipError* err);
 // Gather rows with int32 or int64 ids (clamped).
 int launch_gather_rows(const void* table, int64_t V, int64_t row_bytes, const void* ids,
                        int id_dtype, int64_t n, void* out, hipStream_t s, GHipError* err);

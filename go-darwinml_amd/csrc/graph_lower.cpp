@@ -910,39 +910,7 @@ struct Lowerer {
     return y;
   }
 
-  View emit_reduce(int v) {
-    if (reduce_prod[v] >= 0) return emit_reduce_fused(v, reduce_prod[v], -1);
-    const Node& n = N[v];
-    const Shape& xs = N[n.in[0]].shape;
-    View x = get(n.in[0]);
-    if (failed) return bad();
-    ReduceDesc d;
-    for (int i = 0; i < xs.rank(); ++i) {
-      if (std::find(n.a0.begin(), n.a0.end(), i) != n.a0.end()) {
-        d.rdims[d.rrank] = xs.dims[i];
-        d.rst[d.rrank++] = x.strides[i];
-      } else {
-        d.odims[d.orank] = xs.dims[i];
-        d.ost[d.orank++] = x.strides[i];
-      }
-    }
-    if (d.orank == 0) {  // scalar output
-      d.odims[0] = 1;
-      d.ost[0] = 0;
-      d.orank = 1;
-    }
-    if (d.rrank == 0) {
-      d.rdims[0] = 1;
-      d.rst[0] = 0;
-      d.rrank = 1;
-    }
-    View y = fresh(n.shape);
-    const int dt = xs.dtype, op = n.sub;
-    static const char* names[] = {"sum", "product", "max", "min"};
-    add_step(fmt("reduce_%s %s -> %s", names[op], xs.str().c_str(), n.shape.str().c_str()), {x.slot}, {y.slot},
-             [=](ExecState& st, GHipError* e) { return launch_reduce(dt, op, st.ptr(x, dt), d, st.ptr(y, dt), st.stream, e); });
-    return y;
-  }
+  View emit_reduce(int v) { return emit_reduce_fused(v, reduce_prod[v], -1); }
 
   View emit_argminmax(int v) {
     const Node& n = N[v];
@@ -2301,13 +2269,24 @@ std::string Lowerer::member_stmt(int u, std::map<int, std::string>& expr, const 
 
 
 // One generated kernel for Reduce R, evaluating its producer cluster (rooted at
-// prod_root, over R's input shape) on the fly instead of reading it from HBM,
-// and, when cons_root >= 0, the consumer cluster (over R's output shape) on the
-// reduced value before the one store.  The accumulation order is the generic
-// reduce kernels' (one wave per output, lanes striding the reduced index, then a
-// butterfly, when >= 64 values are reduced; else one thread per output in
-// order), and the reduced value is rounded to R's dtype before the consumers
-// see it, so results are bit-identical to the unfused plan.
+// prod_root, over R's input shape; -1: none) on the fly instead of reading it from
+// HBM, and, when cons_root >= 0, the consumer cluster (over R's output shape) on the
+// reduced value before the one store.  The accumulation order depends on R's shapes,
+// axes and dtype alone, and the reduced value is rounded to R's dtype before the
+// consumers see it, so results do not depend on what is fused.  Three forms:
+//   rows:    the reduced axes are the last ones.  A wave (few outputs: a workgroup of
+//            256 or 1024 threads) per output, V consecutive elements a lane and load.
+//   columns: one block of reduced axes before the last kept axes.  A workgroup takes
+//            TX vectors of V adjacent columns and strides the reduced index with its
+//            other lanes, so every load is coalesced; a butterfly, then LDS, combine.
+//   general: any other axes.  A wave per output (one thread below 64 values), an
+//            element a load.
+// The first two are bound by HBM; where they have too few workgroups to fill the chip
+// and enough data to pay for a second launch (from 2 MB read), the reduced range
+// splits over workgroups, whose partial results a finishing kernel combines in order.
+// Measured, us, a wave per output with an element a load / here: bf16 [4096,2048] over
+// the rows, product fused 64 / 12.7 (8 ranges, both kernels); over the columns 19 / 5.8;
+// fp32 [256,10] to a scalar 12.7 / 2.0; [256,512] over the rows 5.3 / 4.4.
 View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
   const Node& rn = N[R];
   const int x = rn.in[0];
@@ -2321,41 +2300,100 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
   for (int i : kept) osize *= xs.dims[i];
   for (int i : red) rsize *= xs.dims[i];
   const int rdt = rs.dtype, xdt = xs.dtype;
-  const bool wave = rsize >= 64;
-  // Accumulator type of the generic reduce kernels (RAcc).
+  // ---- form and launch shape
+  const int64_t last = rx ? xs.dims[rx - 1] : 1;
+  int64_t inner = 1;  // kept elements after the last reduced axis
+  for (int i = red.empty() ? 0 : red.back() + 1; i < rx; ++i) inner *= xs.dims[i];
+  bool block = !red.empty();  // reduced axes adjacent
+  for (size_t k = 1; k < red.size(); ++k) block = block && red[k] == red[k - 1] + 1;
+  const bool rows = block && red.back() == rx - 1 && rsize >= 64;
+  const bool cols = block && !rows && inner >= 8 && osize > 0 && rsize > 0;
+  int V = 1;
+  if (rows || cols) {
+    V = std::max(1, 16 / dtype_size(xdt));
+    while (V > 1 && (last % V != 0 || (rows ? rsize / V < 64 : inner / V < 8))) V /= 2;
+  }
+  int64_t C = 1;                     // ranges of the reduced index
+  int L = 64, NT = 256;              // rows: lanes per output
+  int TX = 64;                       // columns: vectors per workgroup
+  int64_t gx = 0, cblocks = 1;
+  const int64_t bytes = osize * rsize * dtype_size(xdt);
+  const bool split_pays = bytes >= (int64_t{1} << 21);
+  if (rows) {
+    if (osize <= 256 && rsize >= 2048 * V) L = 1024;
+    else if (osize <= 1024 && rsize >= 512 * V) L = 256;
+    NT = std::max(256, L);
+    gx = (osize + NT / L - 1) / (NT / L);
+    if (split_pays && osize > 0 && gx < 128) C = std::min<int64_t>(256 / gx, rsize / (int64_t{4} * L * V));
+  } else if (cols) {
+    const int64_t outer = osize / inner, vecs = (inner + V - 1) / V;
+    while (TX > 1 && TX / 2 >= vecs) TX /= 2;
+    // Narrower column blocks until the chip is full, down to a 128-byte line.
+    while (TX > 1 && TX * V * dtype_size(xdt) > 128 && outer * ((vecs + TX - 1) / TX) < 512) TX /= 2;
+    cblocks = (vecs + TX - 1) / TX;
+    gx = outer * cblocks;
+    NT = rsize >= 512 && gx < 1024 ? 1024 : 256;
+    if (split_pays && gx < 128) C = std::min<int64_t>(256 / gx, rsize / (int64_t{4} * (NT / TX)));
+  } else {
+    gx = rsize >= 64 ? (osize + 3) / 4 : (osize + 255) / 256;
+  }
+  if (C < 2) C = 1;
+  const int64_t unit = rows ? static_cast<int64_t>(L) * V : cols ? NT / TX : 1;
+  const int64_t chunk = C > 1 ? (rsize + C * unit - 1) / (C * unit) * unit : rsize;
+  if (C > 1) C = (rsize + chunk - 1) / chunk;
+  if (gx > 0x7fffffffLL) return fail(GHIP_ERR_UNSUPPORTED, "Reduce: too many outputs");
+  const bool wave = !rows && !cols && rsize >= 64;
+  // Accumulator type (fp32, fp64 or 64-bit integers).
   std::string acc_t = "float";
   if (rdt == GHIP_DTYPE_FLOAT64) acc_t = "double";
   else if (dtype_is_int(rdt)) acc_t = dtype_is_unsigned(rdt) ? "unsigned long long" : "long long";
   struct In {
     View view;
     int dt;
-    std::string off;  // element offset expression
   };
   std::vector<In> ins;
-  std::ostringstream pbody, cbody;
+  std::ostringstream loads, pbody, cbody;
   std::map<int, std::string> expr;
-  // Input coordinates: x_i for input axis i (kept axes from the output index,
-  // reduced axes from the reduced index); output coordinates o_k.
-  auto load_input = [&](int o, const std::vector<std::string>& coord, const Shape& cs, std::ostringstream& body) {
+  // Input coordinates: x axis i from the output index (kept, o_k) or the reduced index
+  // (r_k); the last axis steps with e over a vector.  Output coordinates o_k.
+  auto load_input = [&](int o, const std::vector<std::string>& coord, const Shape& cs, int vec, std::ostringstream& body) {
     View w = get(o);
     if (failed) return;
     const Shape& sh = N[o].shape;
     const int off = cs.rank() - sh.rank();
-    std::string e = "0";
+    const std::string ks = std::to_string(ins.size()), T = stype(sh.dtype);
+    std::string base = "0";
+    int64_t step = 0;
     for (int d = 0; d < sh.rank(); ++d)
-      if (sh.dims[d] != 1 && w.strides[d] != 0) e += " + " + coord[off + d] + " * " + std::to_string(w.strides[d]) + "LL";
-    const int k = static_cast<int>(ins.size());
-    body << "      const " << ctype(sh.dtype) << " in" << k << " = "
-         << load_expr(sh.dtype, "((const " + stype(sh.dtype) + "*)p_in" + std::to_string(k) + ")[" + e + "]") << ";\n";
-    expr[o] = "in" + std::to_string(k);
-    ins.push_back(In{w, sh.dtype, e});
+      if (sh.dims[d] != 1 && w.strides[d] != 0) {
+        base += " + " + coord[off + d] + " * " + std::to_string(w.strides[d]) + "LL";
+        if (off + d == cs.rank() - 1) step = w.strides[d];
+      }
+    expr[o] = "in" + ks;
+    ins.push_back(In{w, sh.dtype});
+    const std::string src = "((const " + T + "*)p_in" + ks + " + (" + base + "))";
+    if (vec == 0) {  // consumer: one element
+      body << "      const " << ctype(sh.dtype) << " in" << ks << " = " << load_expr(sh.dtype, "*" + src) << ";\n";
+      return;
+    }
+    loads << "      " << T << " x" << ks << "[" << vec << "];\n      {\n        const " << T << "* src = " << src << ";\n";
+    if (vec > 1 && step == 1)
+      loads << "        struct __attribute__((packed)) W { " << T << " x[" << vec << "]; };\n        const W w = *(const W*)src;\n"
+            << "#pragma unroll\n        for (int e = 0; e < " << vec << "; ++e) x" << ks << "[e] = w.x[e];\n      }\n";
+    else
+      loads << "#pragma unroll\n        for (int e = 0; e < " << vec << "; ++e) x" << ks << "[e] = src[e * " << step << "LL];\n      }\n";
+    body << "      const " << ctype(sh.dtype) << " in" << ks << " = " << load_expr(sh.dtype, "x" + ks + "[e]") << ";\n";
   };
-  auto cluster_code = [&](int root, const Shape& cs, const std::vector<std::string>& coord, std::ostringstream& body,
-                          const std::set<int>& preset) {
+  auto cluster_code = [&](int root, const Shape& cs, const std::vector<std::string>& coord, int vec,
+                          std::ostringstream& body, const std::set<int>& preset) {
     std::vector<int> mem;
     for (int u = 0; u <= root; ++u)
       if (cluster[u] == root) mem.push_back(u);
     std::set<int> inset(mem.begin(), mem.end());
+    auto iota = [&](int u) {
+      const int ax = static_cast<int>(N[u].i0);
+      return "((" + ctype(N[u].shape.dtype) + ")(" + coord[ax] + (vec > 0 && ax == cs.rank() - 1 ? " + e" : "") + "))";
+    };
     for (int u : mem) {
       for (int o : N[u].in) {
         if (o < 0 || inset.count(o) || expr.count(o) || preset.count(o)) continue;
@@ -2365,16 +2403,16 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
           continue;
         }
         if (N[o].kind == Kind::Iota && N[o].shape.dims == cs.dims) {
-          expr[o] = "((" + ctype(N[o].shape.dtype) + ")" + coord[N[o].i0] + ")";
+          expr[o] = iota(o);
           continue;
         }
-        load_input(o, coord, cs, body);
+        load_input(o, coord, cs, vec, body);
         if (failed) return;
       }
       if (N[u].kind == Kind::Iota) {
         const std::string name = "v" + std::to_string(u);
-        body << "      const " << ctype(N[u].shape.dtype) << " " << name << " = "
-             << round_expr(N[u].shape.dtype, "((" + ctype(N[u].shape.dtype) + ")" + coord[N[u].i0] + ")") << ";\n";
+        body << "      const " << ctype(N[u].shape.dtype) << " " << name << " = " << round_expr(N[u].shape.dtype, iota(u))
+             << ";\n";
         expr[u] = name;
       } else {
         body << "  " << member_stmt(u, expr, "v" + std::to_string(u));
@@ -2388,21 +2426,21 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
   // element value fed to the accumulator
   std::string val;
   if (prod_root >= 0) {
-    cluster_code(prod_root, xs, xc, pbody, {});
+    cluster_code(prod_root, xs, xc, V, pbody, {});
     if (failed) return bad();
     val = round_expr(xdt, expr[prod_root]);
   } else {
-    load_input(x, xc, xs, pbody);
+    load_input(x, xc, xs, V, pbody);
     if (failed) return bad();
     val = expr[x];
   }
   // consumer cluster over the output shape, with R's value preset
-  std::string outv = "red", odt_s;
+  std::string outv = "red";
   int out_v = R, odt = rdt;
   if (cons_root >= 0) {
     expr.clear();  // the producer's names are scoped to the reduction loop
     expr[R] = "red";
-    cluster_code(cons_root, rs, oc, cbody, {R});
+    cluster_code(cons_root, rs, oc, 0, cbody, {R});
     if (failed) return bad();
     out_v = cons_root;
     odt = N[cons_root].shape.dtype;
@@ -2421,49 +2459,116 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
       init = acc_t == "float" ? "__builtin_inff()" : acc_t == "double" ? "__builtin_inf()"
            : acc_t == "long long" ? "9223372036854775807LL" : "18446744073709551615ull";
   }
+  std::string params, args_s;
+  for (size_t k = 0; k < ins.size(); ++k) {
+    params += "const void* __restrict__ p_in" + std::to_string(k) + ", ";
+    args_s += "p_in" + std::to_string(k) + ", ";
+  }
+  const std::string ws_t = acc_t + "* __restrict__ p_ws";
+  // Coordinates: 32-bit where the index fits.
+  auto coords = [&](const std::string& idx, const std::vector<int>& axes, const char* name, int64_t size, const char* ind) {
+    std::ostringstream s;
+    const std::string I = size < (int64_t{1} << 31) ? "unsigned" : "long long";
+    if (axes.size() == 1) {
+      s << ind << "const long long " << name << "0 = " << idx << ";\n";
+    } else if (!axes.empty()) {
+      s << ind << I << " q_" << name << " = (" << I << ")(" << idx << ");\n";
+      for (int k = static_cast<int>(axes.size()) - 1; k >= 0; --k)
+        s << ind << "const long long " << name << k << " = (long long)(q_" << name << " % (" << I << ")" << xs.dims[axes[k]]
+          << "LL); q_" << name << " /= (" << I << ")" << xs.dims[axes[k]] << "LL;\n";
+    }
+    return s.str();
+  };
+  std::ostringstream pre;
+  pre << kRtcPrelude << "__device__ __forceinline__ " << acc_t << " comb(" << acc_t << " a, " << acc_t << " b) { return "
+      << ops[rn.sub] << "; }\n"
+      // Output o from its reduced value, which is rounded as the unfused plan stores it.
+      << "__device__ __forceinline__ void finish(long long o, " << acc_t << " acc, " << params << "void* __restrict__ p_out) {\n"
+      << coords("o", kept, "o", osize, "  ") << "  const " << ctype(rdt) << " red = "
+      << load_expr(rdt, "(" + stype(rdt) + ")(" + store_expr(rdt, "(" + ctype(rdt) + ")acc") + ")") << ";\n"
+      << cbody.str() << "  ((" << stype(odt) << "*)p_out)[o] = " << store_expr(odt, outv) << ";\n}\n";
+  auto done = [&](const std::string& o, const std::string& a) {
+    return C > 1 ? "p_ws[(long long)blockIdx.y * " + std::to_string(osize) + "LL + " + o + "] = " + a + ";"
+                 : "finish(" + o + ", " + a + ", " + args_s + "p_out);";
+  };
   std::ostringstream src;
-  src << kRtcPrelude << "__device__ __forceinline__ " << acc_t << " comb(" << acc_t << " a, " << acc_t << " b) { return "
-      << ops[rn.sub] << "; }\n";
-  src << "extern \"C\" __global__ void __launch_bounds__(256) fused_reduce(\n";
-  for (size_t k = 0; k < ins.size(); ++k) src << "    const void* __restrict__ p_in" << k << ",\n";
-  src << "    void* __restrict__ p_out) {\n";
-  if (wave)
-    src << "  const long long o = (long long)blockIdx.x * 4 + threadIdx.x / 64;\n  const int lane = threadIdx.x % 64;\n";
-  else
-    src << "  const long long o = (long long)blockIdx.x * 256 + threadIdx.x;\n";
-  src << "  if (o >= " << osize << "LL) return;\n";
-  // output coordinates
-  if (kept.size() == 1) {
-    src << "  const long long o0 = o;\n";
-  } else if (!kept.empty()) {
-    src << "  long long q = o;\n";
-    for (int k = static_cast<int>(kept.size()) - 1; k >= 0; --k)
-      src << "  const long long o" << k << " = q % " << xs.dims[kept[k]] << "LL; q /= " << xs.dims[kept[k]] << "LL;\n";
-  }
-  src << "  " << acc_t << " acc = " << init << ";\n";
-  src << (wave ? "  for (long long r = lane; r < " : "  for (long long r = 0; r < ") << rsize << "LL; r += " << (wave ? 64 : 1)
-      << ") {\n";
-  if (red.size() == 1) {
-    src << "      const long long r0 = r;\n";
+  src << pre.str() << "extern \"C\" __global__ void __launch_bounds__(" << NT << ") fused_reduce(" << params
+      << "void* __restrict__ p_out, " << ws_t << ") {\n  const int t = threadIdx.x;\n";
+  const std::string accs = "  " + acc_t + " acc[" + std::to_string(V) + "];\n#pragma unroll\n  for (int e = 0; e < " +
+                           std::to_string(V) + "; ++e) acc[e] = " + init + ";\n";
+  const std::string range = "  const long long r_end = " +
+      (C > 1 ? "((long long)blockIdx.y + 1) * " + std::to_string(chunk) + "LL < " + std::to_string(rsize) +
+                   "LL ? ((long long)blockIdx.y + 1) * " + std::to_string(chunk) + "LL : " + std::to_string(rsize) + "LL"
+             : std::to_string(rsize) + "LL") + ";\n";
+  const std::string start = C > 1 ? "(long long)blockIdx.y * " + std::to_string(chunk) + "LL + " : "";
+  auto step = [&]() {
+    std::ostringstream s;
+    s << coords("r", red, "r", rsize, "      ") << loads.str() << "#pragma unroll\n      for (int e = 0; e < " << V << "; ++e) {\n"
+      << pbody.str() << "      acc[e] = comb(acc[e], (" << acc_t << ")(" << val << "));\n      }\n    }\n";
+    return s.str();
+  };
+  if (rows) {
+    src << "  const int lane = t % " << L << ";\n  const long long o = (long long)blockIdx.x * " << NT / L << " + t / " << L << ";\n";
+    if (L == 64) src << "  if (o >= " << osize << "LL) return;\n";
+    src << coords("o", kept, "o", osize, "  ") << accs << range << "#pragma unroll 4\n  for (long long r = " << start << "lane * " << V
+        << "; r < r_end; r += " << L * V << ") {\n"
+        << step() << "  " << acc_t << " a = acc[0];\n#pragma unroll\n  for (int e = 1; e < " << V << "; ++e) a = comb(a, acc[e]);\n"
+        << "#pragma unroll\n  for (int off = 32; off >= 1; off >>= 1) a = comb(a, __shfl_xor(a, off, 64));\n";
+    if (L > 64)
+      src << "  __shared__ " << acc_t << " part[" << L / 64 << "];\n  if (t % 64 == 0) part[t / 64] = a;\n  __syncthreads();\n"
+          << "  if (t != 0) return;\n  for (int w = 1; w < " << L / 64 << "; ++w) a = comb(a, part[w]);\n";
+    else
+      src << "  if (lane != 0) return;\n";
+    src << "  " << done("o", "a") << "\n}\n";
+  } else if (cols) {
+    const int TY = NT / TX, NW = NT / 64;
+    // Kept index of the vector's first column: axes before the reduced block, then inner.
+    src << "  const int tx = t % " << TX << ", ty = t / " << TX << ";\n  const long long ou = blockIdx.x / " << cblocks
+        << ", col = ((long long)(blockIdx.x % " << cblocks << ") * " << TX << " + tx) * " << V << ";\n"
+        << "  const bool ok = col < " << inner << "LL;\n  const long long o = ou * " << inner << "LL + (ok ? col : 0);\n"
+        << coords("o", kept, "o", osize, "  ") << accs << range << "#pragma unroll 4\n  for (long long r = " << start << "ty; r < r_end; r += "
+        << TY << ") {\n" << step();
+    const int W = std::max(TX, 1);
+    if (TX < 64)
+      src << "#pragma unroll\n  for (int off = " << TX << "; off <= 32; off <<= 1)\n#pragma unroll\n    for (int e = 0; e < " << V
+          << "; ++e) acc[e] = comb(acc[e], __shfl_xor(acc[e], off, 64));\n";
+    src << "  __shared__ " << acc_t << " part[" << NW << "][" << W * V << "];\n  if (t % 64 < " << TX << ")\n#pragma unroll\n    for (int e = 0; e < "
+        << V << "; ++e) part[t / 64][tx * " << V << " + e] = acc[e];\n  __syncthreads();\n"
+        << "  for (int c = t; c < " << W * V << "; c += " << NT << ") {\n    const long long oc = (long long)(blockIdx.x % " << cblocks << ") * "
+        << TX * V << " + c;\n    if (oc >= " << inner << "LL) return;\n    " << acc_t << " a = part[0][c];\n    for (int w = 1; w < " << NW
+        << "; ++w) a = comb(a, part[w][c]);\n    const long long of = ou * " << inner << "LL + oc;\n    " << done("of", "a") << "\n  }\n}\n";
   } else {
-    src << "      long long t = r;\n";
-    for (int k = static_cast<int>(red.size()) - 1; k >= 0; --k)
-      src << "      const long long r" << k << " = t % " << xs.dims[red[k]] << "LL; t /= " << xs.dims[red[k]] << "LL;\n";
+    if (wave) src << "  const long long o = (long long)blockIdx.x * 4 + t / 64;\n  const int lane = t % 64;\n";
+    else src << "  const long long o = (long long)blockIdx.x * 256 + t;\n";
+    src << "  if (o >= " << osize << "LL) return;\n" << coords("o", kept, "o", osize, "  ") << accs << "  for (long long r = "
+        << (wave ? "lane" : "0") << "; r < " << rsize << "LL; r += " << (wave ? 64 : 1) << ") {\n"
+        << step() << "  " << acc_t << " a = acc[0];\n";
+    if (wave)
+      src << "#pragma unroll\n  for (int off = 32; off >= 1; off >>= 1) a = comb(a, __shfl_xor(a, off, 64));\n  if (lane != 0) return;\n";
+    src << "  " << done("o", "a") << "\n}\n";
   }
-  src << pbody.str() << "      acc = comb(acc, (" << acc_t << ")(" << val << "));\n  }\n";
-  if (wave) {
-    src << "#pragma unroll\n  for (int off = 32; off >= 1; off >>= 1) acc = comb(acc, __shfl_xor(acc, off, 64));\n"
-        << "  if (lane != 0) return;\n";
-  }
-  // the reduced value as the unfused plan stores it, read back in compute type
-  src << "  const " << ctype(rdt) << " red = " << load_expr(rdt, "(" + stype(rdt) + ")(" + store_expr(rdt, "(" + ctype(rdt) + ")acc") + ")") << ";\n";
-  src << cbody.str();
-  src << "  ((" << stype(odt) << "*)p_out)[o] = " << store_expr(odt, outv) << ";\n}\n";
-  RtcKernel kern;
+  RtcKernel kern, fin;
   if (rtc_get(be, src.str(), "fused_reduce", &kern, err) != GHIP_OK) return bad();
+  if (C > 1) {
+    std::ostringstream fs;
+    fs << pre.str() << "extern \"C\" __global__ void __launch_bounds__(256) reduce_finish(" << params << "void* __restrict__ p_out, "
+       << ws_t << ") {\n  const long long o = (long long)blockIdx.x * 256 + threadIdx.x;\n  if (o >= " << osize << "LL) return;\n  "
+       << acc_t << " a = p_ws[o];\n#pragma unroll 16\n  for (int c = 1; c < " << C << "; ++c) a = comb(a, p_ws[o + c * " << osize
+       << "LL]);\n  finish(o, a, " << args_s << "p_out);\n}\n";
+    if (rtc_get(be, fs.str(), "reduce_finish", &fin, err) != GHIP_OK) return bad();
+  }
   const Shape& os = N[out_v].shape;
   View y = fresh(os);
-  std::vector<int> rd;
+  View wsv;
+  std::vector<int> rd, wr{y.slot};
+  const int wdt = acc_t == "float" ? GHIP_DTYPE_FLOAT32 : GHIP_DTYPE_INT64;
+  if (C > 1) {
+    Shape wss;
+    wss.dtype = wdt;
+    wss.dims = {C * osize};
+    wsv = fresh(wss);
+    wr.push_back(wsv.slot);
+  }
   std::vector<View> in_views;
   std::vector<int> in_dt;
   for (auto& in : ins) {
@@ -2472,20 +2577,26 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
     in_dt.push_back(in.dt);
   }
   static const char* names[] = {"sum", "product", "max", "min"};
-  std::string desc = fmt("fused_reduce_%s %s -> %s", names[rn.sub], xs.str().c_str(), os.str().c_str());
+  const bool fused = prod_root >= 0 || cons_root >= 0;
+  std::string desc = fmt("%sreduce_%s %s -> %s", fused ? "fused_" : "", names[rn.sub], xs.str().c_str(), os.str().c_str());
   if (prod_root >= 0) desc += " (producer fused)";
   if (cons_root >= 0) desc += " (consumer fused)";
-  const int64_t blocks = wave ? (osize + 3) / 4 : (osize + 255) / 256;
-  add_step(desc, rd, {y.slot}, [=](ExecState& st, GHipError* e) -> int {
+  if (C > 1) desc += fmt(" (in %lld ranges)", (long long)C);
+  add_step(desc, rd, wr, [=](ExecState& st, GHipError* e) -> int {
     if (osize == 0) return GHIP_OK;
     std::vector<void*> ptrs(in_views.size());
     std::vector<void*> args;
     for (size_t k = 0; k < in_views.size(); ++k) ptrs[k] = st.ptr(in_views[k], in_dt[k]);
     void* outp = st.ptr(y, odt);
+    void* wsp = C > 1 ? st.ptr(wsv, wdt) : nullptr;
     for (size_t k = 0; k < ptrs.size(); ++k) args.push_back(&ptrs[k]);
     args.push_back(&outp);
-    hipError_t h = hipModuleLaunchKernel(kern.func, static_cast<unsigned>(blocks), 1, 1, 256, 1, 1, 0, st.stream,
-                                         args.data(), nullptr);
+    args.push_back(&wsp);
+    hipError_t h = hipModuleLaunchKernel(kern.func, static_cast<unsigned>(gx), static_cast<unsigned>(C), 1, NT, 1, 1, 0,
+                                         st.stream, args.data(), nullptr);
+    if (h == hipSuccess && C > 1)
+      h = hipModuleLaunchKernel(fin.func, static_cast<unsigned>((osize + 255) / 256), 1, 1, 256, 1, 1, 0, st.stream,
+                                args.data(), nullptr);
     if (h != hipSuccess) return check_hip(h, e, "generated reduce kernel launch");
     return GHIP_OK;
   });

@@ -124,142 +124,6 @@ int launch_strided_copy(int elem_bytes, const void* src, void* dst, const CopyDe
 }
 
 // ---------------------------------------------------------------------------
-// Reductions.  Accumulator: fp32 for fp32/bf16/fp16, fp64 for fp64, int64 /
-// uint64 for integers.  One wave per output when the reduced extent is >= 64
-// (lanes stride the reduced index space, then a butterfly), else one thread per
-// output.
-// ---------------------------------------------------------------------------
-template <typename T> struct RAcc { using type = float; };
-template <> struct RAcc<double> { using type = double; };
-template <> struct RAcc<int8_t> { using type = int64_t; };
-template <> struct RAcc<int16_t> { using type = int64_t; };
-template <> struct RAcc<int32_t> { using type = int64_t; };
-template <> struct RAcc<int64_t> { using type = int64_t; };
-template <> struct RAcc<uint8_t> { using type = uint64_t; };
-template <> struct RAcc<uint16_t> { using type = uint64_t; };
-template <> struct RAcc<uint32_t> { using type = uint64_t; };
-template <> struct RAcc<uint64_t> { using type = uint64_t; };
-
-template <typename T> __device__ __forceinline__ typename RAcc<T>::type rload(const T* p) { return *p; }
-template <> __device__ __forceinline__ float rload<bf16_t>(const bf16_t* p) { return bf16_to_f32(p->bits); }
-template <> __device__ __forceinline__ float rload<_Float16>(const _Float16* p) { return static_cast<float>(*p); }
-
-template <typename T> __device__ __forceinline__ void rstore(T* p, typename RAcc<T>::type v) { *p = static_cast<T>(v); }
-template <> __device__ __forceinline__ void rstore<bf16_t>(bf16_t* p, float v) { p->bits = f32_to_bf16(v); }
-template <> __device__ __forceinline__ void rstore<_Float16>(_Float16* p, float v) { *p = static_cast<_Float16>(v); }
-
-template <typename A>
-__device__ __forceinline__ A rcombine(A a, A b, int op) {
-  switch (op) {
-    case GHIP_REDUCE_SUM: return a + b;
-    case GHIP_REDUCE_PRODUCT: return a * b;
-    case GHIP_REDUCE_MAX: return (a > b || a != a) ? a : b;  // NaN propagates
-    default: return (a < b || a != a) ? a : b;
-  }
-}
-
-template <typename A>
-__device__ __forceinline__ A rinit(int op) {
-  switch (op) {
-    case GHIP_REDUCE_SUM: return A(0);
-    case GHIP_REDUCE_PRODUCT: return A(1);
-    case GHIP_REDUCE_MAX:
-      if constexpr (std::is_floating_point<A>::value) return -INFINITY;
-      else return std::numeric_limits<A>::lowest();
-    default:
-      if constexpr (std::is_floating_point<A>::value) return INFINITY;
-      else return std::numeric_limits<A>::max();
-  }
-}
-
-__device__ __forceinline__ int64_t offset_of(int64_t i, int rank, const int64_t* dims, const int64_t* st) {
-  int64_t off = 0;
-  for (int k = rank - 1; k >= 0; --k) {
-    off += (i % dims[k]) * st[k];
-    i /= dims[k];
-  }
-  return off;
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void reduce_thread_kernel(const T* __restrict__ src, T* __restrict__ dst,
-                                                            ReduceDesc d, int64_t osize, int64_t rsize,
-                                                            int op) {
-  using A = typename RAcc<T>::type;
-  const int64_t o = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (o >= osize) return;
-  const T* base = src + offset_of(o, d.orank, d.odims, d.ost);
-  A acc = rinit<A>(op);
-  for (int64_t r = 0; r < rsize; ++r) acc = rcombine<A>(acc, rload(base + offset_of(r, d.rrank, d.rdims, d.rst)), op);
-  rstore(dst + o, acc);
-}
-
-template <typename A>
-__device__ __forceinline__ A shfl_xor_any(A v, int off) {
-  if constexpr (sizeof(A) == 8) {
-    int64_t bits = __builtin_bit_cast(int64_t, v);
-    bits = __shfl_xor(bits, off, 64);
-    return __builtin_bit_cast(A, bits);
-  } else {
-    return __shfl_xor(v, off, 64);
-  }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void reduce_wave_kernel(const T* __restrict__ src, T* __restrict__ dst,
-                                                          ReduceDesc d, int64_t osize, int64_t rsize,
-                                                          int op) {
-  using A = typename RAcc<T>::type;
-  const int64_t o = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / 64;
-  if (o >= osize) return;
-  const int lane = threadIdx.x % 64;
-  const T* base = src + offset_of(o, d.orank, d.odims, d.ost);
-  A acc = rinit<A>(op);
-  for (int64_t r = lane; r < rsize; r += 64) acc = rcombine<A>(acc, rload(base + offset_of(r, d.rrank, d.rdims, d.rst)), op);
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) acc = rcombine<A>(acc, shfl_xor_any(acc, off), op);
-  if (lane == 0) rstore(dst + o, acc);
-}
-
-template <typename T>
-static hipError_t launch_reduce_t(const void* src, const ReduceDesc& d, void* dst, int op, hipStream_t s) {
-  int64_t osize = 1, rsize = 1;
-  for (int k = 0; k < d.orank; ++k) osize *= d.odims[k];
-  for (int k = 0; k < d.rrank; ++k) rsize *= d.rdims[k];
-  if (osize == 0) return hipSuccess;
-  if (rsize >= 64) {
-    hipLaunchKernelGGL(reduce_wave_kernel<T>, dim3(static_cast<unsigned>((osize + 3) / 4)), dim3(256), 0, s,
-                       static_cast<const T*>(src), static_cast<T*>(dst), d, osize, rsize, op);
-  } else {
-    hipLaunchKernelGGL(reduce_thread_kernel<T>, dim3(static_cast<unsigned>((osize + 255) / 256)), dim3(256), 0, s,
-                       static_cast<const T*>(src), static_cast<T*>(dst), d, osize, rsize, op);
-  }
-  return hipGetLastError();
-}
-
-int launch_reduce(int dtype, int op, const void* src, const ReduceDesc& d, void* dst, hipStream_t s,
-                  GHipError* err) {
-  hipError_t e;
-  switch (dtype) {
-    case GHIP_DTYPE_FLOAT32: e = launch_reduce_t<float>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_BFLOAT16: e = launch_reduce_t<bf16_t>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_FLOAT16: e = launch_reduce_t<_Float16>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_FLOAT64: e = launch_reduce_t<double>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_INT8: e = launch_reduce_t<int8_t>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_INT16: e = launch_reduce_t<int16_t>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_INT32: e = launch_reduce_t<int32_t>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_INT64: e = launch_reduce_t<int64_t>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_UINT8: e = launch_reduce_t<uint8_t>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_UINT16: e = launch_reduce_t<uint16_t>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_UINT32: e = launch_reduce_t<uint32_t>(src, d, dst, op, s); break;
-    case GHIP_DTYPE_UINT64: e = launch_reduce_t<uint64_t>(src, d, dst, op, s); break;
-    default: return set_error(err, GHIP_ERR_UNSUPPORTED, "reduce: dtype %d", dtype);
-  }
-  GHIP_CHECK(e, err);
-  return GHIP_OK;
-}
-
-// ---------------------------------------------------------------------------
 // Row gather with int32 / int64 ids (the public ghip_gather_rows takes int32).
 // ---------------------------------------------------------------------------
 // One wave per output row.  A wave issues the loads of up to 4 vectors per lane

@@ -1,0 +1,87 @@
+"""The generated reduce kernels' forms (rows, columns, general; whole or split into
+ranges) at the sizes where the form, vector width or launch shape changes, against
+numpy in float64, and with a fused producer bit for bit against the unfused plan.
+
+Bounds: a sum of n fp32 terms in any order is within n 2^-24 of sum |x| (here far
+fewer terms meet in one accumulator: 2^-20 is allowed); the result of a 16-bit
+reduction rounds once more (2^-8 bf16, 2^-11 f16).  Maxima and integers are exact."""
+import numpy as np
+import pytest
+
+from gomlx_hip import synth
+from gomlx_hip.backend import Backend, dtypes, make_shape
+
+pytestmark = pytest.mark.gpu
+
+F32, BF16, F16, I32 = dtypes.Float32, dtypes.BFloat16, dtypes.Float16, dtypes.Int32
+# (shape, reduced axes)
+CASES = [
+    ((3, 64), [1]), ((5, 1000), [1]), ((7, 1002), [1]), ((4, 513), [1]),          # rows, a wave each
+    ((1, 10000), [1]), ((600, 4096), [1]), ((2, 3, 40, 128), [2, 3]),             # wider groups, two axes
+    ((3, 1 << 20), [1]), ((256, 10), [0, 1]),                                     # split rows; everything
+    ((64, 8), [0]), ((2000, 64), [0]), ((7, 50, 24), [1]), ((3, 129, 9), [1]),    # columns
+    ((4096, 2048), [0]), ((2, 70000, 8), [1]), ((513, 130), [0]), ((6, 5, 4, 40), [1, 2]),
+    ((6, 40, 5), [0, 2]), ((70, 3), [0]), ((9, 7, 3), [1]),                       # general, wave and thread
+    ((0, 8), [0]), ((8, 0), [1]),                                                 # nothing to reduce
+]
+
+
+@pytest.fixture(scope="module")
+def be(cuda):
+    b = Backend("")
+    yield b
+    b.Finalize()
+
+
+def _run(be, shape, axes, dt, op, feed, square):
+    b = be.Builder("reduce")
+    f = b.Main()
+    x = f.Parameter("x", make_shape(dt, *shape))
+    f.Return([getattr(f, op)(f.Mul(x, x) if square else x, *axes)])
+    ex = b.Compile()
+    buf = be.BufferFromFlatData(0, feed, make_shape(dt, *shape))
+    (y,) = ex.Execute([buf])
+    s = be.BufferShape(y)
+    out = be.BufferToFlatData(y).reshape(s.dims).copy()
+    plan = ex.Plan()
+    ex.Finalize()
+    return (synth.bf16_bits_to_f32(out) if dt == BF16 else out), plan
+
+
+@pytest.mark.parametrize("shape,axes", CASES)
+@pytest.mark.parametrize("dt", [F32, BF16, F16, I32])
+def test_reduce_forms(be, shape, axes, dt, monkeypatch):
+    if dt == I32:
+        x = synth.uniform_f32(9001, shape, -1000, 1000).astype(np.int32)
+        feed = x
+    else:
+        x = synth.normal(9001, shape)
+        feed = synth.to_bf16_bits(x) if dt == BF16 else x.astype(np.float16) if dt == F16 else x
+        x = synth.round_bf16(x) if dt == BF16 else feed.astype(np.float32)
+    print(shape, axes, dt, flush=True)
+    x64 = x.astype(np.float64)
+    ax = tuple(axes)
+    got, plan = _run(be, shape, axes, dt, "ReduceSum", feed, False)
+    want = x64.sum(ax)
+    if dt == I32:
+        assert np.array_equal(got, want.astype(np.int64).astype(np.int32))
+    else:
+        err = np.abs(got.astype(np.float64) - want)
+        r = {F32: 0.0, BF16: 2.0 ** -8, F16: 2.0 ** -11}[dt]
+        assert np.all(err <= 2.0 ** -20 * np.abs(x64).sum(ax) + r * np.abs(want) + 2.0 ** -24), plan
+    if x.size:
+        assert np.array_equal(_run(be, shape, axes, dt, "ReduceMax", feed, False)[0].astype(np.float64), x64.max(ax))
+    fused, plan = _run(be, shape, axes, dt, "ReduceSum", feed, True)
+    monkeypatch.setenv("GHIP_REDUCE_FUSION", "0")
+    plain, _ = _run(be, shape, axes, dt, "ReduceSum", feed, True)
+    assert "producer fused" in plan and np.array_equal(fused, plain, equal_nan=True)
+
+
+def test_split_reduce_says_so(be):
+    for shape, axes in [((3, 1 << 20), [1]), ((4096, 2048), [0])]:
+        b = be.Builder("reduce")
+        f = b.Main()
+        f.Return([f.ReduceSum(f.Parameter("x", make_shape(F32, *shape)), *axes)])
+        ex = b.Compile()
+        assert "ranges)" in ex.Plan()
+        ex.Finalize()
