@@ -153,6 +153,9 @@ struct Lowerer {
   std::vector<char> live;
   std::vector<std::vector<int>> users;
   std::vector<int> cluster;  // elementwise cluster id (= root node) or -1
+  std::vector<std::vector<int>> members;  // per cluster root: its nodes, in node order
+  std::vector<char> copied;  // evaluated anew in each cluster that reads it (never stored)
+  std::vector<char> needed;  // reached by emission (not only inside a fused pattern)
   std::vector<Fusion> fusion;
   std::vector<char> have;
   std::vector<View> views;
@@ -220,8 +223,22 @@ struct Lowerer {
     fusion.assign(n, Fusion{});
     for (int v = n - 1; v >= 0; --v)
       if (live[v]) match_patterns(v);
+    find_copied();
     build_clusters();
     find_reduce_fusions();
+    needed.assign(n, 0);
+    stack.assign(fn->outputs.begin(), fn->outputs.end());
+    while (!stack.empty()) {
+      const int v = stack.back();
+      stack.pop_back();
+      if (v < 0 || needed[v]) continue;
+      needed[v] = 1;
+      if (fusion[v].kind != Fusion::None) {
+        for (int o : {fusion[v].x, fusion[v].gamma, fusion[v].beta}) stack.push_back(o);
+      } else {
+        for (int o : N[v].in) stack.push_back(o);
+      }
+    }
   }
 
   // ------------------------------------------------------------------ patterns
@@ -495,27 +512,83 @@ struct Lowerer {
     const Kind k = N[v].kind;
     return is_elementwise(k);
   }
+  // Values that the clusters reading v load in its place when v is evaluated inside
+  // them: v's operands, through the elementwise nodes that only v (or copied nodes)
+  // read.  False: not worth it, or too many nodes.
+  bool copy_leaves(int v, std::set<int>* leaves, int* nodes, const std::set<int>& outs) {
+    if (++*nodes > 8) return false;
+    for (int p : N[v].in) {
+      double c;
+      if (p < 0 || scalar_const(p, &c)) continue;
+      bool inside = clusterable(p) && !outs.count(p) && N[p].shape.dims == N[v].shape.dims;
+      for (int w : users[p]) inside = inside && (w == v || copied[w]);
+      if (inside || copied[p]) {
+        if (!copy_leaves(p, leaves, nodes, outs)) return false;
+        continue;
+      }
+      // A value that reaches only v is stored for v's sake alone, and a DotGeneral or
+      // Reduce that v could finish in its own kernel would have to be.
+      bool only_v = true;
+      for (int w : users[p]) only_v = only_v && (w == v || copied[w]);
+      if (only_v && (N[p].kind == Kind::Dot || N[p].kind == Kind::Reduce)) return false;
+      int q = p;
+      while (N[q].kind == Kind::Broadcast) q = N[q].in[0];
+      if (N[q].shape.size() * 4 > N[v].shape.size()) leaves->insert(p);
+    }
+    return true;
+  }
+  // Elementwise nodes with several readers, all elementwise at the node's shape: where
+  // at most one large value would be loaded in the node's place, every cluster that
+  // reads it evaluates it itself (in registers, the same rounding: the same bits), so
+  // it is neither stored nor read.  silu(x Wg) * (x Wu) and its gradient, bf16
+  // [4096, 8192]: logistic, silu and the product were kernels of 20, 31 and 31 us and
+  // are one of 31.
+  void find_copied() {
+    const int n = static_cast<int>(N.size());
+    copied.assign(n, 0);
+    std::set<int> outs(fn->outputs.begin(), fn->outputs.end());
+    for (int v = 0; v < n; ++v) {
+      if (!clusterable(v) || outs.count(v) || N[v].kind == Kind::Iota || users[v].size() < 2) continue;
+      bool ok = true, several = false;
+      for (int w : users[v]) {
+        ok = ok && clusterable(w) && N[w].kind != Kind::Iota && N[w].shape.dims == N[v].shape.dims;
+        several = several || w != users[v][0];
+      }
+      std::set<int> leaves;
+      int nodes = 0;
+      if (ok && several && copy_leaves(v, &leaves, &nodes, outs) && leaves.size() <= 1) copied[v] = 1;
+    }
+  }
   void build_clusters() {
     const int n = static_cast<int>(N.size());
     cluster.assign(n, -1);
+    members.assign(n, {});
     std::set<int> outs(fn->outputs.begin(), fn->outputs.end());
     for (int v = n - 1; v >= 0; --v) {
       if (!clusterable(v) || cluster[v] >= 0) continue;
       cluster[v] = v;  // new root
+      std::set<int> in{v};
       std::vector<int> work{v};
       while (!work.empty()) {
         const int u = work.back();
         work.pop_back();
         for (int o : N[u].in) {
-          if (o < 0 || cluster[o] >= 0 || !clusterable(o) || outs.count(o)) continue;
+          if (o < 0 || in.count(o) || !clusterable(o) || outs.count(o)) continue;
           if (N[o].shape.dims != N[v].shape.dims) continue;
-          bool all_in = true;
-          for (int w : users[o]) all_in = all_in && cluster[w] == v;
-          if (!all_in) continue;
+          bool all_in = cluster[o] < 0;
+          for (int w : users[o]) all_in = all_in && cluster[w] == v && !copied[w];
+          // Read only inside this cluster, or by copies of a node: its value goes where
+          // they go.
+          bool with_copies = !all_in;
+          for (int w : users[o]) with_copies = with_copies && copied[w];
+          if (with_copies) copied[o] = 1;
+          if (!all_in && !copied[o]) continue;
           cluster[o] = v;
+          in.insert(o);
           work.push_back(o);
         }
       }
+      members[v].assign(in.begin(), in.end());
     }
   }
 
@@ -537,10 +610,9 @@ struct Lowerer {
         if (c >= 0 && cons_reduce[c] < 0 && N[c].shape.dims == N[v].shape.dims) {
           // a cluster fed by a DotGeneral prefers the GEMM epilogue
           bool has_dot = false;
-          for (int w = 0; w <= c; ++w)
-            if (cluster[w] == c)
-              for (int o : N[w].in) has_dot = has_dot || (o >= 0 && N[o].kind == Kind::Dot);
-          if (!has_dot) cons_reduce[c] = v;
+          for (int w : members[c])
+            for (int o : N[w].in) has_dot = has_dot || (o >= 0 && N[o].kind == Kind::Dot);
+          if (!has_dot && !copied[u]) cons_reduce[c] = v;
         }
       }
     }
@@ -2386,9 +2458,7 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
   };
   auto cluster_code = [&](int root, const Shape& cs, const std::vector<std::string>& coord, int vec,
                           std::ostringstream& body, const std::set<int>& preset) {
-    std::vector<int> mem;
-    for (int u = 0; u <= root; ++u)
-      if (cluster[u] == root) mem.push_back(u);
+    const std::vector<int>& mem = members[root];
     std::set<int> inset(mem.begin(), mem.end());
     auto iota = [&](int u) {
       const int ax = static_cast<int>(N[u].i0);
@@ -2613,8 +2683,7 @@ View Lowerer::emit_cluster(int root, int v) {
   if (root >= 0 && cons_reduce[root] >= 0 && !have[cons_reduce[root]])
     return emit_reduce_fused(cons_reduce[root], reduce_prod[cons_reduce[root]], root);
   if (root >= 0) {
-    for (int u = 0; u <= root; ++u)
-      if (cluster[u] == root) mem.push_back(u);
+    mem = members[root];
     if (fuse_epilogues) {
       bool fused = false;
       View y = emit_gemm_epilogue(v, mem, &fused);
@@ -2625,6 +2694,48 @@ View Lowerer::emit_cluster(int root, int v) {
     mem.push_back(v);
   }
   const Shape& os = N[v].shape;
+  // Other clusters of the same shape whose operands are all at hand and that read a
+  // large operand of this one join its kernel as further outputs: the shared operands
+  // are read once.
+  std::vector<int> roots{v};
+  if (root >= 0) {
+    auto externals = [&](const std::vector<int>& ms) {
+      std::set<int> in(ms.begin(), ms.end()), ext;
+      for (int u : ms)
+        for (int o : N[u].in) {
+          double c;
+          if (o >= 0 && !in.count(o) && !scalar_const(o, &c) && N[o].kind != Kind::Iota) ext.insert(o);
+        }
+      return ext;
+    };
+    std::set<int> mine = externals(mem);
+    auto at_hand = [&](int o) {
+      while (!have[o] && (N[o].kind == Kind::Broadcast || N[o].kind == Kind::Reshape || N[o].kind == Kind::Transpose))
+        o = N[o].in[0];
+      return have[o] || mine.count(o) || N[o].kind == Kind::Param || N[o].kind == Kind::Const || N[o].kind == Kind::Capture;
+    };
+    const int n = static_cast<int>(N.size());
+    size_t inputs = mine.size();
+    for (int w = 0; w < n && roots.size() < 4; ++w) {
+      if (w == v || cluster[w] != w || !needed[w] || have[w] || N[w].shape.dims != os.dims || os.size() < 65536) continue;
+      if (cons_reduce[w] >= 0 && !have[cons_reduce[w]]) continue;
+      bool into_reduce = false;  // absorbed by a Reduce
+      for (int r : users[w]) into_reduce = into_reduce || (N[r].kind == Kind::Reduce && reduce_prod[r] == w);
+      if (into_reduce) continue;
+      const std::set<int> ext = externals(members[w]);
+      bool ok = !ext.empty(), shares = false;
+      for (int o : ext) {
+        ok = ok && at_hand(o) && o != v;
+        shares = shares || (mine.count(o) && N[o].shape.dims == os.dims && N[o].kind != Kind::Broadcast);
+      }
+      if (!ok || !shares || inputs + ext.size() > 12) continue;
+      roots.push_back(w);
+      inputs += ext.size();
+      for (int u : members[w])
+        if (std::find(mem.begin(), mem.end(), u) == mem.end()) mem.push_back(u);
+    }
+    std::sort(mem.begin(), mem.end());
+  }
   std::set<int> inset(mem.begin(), mem.end());
   const int64_t total = os.size();
   const int rank = os.rank();
@@ -2713,7 +2824,9 @@ View Lowerer::emit_cluster(int root, int v) {
   // the loads' latency better than wider loads.  A vector stays inside a row of the
   // last axis when coordinates are needed.  Bound by HBM; bf16 [4096, 8192], two
   // inputs: 41 us (4.9 TB/s) with an element a thread, 31 (6.5 TB/s) with eight.
-  int V = std::max(1, 16 / dtype_size(os.dtype));
+  int widest = 1;
+  for (int r : roots) widest = std::max(widest, dtype_size(N[r].shape.dtype));
+  int V = std::max(1, 16 / widest);
   while (V > 1 && (total / V < 65536 || (need_idx && inner % V != 0))) V /= 2;
   const std::string Vs = std::to_string(V);
   // Slots every read of which is at the output's own element index (linear,
@@ -2723,7 +2836,7 @@ View Lowerer::emit_cluster(int root, int v) {
   // vector all precede its store.)
   std::vector<int> inplace;
   for (auto& in : ins) {
-    bool ok = !in.partial;
+    bool ok = !in.partial && roots.size() == 1;
     for (auto& o2 : ins)
       if (o2.view.slot == in.view.slot)
         ok = ok && !o2.partial && o2.linear && o2.view.offset == 0 &&
@@ -2737,7 +2850,9 @@ View Lowerer::emit_cluster(int root, int v) {
 )";
   for (size_t k = 0; k < ins.size(); ++k)
     src << "    const void* " << (may_alias(ins[k].view) ? "" : "__restrict__ ") << "p_in" << k << ",\n";
-  src << "    void* " << (inplace.empty() ? "__restrict__ " : "") << "p_out, long long n) {\n";
+  for (size_t k = 0; k < roots.size(); ++k)
+    src << "    void* " << (inplace.empty() ? "__restrict__ " : "") << "p_out" << k << ",\n";
+  src << "    long long n) {\n";
   src << "  for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * " << V << "; i < n; i += (long long)gridDim.x * "
       << 256 * V << ") {\n";
   if (V > 1 && total % V != 0) src << "    const bool whole = i + " << V << " <= n;\n";
@@ -2788,18 +2903,35 @@ View Lowerer::emit_cluster(int root, int v) {
     }
     src << "    }\n";
   }
-  src << "    struct __attribute__((packed)) O { " << stype(os.dtype) << " x[" << V
-      << "]; } r;\n#pragma unroll\n    for (int e = 0; e < " << V << "; ++e) {\n"
-      << body.str() << "      r.x[e] = " << store_expr(os.dtype, expr[v]) << ";\n    }\n    " << stype(os.dtype) << "* dst = ("
-      << stype(os.dtype) << "*)p_out + i;\n";
-  if (V > 1 && total % V != 0)
-    src << "    if (!whole) {\n#pragma unroll\n      for (int e = 0; e < " << V << "; ++e)\n        if (i + e < n) dst[e] = r.x[e];\n"
-        << "    } else\n";
-  src << "    *(O*)dst = r;\n  }\n}\n";
+  for (size_t k = 0; k < roots.size(); ++k)
+    src << "    struct __attribute__((packed)) { " << stype(N[roots[k]].shape.dtype) << " x[" << V << "]; } r" << k << ";\n";
+  src << "#pragma unroll\n    for (int e = 0; e < " << V << "; ++e) {\n" << body.str();
+  for (size_t k = 0; k < roots.size(); ++k)
+    src << "      r" << k << ".x[e] = " << store_expr(N[roots[k]].shape.dtype, expr[roots[k]]) << ";\n";
+  src << "    }\n";
+  for (size_t k = 0; k < roots.size(); ++k) {
+    const std::string T = stype(N[roots[k]].shape.dtype);
+    src << "    " << T << "* dst" << k << " = (" << T << "*)p_out" << k << " + i;\n";
+    if (V > 1 && total % V != 0)
+      src << "    if (!whole) {\n#pragma unroll\n      for (int e = 0; e < " << V << "; ++e)\n        if (i + e < n) dst" << k
+          << "[e] = r" << k << ".x[e];\n    } else\n";
+    src << "    *(decltype(r" << k << ")*)dst" << k << " = r" << k << ";\n";
+  }
+  src << "  }\n}\n";
   const std::string code = src.str();
   RtcKernel kern;
   if (rtc_get(be, code, "fused", &kern, err) != GHIP_OK) return bad();
-  View y = fresh(os);
+  std::vector<View> ys;
+  std::vector<int> wr, odts;
+  for (int r : roots) {
+    ys.push_back(fresh(N[r].shape));
+    wr.push_back(ys.back().slot);
+    odts.push_back(N[r].shape.dtype);
+    if (r != v) {
+      views[r] = ys.back();
+      have[r] = 1;
+    }
+  }
   std::vector<int> rd;
   std::vector<View> in_views;
   std::vector<int> in_dt;
@@ -2817,16 +2949,15 @@ View Lowerer::emit_cluster(int root, int v) {
   }
   d << "]";
   if (n_partial) d << " (sums the split partials of " << n_partial << " product" << (n_partial > 1 ? "s" : "") << ")";
-  const int odt = os.dtype;
-  add_step(d.str(), rd, {y.slot}, [=](ExecState& st, GHipError* e) -> int {
+  if (roots.size() > 1) d << " outputs=" << roots.size();
+  add_step(d.str(), rd, wr, [=](ExecState& st, GHipError* e) -> int {
     if (total == 0) return GHIP_OK;
-    std::vector<void*> ptrs(in_views.size());
+    std::vector<void*> ptrs(in_views.size() + ys.size());
     std::vector<void*> args;
     for (size_t k = 0; k < in_views.size(); ++k) ptrs[k] = st.ptr(in_views[k], in_dt[k]);
-    void* outp = st.ptr(y, odt);
+    for (size_t k = 0; k < ys.size(); ++k) ptrs[in_views.size() + k] = st.ptr(ys[k], odts[k]);
     long long nn = total;
     for (size_t k = 0; k < ptrs.size(); ++k) args.push_back(&ptrs[k]);
-    args.push_back(&outp);
     args.push_back(&nn);
     int64_t g = ((total + V - 1) / V + 255) / 256;
     if (g > 16384) g = 16384;
@@ -2834,7 +2965,7 @@ View Lowerer::emit_cluster(int root, int v) {
     if (h != hipSuccess) return check_hip(h, e, "generated elementwise kernel launch");
     return GHIP_OK;
   }, inplace);
-  return y;
+  return ys[0];
 }
 
 // Compile-time image of the run-time checks ghip_gemm_batched makes before it
@@ -2861,7 +2992,7 @@ bool Lowerer::emit_split_partials(int o, const Shape& os, const std::set<int>& i
   for (int r : fn->outputs)
     if (r == o) return false;
   for (int w : users[o])
-    if (!inset.count(w)) return false;
+    if (!inset.count(w) || copied[w]) return false;
   const int dt = N[n.in[0]].shape.dtype, odt = n.shape.dtype;
   if ((dt != GHIP_DTYPE_BFLOAT16 && dt != GHIP_DTYPE_FLOAT16) || N[n.in[1]].shape.dtype != dt) return false;
   if (odt != dt && odt != GHIP_DTYPE_FLOAT32) return false;
@@ -2902,32 +3033,36 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   const Shape& os = N[v].shape;
   std::set<int> inset(mem.begin(), mem.end());
   std::set<int> outs(fn->outputs.begin(), fn->outputs.end());
-  // Dot inputs, in first-use order.
+  // Dot inputs that only this cluster reads, in first-use order; any other Dot is
+  // stored by its own GEMM and enters as an operand.
+  auto fusable = [&](int d) {
+    const Node& n = N[d];
+    if (!live[d] || have[d] || outs.count(d) || fusion[d].kind != Fusion::None || n.shape.dims != os.dims) return false;
+    for (int w : users[d])
+      if (!inset.count(w) || copied[w]) return false;
+    return N[n.in[0]].shape.dtype == GHIP_DTYPE_BFLOAT16 && N[n.in[1]].shape.dtype == GHIP_DTYPE_BFLOAT16 &&
+           (n.shape.dtype == GHIP_DTYPE_BFLOAT16 || n.shape.dtype == GHIP_DTYPE_FLOAT32);
+  };
   std::vector<int> dots;
   for (int u : mem) {
     if (N[u].kind == Kind::Iota) return View{};
     for (int o : N[u].in)
-      if (o >= 0 && !inset.count(o) && N[o].kind == Kind::Dot &&
+      if (o >= 0 && !inset.count(o) && N[o].kind == Kind::Dot && fusable(o) &&
           std::find(dots.begin(), dots.end(), o) == dots.end())
         dots.push_back(o);
   }
-  if (dots.empty() || dots.size() > 2) return View{};
-  for (int d : dots) {
-    const Node& n = N[d];
-    if (!live[d] || have[d] || outs.count(d) || fusion[d].kind != Fusion::None) return View{};
-    if (n.shape.dims != os.dims) return View{};
-    for (int w : users[d])
-      if (!inset.count(w)) return View{};
-    if (N[n.in[0]].shape.dtype != GHIP_DTYPE_BFLOAT16 || N[n.in[1]].shape.dtype != GHIP_DTYPE_BFLOAT16) return View{};
-    if (n.shape.dtype != GHIP_DTYPE_BFLOAT16 && n.shape.dtype != GHIP_DTYPE_FLOAT32) return View{};
-  }
-  if (dots.size() == 2) {
+  if (dots.empty()) return View{};
+  // Two products run as one GEMM where they share the left operand; else the last one
+  // carries the epilogue (a sum of two products: the second GEMM adds the first's
+  // result in place of a kernel that reads both).
+  bool share = dots.size() == 2;
+  if (share) {
     const Node& a = N[dots[0]];
     const Node& b = N[dots[1]];
-    if (a.in[0] != b.in[0] || a.shape.dtype != b.shape.dtype || N[a.in[1]].shape.dims != N[b.in[1]].shape.dims ||
-        a.a0 != b.a0 || a.a1 != b.a1 || a.a2 != b.a2 || a.a3 != b.a3)
-      return View{};
+    share = a.in[0] == b.in[0] && a.shape.dtype == b.shape.dtype && N[a.in[1]].shape.dims == N[b.in[1]].shape.dims &&
+            a.a0 == b.a0 && a.a1 == b.a1 && a.a2 == b.a2 && a.a3 == b.a3;
   }
+  if (!share) dots.erase(dots.begin(), dots.end() - 1);
   const int NB = static_cast<int>(dots.size());
   DotPlan dp[2];
   for (int k = 0; k < NB; ++k) {
