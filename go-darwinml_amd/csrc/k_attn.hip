@@ -51,7 +51,9 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 
-enum MaskKind { kNoMask = 0, kBoolMask = 1, kAddMask = 2 };
+// kKeyMask: a boolean keep-mask that no query axis enters (key padding), up to
+// kMaxBitTiles key tiles: held as one bit per key in LDS.
+enum MaskKind { kNoMask = 0, kBoolMask = 1, kAddMask = 2, kKeyMask = 3 };
 
 struct Params {
   const void* q;
@@ -88,6 +90,7 @@ constexpr int kBKV = 64;    // keys per tile
 constexpr int kQW = 32;     // queries per wave
 constexpr int kWaves = 4;   // waves per workgroup
 constexpr int kBQ = kQW * kWaves;
+constexpr int kMaxBitTiles = 512;
 constexpr float kLazyLog2 = 8.f;  // the reference max may trail the true max by 2^8
 // A buffer offset past every descriptor's records (< 2 GiB, or capped at it in the
 // BIG kernels): a DMA lane given it loads zeros.
@@ -222,12 +225,14 @@ template <int DP, bool F16, int MK, bool SPLIT, bool BIG = false>
 // DP = 128: without the bound the compiler took 172 VGPRs for the plain schedule
 // (two a SIMD, 12% slower on the block's attention) once the decoding forms added
 // per-lane row indices; with it, 168 and no scratch.
-__global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask ? 3 : 2)) void sdpa_fwd_kernel(Params p) {
+__global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMask ? 3 : 2)) void sdpa_fwd_kernel(
+    Params p) {
   constexpr int NCH = DP / 8;  // 16-byte chunks per key row
   constexpr int NDMA = kBKV * DP * 2 / 1024 / kWaves;  // DMA instructions per wave per K (or V) tile
   constexpr int RPI = 1024 / (DP * 2);                 // key rows per DMA instruction
   // [stage][K | V][64 keys x DP]
   __shared__ __attribute__((aligned(1024))) uint16_t smem[1][2][kBKV * DP];
+  __shared__ uint64_t keep[MK == kKeyMask ? kMaxBitTiles : 1];
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((GHIP_ALDS void*)&smem[0][0][0]));
 
   const int lane = threadIdx.x & 63;
@@ -294,6 +299,40 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask ? 3 : 2)) void 
   // scale_log2 > 0, so the running max is kept on the raw scores and the scale
   // is folded into one FMA per exponent: exp2(s * c - m * c).
   const float c = p.scale_log2;
+
+  // Key mask: bit i of keep[t - t0] is set when key 64 t + i exists and is kept (one
+  // key a lane, read once per workgroup).  A tile without a kept key is neither loaded
+  // nor computed (its weights are exactly zero), one of kept keys alone needs no mask.
+  // [8,12,1000,64] f16, padded sequences of 500 to 1000 keys: 57.6 us with every lane
+  // loading its keys' mask bytes in every tile, 36.5 with the bits.
+  if constexpr (MK == kKeyMask) {
+    const uint8_t* mp = static_cast<const uint8_t*>(p.mask) + b * p.m_sb + (p.gqa_pack ? 0 : h * p.m_sh);
+    for (int tw = t0 + 4 * wave; tw < ntiles; tw += 4 * kWaves) {  // four tiles' bytes in flight
+      uint8_t kept[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = (tw + i) * kBKV + lane;
+        kept[i] = mp[static_cast<int64_t>(key < p.Sk ? key : p.Sk - 1) * p.m_sk];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint64_t bits = __builtin_amdgcn_ballot_w64((tw + i) * kBKV + lane < p.Sk && kept[i] != 0);
+        if (lane == 0 && tw + i < ntiles) keep[tw + i - t0] = bits;
+      }
+    }
+    __syncthreads();
+  }
+  auto tile_bits = [&](int t) -> uint64_t {
+    const uint64_t v = keep[t - t0];
+    return static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)))) |
+           static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32)))) << 32;
+  };
+  // First tile at or after t with a key to see (the same for every wave).
+  auto next = [&](int t) {
+    if constexpr (MK == kKeyMask)
+      while (t < ntiles && tile_bits(t) == 0) ++t;
+    return t;
+  };
 
   // Per-lane byte offsets of this wave's NDMA K and NDMA V DMA instructions within
   // a tile (instruction i fills key rows RPI (NDMA wave + i) .. +RPI, NCH lanes a
@@ -381,8 +420,9 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask ? 3 : 2)) void 
     const int key0 = t * kBKV;
     // The mask terms of this tile, fetched before the MFMAs so their latency
     // overlaps them.
+    constexpr bool kLaneMask = MK == kBoolMask || MK == kAddMask;
     float mk[2][16];
-    if constexpr (MK != kNoMask) {
+    if constexpr (kLaneMask) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -401,16 +441,28 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask ? 3 : 2)) void 
       s1 = mma<F16>(frag_k<DP>(sk, 1, s, lane), qf[s], s1);
     }
     // s{kb}[v] is key key0 + 32 kb + 4 h2 + kv, kv = (v/4)*8 + v%4, for query qi.
-    if constexpr (MK != kNoMask) {
+    if constexpr (kLaneMask) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         s0[v] += mk[0][v];
         s1[v] += mk[1][v];
       }
     }
-    // Only the diagonal tile(s) and a ragged last tile need the element mask:
-    // visible iff kv (+32 for s1) < lim.
-    if ((p.causal && key0 + kBKV - 1 > qw) || key0 + kBKV > p.Sk) {
+    if constexpr (MK == kKeyMask) {
+      const uint64_t bits = tile_bits(t);
+      if (bits != ~0ull) {
+        const uint32_t w0 = static_cast<uint32_t>(bits) >> (4 * h2), w1 = static_cast<uint32_t>(bits >> 32) >> (4 * h2);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int kv = (v >> 2) * 8 + (v & 3);
+          s0[v] = (w0 >> kv) & 1u ? s0[v] : -INFINITY;
+          s1[v] = (w1 >> kv) & 1u ? s1[v] : -INFINITY;
+        }
+      }
+    }
+    // Only the diagonal tile(s) and a ragged last tile (whose keys past Sk a key mask
+    // drops already) need the element mask: visible iff kv (+32 for s1) < lim.
+    if ((p.causal && key0 + kBKV - 1 > qw) || (MK != kKeyMask && key0 + kBKV > p.Sk)) {
       const int lim = min(p.Sk, p.causal ? qi + 1 : p.Sk) - key0 - 4 * h2;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
@@ -499,9 +551,13 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask ? 3 : 2)) void 
       // refilled.
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
-    for (int t = t0; t < ntiles; t += 2) {
-      tile(t);
-      if (t + 1 < ntiles) tile(t + 1);
+    if constexpr (MK == kKeyMask) {
+      for (int t = next(t0); t < ntiles; t = next(t + 1)) tile(t);
+    } else {
+      for (int t = t0; t < ntiles; t += 2) {
+        tile(t);
+        if (t + 1 < ntiles) tile(t + 1);
+      }
     }
   } else {
     // K and V load separately, each under the other half of the tile: V_t during
@@ -511,23 +567,25 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask ? 3 : 2)) void 
     constexpr int kWaitOneTile = NDMA | (7 << 4) | (15 << 8);  // vmcnt(NDMA), other counters not waited
     static_assert(NDMA < 16, "vmcnt immediate");
     // (A split with no keys for this query block issues nothing.)
-    if (t0 < ntiles) {
-      issue_k(t0);
-      issue_v(t0);
+    const int first = next(t0);
+    if (first < ntiles) {
+      issue_k(first);
+      issue_v(first);
     }
-    for (int t = t0; t < ntiles; ++t) {
-      if (t == t0) __builtin_amdgcn_s_waitcnt(kWaitOneTile);  // K_t0 landed (V_t0 may be in flight)
+    for (int t = first, tn; t < ntiles; t = tn) {
+      tn = next(t + 1);
+      if (t == first) __builtin_amdgcn_s_waitcnt(kWaitOneTile);  // its K landed (V may be in flight)
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // K_t landed
       __syncthreads();  // K_t visible; every wave done with P V of tile t-1
-      if (t > t0) issue_v(t);
+      if (t > first) issue_v(t);
       bf16x8_t pb[4];
       const bool sk = skip(t);
       if (!sk) scores(t, pb);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();  // every wave done reading K_t
-      if (t + 1 < ntiles) {
-        issue_k(t + 1);
-        __builtin_amdgcn_s_waitcnt(kWaitOneTile);  // V_t landed, K_{t+1} in flight
+      if (tn < ntiles) {
+        issue_k(tn);
+        __builtin_amdgcn_s_waitcnt(kWaitOneTile);  // V_t landed, the next tile's K in flight
       } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
@@ -583,16 +641,18 @@ template <int DP, bool F16, bool SPLIT, bool BIG>
 static void launch_dm(const Params& p, int mk, dim3 grid, hipStream_t s) {
   static_assert(!SPLIT, "masked kernels use the plain schedule");
   if (mk == kBoolMask) hipLaunchKernelGGL((sdpa_fwd_kernel<DP, F16, kBoolMask, SPLIT, BIG>), grid, dim3(256), 0, s, p);
+  else if (mk == kKeyMask) hipLaunchKernelGGL((sdpa_fwd_kernel<DP, F16, kKeyMask, SPLIT, BIG>), grid, dim3(256), 0, s, p);
   else if (mk == kAddMask) hipLaunchKernelGGL((sdpa_fwd_kernel<DP, F16, kAddMask, SPLIT, BIG>), grid, dim3(256), 0, s, p);
   else hipLaunchKernelGGL((sdpa_fwd_kernel<DP, F16, kNoMask, SPLIT, BIG>), grid, dim3(256), 0, s, p);
 }
-// The split schedule only without a mask: with one, the compiler's waits for the
+// The split schedule only without a mask or with a key mask (LDS bits): with another, the compiler's waits for the
 // mask loads also wait for the K / V DMA (vmcnt counts both in issue order), and
 // the masked variants would spill at the extra barrier.
 // BIG: K / V slices of 2 GiB or more (KvOff).
 template <int DP, bool F16, bool BIG>
 static void launch_db(const Params& p, int mk, dim3 grid, bool split, hipStream_t s) {
   if (split && mk == kNoMask) hipLaunchKernelGGL((sdpa_fwd_kernel<DP, F16, kNoMask, true, BIG>), grid, dim3(256), 0, s, p);
+  else if (split && mk == kKeyMask) hipLaunchKernelGGL((sdpa_fwd_kernel<DP, F16, kKeyMask, true, BIG>), grid, dim3(256), 0, s, p);
   else launch_dm<DP, F16, false, BIG>(p, mk, grid, s);
 }
 template <int DP, bool F16>
@@ -1031,6 +1091,10 @@ extern "C" int ghip_sdpa_fwd_masked_ws(int dtype, const void* q, const void* k, 
     // Vector loads of 4-key groups (keys are multiples of 4 apart): unit key stride
     // and every row start aligned to 4 elements.
     const int64_t mes = mask_dtype == GHIP_DTYPE_BOOL ? 1 : es;
+    // A mask over the keys alone (a packed group's heads must share it): bits.
+    if (mk == attn::kBoolMask && !f32 && (p.m_sq == 0 || Sq == 1) && Sk <= attn::kMaxBitTiles * attn::kBKV &&
+        (!sg.pack || p.m_sh == 0))
+      mk = attn::kKeyMask;
     p.mask_vec = p.m_sk == 1 && p.m_sb % 4 == 0 && p.m_sh % 4 == 0 && p.m_sq % 4 == 0 && al(mask, 4 * mes);
   }
   // A split key range when a workspace is given and the grid is small.
