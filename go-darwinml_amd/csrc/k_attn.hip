@@ -232,7 +232,6 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
   constexpr int RPI = 1024 / (DP * 2);                 // key rows per DMA instruction
   // [stage][K | V][64 keys x DP]
   __shared__ __attribute__((aligned(1024))) uint16_t smem[1][2][kBKV * DP];
-  __shared__ uint64_t keep[MK == kKeyMask ? kMaxBitTiles : 1];
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((GHIP_ALDS void*)&smem[0][0][0]));
 
   const int lane = threadIdx.x & 63;
@@ -305,7 +304,10 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
   // nor computed (its weights are exactly zero), one of kept keys alone needs no mask.
   // [8,12,1000,64] f16, padded sequences of 500 to 1000 keys: 57.6 us with every lane
   // loading its keys' mask bytes in every tile, 36.5 with the bits.
+  uint64_t* keep = nullptr;
   if constexpr (MK == kKeyMask) {
+    __shared__ uint64_t bits_lds[kMaxBitTiles];
+    keep = bits_lds;
     const uint8_t* mp = static_cast<const uint8_t*>(p.mask) + b * p.m_sb + (p.gqa_pack ? 0 : h * p.m_sh);
     for (int tw = t0 + 4 * wave; tw < ntiles; tw += 4 * kWaves) {  // four tiles' bytes in flight
       uint8_t kept[4];
@@ -572,8 +574,7 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
       issue_k(first);
       issue_v(first);
     }
-    for (int t = first, tn; t < ntiles; t = tn) {
-      tn = next(t + 1);
+    for (int t = first; t < ntiles; t = next(t + 1)) {
       if (t == first) __builtin_amdgcn_s_waitcnt(kWaitOneTile);  // its K landed (V may be in flight)
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // K_t landed
       __syncthreads();  // K_t visible; every wave done with P V of tile t-1
@@ -583,6 +584,7 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
       if (!sk) scores(t, pb);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();  // every wave done reading K_t
+      const int tn = next(t + 1);
       if (tn < ntiles) {
         issue_k(tn);
         __builtin_amdgcn_s_waitcnt(kWaitOneTile);  // V_t landed, the next tile's K in flight
