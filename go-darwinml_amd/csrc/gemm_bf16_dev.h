@@ -162,25 +162,34 @@ inline GemmSplit gemm_k_split(int64_t batch, int64_t M, int64_t N, int64_t K, in
 inline bool gemm_small_tiles(int64_t batch, int64_t M, int64_t N, int es) {
   return batch * ((M + 127) / 128) * ((N + 127) / 128) <= (es == 4 ? 192 : 128);
 }
-// Whether a product that gemm_k_split would split runs as its split: not where the
-// 64 x 64 tiles, unsplit, are modelled at less than 0.8 of the split's cost.  Their
-// cost: one round of 256 tiles ~2.4 us + 4.6 ns a contraction step (fp32 3 + 20.9),
-// two rounds ~4 + 8.3 (4 + 37); measured, us, split / 64 x 64 tiles: bf16 [256,4096,2048]
-// 20.9 / 12.2, [1024,1024,2048] 21.1 / 12.3, [256,4096,4096] 23.4 / 21.4, and the split
-// kept at [128,4096,4096] 17.6 / 20.4, [512,512,4096] 15.6 / 20.0, [1024,2048,4096]
-// 31.8 / 32.8; fp32 [256,4096,1024] 35.5 / 25.4.  At most 64 rows (decoding, weights
+// fp32 grids of at most 128 tiles of 64 x 64: 32 x 32 tiles with the contraction spread
+// over a workgroup's waves.  us, 64 x 64 / 32 x 32: [256,512,256] 8.1 / 4.9, [256,256,512]
+// 13.0 / 6.5, [512,1024,1024] (128 tiles) 23.7 / 16.7, but 24.7 / 27.0 at 256.
+inline bool gemm_f32_tiny(int64_t batch, int64_t M, int64_t N) {
+  return batch * ((M + 63) / 64) * ((N + 63) / 64) <= 128;
+}
+// Whether a product that gemm_k_split would split runs as its split: not where small
+// tiles, unsplit, are modelled at less than 0.8 of the split's cost.  Their cost: one
+// round of 256 tiles ~2.4 us + 4.6 ns a contraction step, two rounds ~4 + 8.3 (fp32
+// 32 x 32: 2 + 7.6 and 3 + 13.3; 64 x 64: 3 + 20.9 and 4 + 37); measured, us, split /
+// small tiles: bf16 [256,4096,2048] 20.9 / 12.2, [1024,1024,2048] 21.1 / 12.3,
+// [256,4096,4096] 23.4 / 21.4, and the split kept at [128,4096,4096] 17.6 / 20.4,
+// [512,512,4096] 15.6 / 20.0, [1024,2048,4096] 31.8 / 32.8; fp32 [256,4096,1024] 35.5 /
+// 25.4, [128,4096,1024] 25.9 / 16.6.  16-bit with at most 64 rows (decoding, weights
 // from HBM): always the split, whose ranges keep more loads in flight.
 inline bool gemm_uses_split(int64_t batch, int64_t M, int64_t N, int64_t K, int es) {
   const GemmSplit sp = gemm_k_split(batch, M, N, K, es);
   if (sp.s <= 1) return false;
-  if (M <= 64 || !gemm_small_tiles(batch, M, N, es)) return true;
-  const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
+  if ((es == 2 && M <= 64) || !gemm_small_tiles(batch, M, N, es)) return true;
+  const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64), t32 = ((M + 31) / 32) * ((N + 31) / 32);
   const double k = static_cast<double>(K);
-  const double c64 = es == 4 ? (t64 <= 256 ? 3.0 + 0.0209 * k : 4.0 + 0.037 * k)
-                             : (t64 <= 256 ? 2.4 + 0.0046 * k : 4.0 + 0.0083 * k);
+  double small_us;
+  if (es == 4 && gemm_f32_tiny(batch, M, N)) small_us = t32 <= 256 ? 2.0 + 0.0076 * k : 3.0 + 0.0133 * k;
+  else if (es == 4) small_us = t64 <= 256 ? 3.0 + 0.0209 * k : 4.0 + 0.037 * k;
+  else small_us = t64 <= 256 ? 2.4 + 0.0046 * k : 4.0 + 0.0083 * k;
   const double step_us = es == 4 ? 0.065 : 0.0146;
   const double split_us = 4.0 + static_cast<double>(sp.kc) * step_us + static_cast<double>(sp.s) * M * N * 8 / 3e6;
-  return c64 >= 0.8 * split_us;
+  return small_us >= 0.8 * split_us;
 }
 // Workspace bytes of a split (0 for s = 1): s fp32 partial products [M, N].
 inline int64_t gemm_split_bytes(const GemmSplit& sp, int64_t M, int64_t N) {

@@ -259,6 +259,24 @@ __device__ __forceinline__ void f32_tile_mma(const float* As, const float* Bs, i
   }
 }
 
+// Columns n .. n + 3 (those below N) of an output row.
+template <typename OutT>
+__device__ __forceinline__ void f32_store4(const GemmParams& p, OutT* dst, int64_t n, const float (&v)[4]) {
+  if (p.vec_c && n + 3 < p.N) {
+    if constexpr (sizeof(OutT) == 2)
+      *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    else
+      *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+  } else if (sizeof(OutT) == 4 && n + 3 < p.N) {  // one store at element alignment
+    *reinterpret_cast<u32x4_a4_t*>(dst) = u32x4_t{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
+                                                   __float_as_uint(v[3])};
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < p.N) store_out<OutT>(dst + e, v[e]);
+  }
+}
+
 // Output of an fp32 core.
 template <int BM, int BN, int WM, int WN, typename OutT, int FM, int FN>
 __device__ __forceinline__ void f32_tile_store(const GemmParams& p, int64_t bb, int64_t m0, int64_t n0, int wm, int wn,
@@ -280,20 +298,7 @@ __device__ __forceinline__ void f32_tile_store(const GemmParams& p, int64_t bb, 
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = acc[i][j][q * 4 + e];
-        OutT* dst = C + m * p.sc_m + n;
-        if (p.vec_c && n + 3 < p.N) {
-          if constexpr (sizeof(OutT) == 2)
-            *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-          else
-            *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-        } else if (sizeof(OutT) == 4 && n + 3 < p.N) {  // one store at element alignment
-          *reinterpret_cast<u32x4_a4_t*>(dst) = u32x4_t{__float_as_uint(v[0]), __float_as_uint(v[1]),
-                                                         __float_as_uint(v[2]), __float_as_uint(v[3])};
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < p.N) store_out<OutT>(dst + e, v[e]);
-        }
+        f32_store4<OutT>(p, C + m * p.sc_m + n, n, v);
       }
   }
 }
@@ -415,6 +420,67 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_rs_kernel(GemmParams p) {
   f32_tile_store<BM, BN, WM, WN, OutT>(p, bb, m0, n0, wm, wn, lane, acc);
 }
 
+// Few-tile fp32 products: one 32 x 32 tile per workgroup, whose four waves take every
+// fourth 8-step group of the contraction and add their sums in wave order at the end.  A
+// lone 64 x 64 tile is bound by its waves' serial MFMAs (1024 cycles per 32 steps, one
+// CU's rate for a grid of a few); here a step is a quarter of that on four times the
+// CUs.  Same operands, alignment and edges as the other register-staged cores; another
+// summation order.
+template <bool A_K, bool B_K, typename OutT>
+__global__ __launch_bounds__(256, 2) void gemm_f32_ks_kernel(GemmParams p) {
+  constexpr int T = 32, PD = 8;
+  using TA = RsTile<4, T, A_K>;
+  using TB = RsTile<4, T, B_K>;
+  __shared__ __attribute__((aligned(1024))) float smem[4 * T * kBK32];
+  float* sa = smem;
+  float* sb = smem + 2 * T * kBK32;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int64_t bb;
+  int tm, tn;
+  map_tile(blockIdx.x, p.batch * p.tiles_m * p.tiles_n, p.tiles_m, p.tiles_n, bb, tm, tn);
+  const int64_t m0 = static_cast<int64_t>(tm) * T, n0 = static_cast<int64_t>(tn) * T;
+  const uint32_t* A = static_cast<const uint32_t*>(p.a) + bb * p.sa_b + m0 * p.sa_m;
+  const uint32_t* B = static_cast<const uint32_t*>(p.b) + bb * p.sb_b + n0 * p.sb_n;
+  TA ta;
+  TB tb;
+  ta.init(threadIdx.x, p.M - m0, p.sa_m, p.sa_k);
+  tb.init(threadIdx.x, p.N - n0, p.sb_n, p.sb_k);
+  f32x16_t acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+  auto compute = [&](int st) {
+    const float* As = sa + st * T * kBK32;
+    const float* Bs = sb + st * T * kBK32;
+    float4 a4, b4;
+    if constexpr (A_K) a4 = frag_f32_kc(As, 0, wave, lane);
+    if constexpr (B_K) b4 = frag_f32_kc(Bs, 0, wave, lane);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float af = A_K ? f4_at(a4, e) : frag_f32_mn<T>(As, 0, wave, e, lane);
+      const float bf = B_K ? f4_at(b4, e) : frag_f32_mn<T>(Bs, 0, wave, e, lane);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(bf, af, acc, 0, 0, 0);
+    }
+  };
+  rs_main_loop<PD>(ta, tb, A, B, p.K, static_cast<int>((p.K + kBK32 - 1) / kBK32), p.k_fast,
+                   reinterpret_cast<uint32_t*>(sa), reinterpret_cast<uint32_t*>(sb), T * kBK32, T * kBK32, compute);
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < 16; ++v) smem[(wave * 16 + v) * 64 + lane] = acc[v];
+  __syncthreads();
+  // Wave w finishes accumulator values 4 w .. 4 w + 3: columns 8 w + 4 (lane / 32) + e.
+  const int64_t m = m0 + (lane & 31), n = n0 + wave * 8 + (lane >> 5) * 4;
+  if (m >= p.M || n >= p.N) return;
+  float r[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    r[e] = smem[(wave * 4 + e) * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) r[e] += smem[(w * 16 + wave * 4 + e) * 64 + lane];
+  }
+  f32_store4<OutT>(p, static_cast<OutT*>(p.c) + bb * p.sc_b + m * p.sc_m + n, n, r);
+}
+
 // The 256 x 256 cores (grids of >= 128 tiles).  BIG: the 64-bit-records
 // instantiations (operand slices of 2 GiB or more), instantiated in k_gemm_big.hip.
 template <bool BIG, typename InT, typename OutT>
@@ -451,7 +517,13 @@ hipError_t launch_rs_tile(GemmParams p, hipStream_t s) {
   p.tiles_m = static_cast<int>((p.M + T - 1) / T);
   p.tiles_n = static_cast<int>((p.N + T - 1) / T);
   const dim3 grid(static_cast<unsigned>(p.batch * p.tiles_m * p.tiles_n)), block(256);
-  if constexpr (ES == 4) {
+  if constexpr (T == 32) {
+    static_assert(ES == 4, "32 x 32 tiles: fp32");
+    if (a_k && b_k) hipLaunchKernelGGL((gemm_f32_ks_kernel<true, true, OutT>), grid, block, 0, s, p);
+    else if (a_k) hipLaunchKernelGGL((gemm_f32_ks_kernel<true, false, OutT>), grid, block, 0, s, p);
+    else if (b_k) hipLaunchKernelGGL((gemm_f32_ks_kernel<false, true, OutT>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((gemm_f32_ks_kernel<false, false, OutT>), grid, block, 0, s, p);
+  } else if constexpr (ES == 4) {
     if (a_k && b_k) hipLaunchKernelGGL((gemm_f32_rs_kernel<T, T, true, true, OutT>), grid, block, 0, s, p);
     else if (a_k) hipLaunchKernelGGL((gemm_f32_rs_kernel<T, T, true, false, OutT>), grid, block, 0, s, p);
     else if (b_k) hipLaunchKernelGGL((gemm_f32_rs_kernel<T, T, false, true, OutT>), grid, block, 0, s, p);
@@ -464,6 +536,8 @@ hipError_t launch_rs_tile(GemmParams p, hipStream_t s) {
   }
   return hipGetLastError();
 }
+extern template hipError_t launch_rs_tile<32, float, float>(GemmParams, hipStream_t);
+extern template hipError_t launch_rs_tile<32, float, bf16_t>(GemmParams, hipStream_t);
 extern template hipError_t launch_rs_tile<64, bf16_t, bf16_t>(GemmParams, hipStream_t);
 extern template hipError_t launch_rs_tile<64, bf16_t, float>(GemmParams, hipStream_t);
 extern template hipError_t launch_rs_tile<64, f16_t, f16_t>(GemmParams, hipStream_t);

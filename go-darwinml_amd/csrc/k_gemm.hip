@@ -159,6 +159,8 @@ static int64_t slice_bytes(int64_t rows, int64_t s_row, int64_t K, int64_t s_k, 
 
 template <typename InT, typename OutT>
 static hipError_t launch_rs(const GemmParams& p, hipStream_t s) {
+  if constexpr (sizeof(InT) == 4)
+    if (gemm_f32_tiny(p.batch, p.M, p.N)) return launch_rs_tile<32, InT, OutT>(p, s);
   return gemm_small_tiles(p.batch, p.M, p.N, sizeof(InT)) ? launch_rs_tile<64, InT, OutT>(p, s)
                                                           : launch_rs_tile<128, InT, OutT>(p, s);
 }
@@ -342,7 +344,7 @@ static hipError_t dispatch_f32(GemmParams p, hipStream_t s, GemmWs ws = {}) {
     const GemmSplit sp = gemm_k_split(p.batch, p.M, p.N, p.K, 4);
     if (gemm_split_bytes(sp, p.M, p.N) <= ws.bytes) return launch_split<float, OutT>(p, ma, mb, sp, ws.ptr, s);
   }
-  if (p.K > 0 && gemm_small_tiles(p.batch, p.M, p.N, 4)) return launch_rs_tile<64, float, OutT>(p, s);
+  if (p.K > 0 && gemm_small_tiles(p.batch, p.M, p.N, 4)) return launch_rs<float, OutT>(p, s);
   // The 8-wave 256 x 256 fp32 core only from one full round of its tiles: below
   // that the 4-wave 128 x 128 core (two workgroups per CU) is faster, 1.9x at 128
   // tiles of 256 x 256 ([2048,4096,4096]), 1.3x at 144 and 192, even at 256.

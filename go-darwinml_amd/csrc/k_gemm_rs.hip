@@ -3,6 +3,8 @@
 #include "gemm_kernels.h"
 
 namespace ghip {
+template hipError_t launch_rs_tile<32, float, float>(GemmParams, hipStream_t);
+template hipError_t launch_rs_tile<32, float, bf16_t>(GemmParams, hipStream_t);
 template hipError_t launch_rs_tile<64, bf16_t, bf16_t>(GemmParams, hipStream_t);
 template hipError_t launch_rs_tile<64, bf16_t, float>(GemmParams, hipStream_t);
 template hipError_t launch_rs_tile<64, f16_t, f16_t>(GemmParams, hipStream_t);

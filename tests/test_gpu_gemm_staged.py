@@ -51,6 +51,21 @@ def test_odd_operands(cuda, shape, a_t, b_t, dt, odt, off):
     assert rel_err(c[:, rows], ref) <= tol
 
 
+# fp32 grids around the 32 x 32 (contraction over the waves), 64 x 64 and 128 x 128 tiles.
+@pytest.mark.parametrize("shape", [(1, 31, 33, 7), (1, 33, 31, 9), (1, 32, 32, 32), (2, 64, 96, 264), (1, 512, 1024, 40),
+                                   (1, 513, 1025, 41), (1, 1536, 2048, 36), (1, 1537, 2049, 33)])
+@pytest.mark.parametrize("a_t,b_t", [(False, False), (False, True), (True, False), (True, True)])
+def test_f32_tile_sizes(cuda, shape, a_t, b_t):
+    B, M, N, K = shape
+    a = _operand((B, M), K, 0, a_t, F32, 7401, cuda)
+    b = _operand((B, K), N, 0, b_t, F32, 7402, cuda)
+    rows = np.unique(np.clip(np.array([0, 1, 31, 32, 33, 63, 64, 100, 511, 512, M - 2, M - 1]), 0, M - 1))
+    c = ops.gemm(a, b).cpu().numpy()[:, rows]
+    ref = orc.dot_general(np.ascontiguousarray(a.cpu().numpy()[:, rows]), [2], [0], np.ascontiguousarray(b.cpu().numpy()),
+                          [1], [0])
+    assert rel_err(c, ref) <= 1e-5
+
+
 def test_values_past_the_edges_do_not_leak(cuda):
     """Neighbouring rows / columns of NaN around every odd operand stay out."""
     for dt in (BF16, F32):
