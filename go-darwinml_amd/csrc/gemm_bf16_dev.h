@@ -162,6 +162,21 @@ inline GemmSplit gemm_k_split(int64_t batch, int64_t M, int64_t N, int64_t K, in
 inline bool gemm_small_tiles(int64_t batch, int64_t M, int64_t N, int es) {
   return batch * ((M + 127) / 128) * ((N + 127) / 128) <= (es == 4 ? 192 : 128);
 }
+// 16-bit products for 256 x 128 tiles (gemm_bf16_body4h): grids that are one round of
+// them but more than one 128 x 128 tile per CU, with a contraction long enough to pay for
+// a prologue and an epilogue that no second workgroup hides.  Graph-replayed, us, 128 x
+// 128 core / 256 x 128: [4096,2048,8192] 127 / 108, [2304,2304,4096] 55.3 / 48.0,
+// [2048,3072,4096] 55 / 49, [4096,2048,2048] 35.0 / 33.0, but [2,2048,2048,1024] 20.4 /
+// 20.7; at 256 tiles of 128 x 128 [2048,2048,2048] 27.5 / 28.5; where 256 x 256 tiles are
+// more than 128 their cores win ([4096,4096,4096] 97 / 112).  Ragged tiles pay for the
+// masks of their loads, more so on an MN-contiguous A: [3080,2056,4096] 60.2 / 56.2, A
+// MN-contiguous 65.0 / 64.0 ([2056,2184,4096] 58.6 / 60.6), [3080,2056,2048] 33.5 / 34.6.
+inline bool gemm_half_whole(int64_t M, int64_t N, int64_t K) { return M % 256 == 0 && N % 128 == 0 && K % 64 == 0; }
+inline bool gemm_half_tiles(int64_t batch, int64_t M, int64_t N, int64_t K, bool a_k) {
+  const int64_t t128 = batch * ((M + 127) / 128) * ((N + 127) / 128);
+  const int64_t half = batch * ((M + 255) / 256) * ((N + 127) / 128);
+  return M >= 256 && t128 > 256 && half <= 256 && (gemm_half_whole(M, N, K) ? K >= 2048 : a_k && K >= 4096);
+}
 // fp32 grids of at most 128 tiles of 64 x 64: 32 x 32 tiles with the contraction spread
 // over a workgroup's waves.  us, 64 x 64 / 32 x 32: [256,512,256] 8.1 / 4.9, [256,256,512]
 // 13.0 / 6.5, [512,1024,1024] (128 tiles) 23.7 / 16.7, but 24.7 / 27.0 at 256.
@@ -379,8 +394,10 @@ struct OperandTile {
   // Byte offsets of this lane's chunk.  The swizzle depends on the parity of the
   // instruction only: even / odd i; instruction i adds (i & ~1) * step, step being
   // kRPI operand rows (in the KC16 layout instruction i + 2 holds the operand rows
-  // 8 further on, so kRPI / 2).
-  static constexpr int kNV = 2;
+  // 8 further on, so kRPI / 2).  A wave whose share of an MN-contiguous swz_n2 tile is
+  // more than the 8 k-rows of one swizzle keeps an offset per instruction.
+  static constexpr bool kEach = !KC && L16 && kPerWave * kRPI > 8;
+  static constexpr int kNV = kEach ? kPerWave : 2;
   uint32_t voff[kNV];
   uint32_t step;
   int mn_valid;
@@ -422,6 +439,7 @@ struct OperandTile {
   }
   __device__ __forceinline__ uint32_t off(int i) const {
     if constexpr (IL) return voff[0] + static_cast<uint32_t>(i) * step;
+    else if constexpr (kEach) return voff[i];
     else return voff[i & 1] + static_cast<uint32_t>(i & ~1) * step;
   }
   // Instruction i of this wave's share (see issue()).
@@ -1621,6 +1639,195 @@ __device__ __forceinline__ void gemm_bf16_body4km(const GemmParams& p, const Epi
   mfma_drain_a(acc);
 
   tile_epilogue<BM, BN, WM, WN, NP>(p, epi, smem, acc, bb, m0, n0, mn_full, lane, wm, wn);
+}
+
+// 4-wave core for grids that 256 x 256 tiles leave half empty: one 256 x 128 tile per
+// workgroup of 2 x 2 waves, each 128 x 64 (32 16x16x32 MFMAs per k32 step, 128
+// accumulators a lane in AGPRs, one wave per SIMD), 64-deep k-tiles in three LDS
+// stages (144 KiB).  What bounds it is the LDS: a CU's MFMAs of a k32 step take 512
+// cycles and its fragments (12 KiB a wave) 384, the DMA's writes another 192 (at 128
+// bytes a cycle), where the 128 x 128 core's 64 x 64 waves need 8 KiB per 16 MFMAs and
+// twice the DMA per output.
+//
+// Issue order as in gemm_bf16_body4km: A fragments roll (fa[i] is refilled for the next
+// k32 step right after row block i's last MFMA), B fragments are double-buffered.
+// Step 0 of tile kt reads step 1 of the same stage.  In step 1, after two row blocks,
+// this wave's reads of stage kt % 3 have completed: wait for tile kt+1 (issued two
+// tiles earlier), barrier, refill the stage with tile kt+3 (12 DMA instructions over
+// the remaining 24 MFMAs) and read step 0 of tile kt+1.  Bit-identical to the other
+// cores (same MFMA, same k order per accumulator).
+template <bool A_K, bool B_K, class Epi, bool F16 = false>
+__device__ __forceinline__ void gemm_bf16_body4h(const GemmParams& p, const Epi& epi) {
+  constexpr int BM = 256, BN = 128, WM = 2, WN = 2, BK = kBK;
+  constexpr int NW = WM * WN, NS = 3;
+  constexpr int TM = BM / WM, TN = BN / WN;
+  constexpr int FM = TM / 16, FN = TN / 16;  // 8 x 4 blocks of 16 x 16
+  using TA = OperandTile<BM, A_K, NW, BK, true, A_K>;
+  using TB = OperandTile<BN, B_K, NW, BK, true, B_K>;
+  constexpr int NA = TA::kPerWave, LPW = NA + TB::kPerWave;  // loads per wave per tile (8 + 4)
+  constexpr int kSA = BM * BK * 2, kSB = BN * BK * 2;        // bytes per stage
+  static_assert(FM == 8 && FN == 4 && LPW == 12, "read and DMA slots of one step");
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[NS * (kSA + kSB) / 2];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+
+  int64_t bb;
+  int tm, tn;
+  map_tile(blockIdx.x, p.batch * p.tiles_m * p.tiles_n, p.tiles_m, p.tiles_n, bb, tm, tn);
+  const int64_t m0 = static_cast<int64_t>(tm) * BM, n0 = static_cast<int64_t>(tn) * BN;
+  const uint16_t* A0 = static_cast<const uint16_t*>(p.a) + bb * p.sa_b + m0 * p.sa_m;
+  const uint16_t* B0 = static_cast<const uint16_t*>(p.b) + bb * p.sb_b + n0 * p.sb_n;
+  const auto a_left0 = ExtSel<false>::a(p, m0 * p.sa_m * 2);
+  const auto b_left0 = ExtSel<false>::b(p, n0 * p.sb_n * 2);
+
+  TA ta;
+  TB tb;
+  ta.init(wave, lane, p.sa_m, p.sa_k, p.M - m0);
+  tb.init(wave, lane, p.sb_n, p.sb_k, p.N - n0);
+  const bool mn_full = m0 + BM <= p.M && n0 + BN <= p.N;
+  const int KT = static_cast<int>((p.K + BK - 1) / BK);
+  const uint32_t lds_b = static_cast<uint32_t>(reinterpret_cast<uint64_t>((GHIP_LDS void*)smem));
+  const uint32_t lds_a = lds_b + NS * kSB;
+
+  f32x4_t acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.f;
+
+  // Per-lane LDS base pointers, as in gemm_bf16_body8x.
+  typedef GHIP_LDS const uint16_t* lds_p;
+  lds_p const ldsB = (lds_p)((GHIP_LDS void*)smem);
+  lds_p const ldsA = ldsB + NS * kSB / 2;
+  constexpr int NBA = A_K ? 4 : FM;
+  lds_p abase[NBA], bbase[4];
+#pragma unroll
+  for (int q = 0; q < NBA; ++q) {
+    if constexpr (A_K) {
+      const int rho = wm * TM + 2 * (lane & 15) + ((lane >> 4) & 1);
+      abase[q] = ldsA + rho * BK + (((4 * (q >> 1) + 2 * (q & 1) + (lane >> 5)) ^ swz_k(rho)) * 8);
+    } else {
+      const int kl = 8 * (lane >> 4) + ((lane & 15) >> 2);
+      const int nl = wm * TM + q * 16 + 4 * (lane & 3);
+      abase[q] = ldsA + kl * BM + (((nl >> 3) ^ swz_n2(kl)) * 8) + (nl & 7);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if constexpr (B_K) {
+      const int rho = wn * TN + 2 * (lane & 15) + ((lane >> 4) & 1);
+      bbase[q] = ldsB + rho * BK + (((4 * (q >> 1) + 2 * (q & 1) + (lane >> 5)) ^ swz_k(rho)) * 8);
+    } else {
+      const int kl = 8 * (lane >> 4) + ((lane & 15) >> 2);
+      const int nl = wn * TN + q * 16 + 4 * (lane & 3);
+      bbase[q] = ldsB + kl * BN + (((nl >> 3) ^ swz_n2(kl)) * 8) + (nl & 7);
+    }
+  }
+  bf16x8_t fa[FM], fb[2][FN];
+  auto rd_tr = [](lds_p p0, int R) {
+    const bf16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((GHIP_LDS bf16x4_t*)(p0));
+    const bf16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((GHIP_LDS bf16x4_t*)(p0 + 4 * R));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  // row block i of A / column block j of B at k32 step s (0, 1) of stage st
+  auto read_a = [&](int i, int st, int s) {
+    if constexpr (A_K) fa[i] = *(GHIP_LDS const bf16x8_t*)(abase[2 * (i & 1) + s] + st * (kSA / 2) + (i >> 1) * 32 * BK);
+    else fa[i] = rd_tr(abase[i] + st * (kSA / 2) + s * 32 * BM, BM);
+  };
+  auto read_b = [&](int j, int st, int s) {
+    if constexpr (B_K) fb[s][j] = *(GHIP_LDS const bf16x8_t*)(bbase[2 * (j & 1) + s] + st * (kSB / 2) + (j >> 1) * 32 * BK);
+    else fb[s][j] = rd_tr(bbase[j] + st * (kSB / 2) + s * 32 * BN, BN);
+  };
+
+  auto run = [&](auto full_c) {
+    constexpr bool FULL = decltype(full_c)::value;
+    auto dma = [&](int t, int st, int d) {  // instruction d of k-tile t into stage st
+      const int64_t k0 = static_cast<int64_t>(t) * BK;
+      const int k_left = static_cast<int>(p.K - k0 < BK ? p.K - k0 : BK);
+      if (d < NA)
+        ta.template issue_one<FULL>(make_rsrc(A0 + k0 * p.sa_k, a_left0.at(k0 * p.sa_k * 2)), lds_a + st * kSA, wave, lane,
+                                    k_left, d);
+      else
+        tb.template issue_one<FULL>(make_rsrc(B0 + k0 * p.sb_k, b_left0.at(k0 * p.sb_k * 2)), lds_b + st * kSB, wave, lane,
+                                    k_left, d - NA);
+    };
+#pragma unroll
+    for (int t = 0; t < NS; ++t)
+      if (t < KT) {
+#pragma unroll
+        for (int d = 0; d < LPW; ++d) dma(t, t, d);
+      }
+    if (KT >= NS) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPW) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < FN; ++j) read_b(j, 0, 0);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) read_a(i, 0, 0);
+
+    // Tile kt in stage ST = kt % 3.  STEADY: tile kt+3 exists.
+    auto tile = [&](int kt, auto st_c, auto steady_c) {
+      constexpr int ST = decltype(st_c)::value, SN = (ST + 1) % NS;
+      constexpr bool STEADY = decltype(steady_c)::value;
+      const bool nx = STEADY || kt + 1 < KT, refill = STEADY || kt + NS < KT;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          mma16x32a<F16>(acc[i][j], fb[0][j], fa[i]);
+          if (j == 1 && i < FN) read_b(i, ST, 1);
+          sched_fence();
+        }
+        read_a(i, ST, 1);
+        sched_fence();
+      }
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          mma16x32a<F16>(acc[i][j], fb[1][j], fa[i]);
+          if (i >= 2) {
+            const int q = (i - 2) * FN + j;  // 0 .. 23
+            if (q % 2 == 0 && refill) dma(kt + NS, ST, q / 2);
+            if (j == 1 && i - 2 < FN && nx) read_b(i - 2, SN, 0);
+          }
+          sched_fence();
+        }
+        if (i == 1 && nx) {
+          if constexpr (STEADY) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory");
+          else asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(0)" ::: "memory");
+          __syncthreads();
+          read_a(0, SN, 0);
+          read_a(1, SN, 0);
+          sched_fence();
+        }
+        if (i >= 2 && nx) {
+          read_a(i, SN, 0);
+          sched_fence();
+        }
+      }
+    };
+    int kt = 0;
+    for (; kt + 2 + NS < KT; kt += NS) {
+      tile(kt, IntC<0>{}, BoolC<true>{});
+      tile(kt + 1, IntC<1>{}, BoolC<true>{});
+      tile(kt + 2, IntC<2>{}, BoolC<true>{});
+    }
+    for (; kt < KT; kt += NS) {
+      tile(kt, IntC<0>{}, BoolC<false>{});
+      if (kt + 1 < KT) tile(kt + 1, IntC<1>{}, BoolC<false>{});
+      if (kt + 2 < KT) tile(kt + 2, IntC<2>{}, BoolC<false>{});
+    }
+  };
+  if (mn_full && (p.K % BK) == 0) run(BoolC<true>{});
+  else run(BoolC<false>{});
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  mfma_drain_a(acc);
+  tile_epilogue<BM, BN, WM, WN, 1>(p, epi, smem, acc, bb, m0, n0, mn_full, lane, wm, wn);
 }
 
 // 8-wave 16x16x32 core for any operand layout (the A K-contiguous / B MN-contiguous

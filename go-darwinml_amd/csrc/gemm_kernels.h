@@ -147,6 +147,13 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_kernel8x(GemmParams p) {
   gemm_bf16_body8x<A_K, B_K, StoreEpi<OutT>, __is_same(InT, f16_t), 1, BIG>(p, epi);
 }
 
+// The 256 x 128 16x16x32 core (grids that 256 x 256 tiles leave half empty).
+template <bool A_K, bool B_K, typename InT, typename OutT>
+__global__ __launch_bounds__(256, 1) void gemm_bf16_kernel4h(GemmParams p) {
+  const StoreEpi<OutT> epi = store_epi<OutT>(p);
+  gemm_bf16_body4h<A_K, B_K, StoreEpi<OutT>, __is_same(InT, f16_t)>(p, epi);
+}
+
 // ---------------------------------------------------------------------------
 // fp32 MFMA path: v_mfma_f32_32x32x2f32, 32-deep k-tiles by buffer_load ... lds
 // (two stages), operands swapped like the bf16 path so a lane stores 4 adjacent
@@ -507,6 +514,19 @@ hipError_t launch_f32(GemmParams p, bool a_k, bool b_k, hipStream_t s) {
   return hipGetLastError();
 }
 
+// The 256 x 128 core (instantiated in k_gemm_half.hip).
+template <typename InT, typename OutT>
+hipError_t launch_bf16_half(GemmParams p, bool a_k, bool b_k, hipStream_t s) {
+  p.tiles_m = static_cast<int>((p.M + 255) / 256);
+  p.tiles_n = static_cast<int>((p.N + 127) / 128);
+  const dim3 grid(static_cast<unsigned>(p.batch * p.tiles_m * p.tiles_n));
+  if (a_k && b_k) hipLaunchKernelGGL((gemm_bf16_kernel4h<true, true, InT, OutT>), grid, dim3(256), 0, s, p);
+  else if (a_k) hipLaunchKernelGGL((gemm_bf16_kernel4h<true, false, InT, OutT>), grid, dim3(256), 0, s, p);
+  else if (b_k) hipLaunchKernelGGL((gemm_bf16_kernel4h<false, true, InT, OutT>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((gemm_bf16_kernel4h<false, false, InT, OutT>), grid, dim3(256), 0, s, p);
+  return hipGetLastError();
+}
+
 // T x T tiles of a register-staged core (instantiated in k_gemm_rs.hip).
 template <int T, typename InT, typename OutT>
 hipError_t launch_rs_tile(GemmParams p, hipStream_t s) {
@@ -550,6 +570,10 @@ extern template hipError_t launch_rs_tile<128, f16_t, f16_t>(GemmParams, hipStre
 extern template hipError_t launch_rs_tile<128, f16_t, float>(GemmParams, hipStream_t);
 extern template hipError_t launch_rs_tile<128, float, float>(GemmParams, hipStream_t);
 extern template hipError_t launch_rs_tile<128, float, bf16_t>(GemmParams, hipStream_t);
+extern template hipError_t launch_bf16_half<bf16_t, bf16_t>(GemmParams, bool, bool, hipStream_t);
+extern template hipError_t launch_bf16_half<bf16_t, float>(GemmParams, bool, bool, hipStream_t);
+extern template hipError_t launch_bf16_half<f16_t, f16_t>(GemmParams, bool, bool, hipStream_t);
+extern template hipError_t launch_bf16_half<f16_t, float>(GemmParams, bool, bool, hipStream_t);
 extern template hipError_t launch_bf16_4w<true, bf16_t, bf16_t>(GemmParams, bool, bool, hipStream_t);
 extern template hipError_t launch_bf16_4w<true, bf16_t, float>(GemmParams, bool, bool, hipStream_t);
 extern template hipError_t launch_bf16_4w<true, f16_t, f16_t>(GemmParams, bool, bool, hipStream_t);

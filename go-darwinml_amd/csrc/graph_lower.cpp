@@ -3188,8 +3188,10 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   //
   // One product on a grid of at most 128 256 x 256 tiles: the 128 x 128 core (two
   // workgroups per CU), as the precompiled GEMMs do (a 256 x 256 grid that small
-  // leaves half the CUs or more idle).
-  bool eight_km = false, eight_x = false, four_km = false;
+  // leaves half the CUs or more idle), or the 256 x 128 core where its rule and whole
+  // tiles allow (128 x 128 / 256 x 128, us: tanh-GELU [4096,2048,8192] 174 / 151,
+  // [4096,2048,2048] 72 / 70; ragged tiles lose, [2056,2184,4096] 87 / 107).
+  bool eight_km = false, eight_x = false, four_km = false, half = false;
   const int64_t t4 = d.B * ((d.M + 255) / 256) * ((d.N + 256 / NB - 1) / (256 / NB));
   if (rs) {
     if (gemm_small_tiles(d.B, d.M, d.N, 2)) BM = BN = 64;
@@ -3200,6 +3202,7 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
     else if (d.M >= 256 && d.N >= 256 && t256 > 128 && (mb || heavy_epilogue))
       BM = 256, BN = 256, WM = 2, WN = 4, eight_x = true;
     else if (d.M >= 256 && d.N >= 256 && t256 > 128) BM = 256, BN = 256, WM = 2, WN = 2, four_wave = true;
+    else if (!big && gemm_half_whole(d.M, d.N, d.K) && gemm_half_tiles(d.B, d.M, d.N, d.K, ma)) BM = 256, BN = 128, half = true;
   } else if (d.M >= 256 && d.N >= 128) {
     BM = 256, BN = 128, WM = 2, WN = 4;
     eight_km = ma && !mb && d.B * ((d.M + 255) / 256) * ((d.N + 127) / 128) >= 128;
@@ -3270,6 +3273,8 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   else if (eight_x)
     src << "  ghip::gemm_bf16_body8x<" << (ma ? "true" : "false") << ", " << (mb ? "true" : "false")
         << ", ghip::GenEpi, false, " << NB << big_arg << ">(p, epi);\n}\n";
+  else if (half)
+    src << "  ghip::gemm_bf16_body4h<" << (ma ? "true" : "false") << ", " << (mb ? "true" : "false") << ", ghip::GenEpi>(p, epi);\n}\n";
   else if (four_wave)
     src << "  ghip::gemm_bf16_body4mn<ghip::GenEpi, false" << big_arg << ">(p, epi);\n}\n";
   else
@@ -3304,7 +3309,7 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   for (auto& in : ins) rd.push_back(in.view.slot);
   std::ostringstream desc;
   // core: waves and k-depth of the main loop (km32: A in 64-deep, B in 32-deep stages)
-  const char* core = four_km ? "4w-km32" : eight_km ? "8w-km32" : eight_x ? "8w-k64" : four_wave ? "4w-mn32" : rs ? "staged" : "small";
+  const char* core = four_km ? "4w-km32" : eight_km ? "8w-km32" : eight_x ? "8w-k64" : four_wave ? "4w-mn32" : half ? "4w-k64" : rs ? "staged" : "small";
   desc << fmt("gemm_batched+epilogue bf16 B=%lld M=%lld N=%lld K=%lld dots=%d tile=%dx%d waves=%d core=%s (%s) ops=%zu "
               "inputs=%zu [",
               (long long)d.B, (long long)d.M, (long long)d.N, (long long)d.K, NB, BM, BN * NB, WM * WN, core,

@@ -259,12 +259,13 @@ static hipError_t dispatch_bf16(GemmParams p, hipStream_t s, GemmWs ws = {}) {
   }
   if (p.K > 0 && gemm_small_tiles(p.batch, p.M, p.N, 2)) return launch_rs_tile<64, InT, OutT>(p, s);
   // Grids of more than 128 256 x 256 tiles: the 256 x 256 cores (one workgroup per
-  // CU).  Up to 128 such tiles they would leave half the 256 CUs or more idle, and
-  // the 128 x 128 core (two workgroups per CU, so up to 512 tiles in one round) is
-  // faster in every layout: 11-33% at 128 tiles ([2048,4096,4096], [8192,1024,2048]),
-  // 12-43% against the 256 x 128 core below that (A/B, one box).  All cores give
-  // the same bits.
+  // CU).  Up to 128 such tiles they would leave half the 256 CUs or more idle, and the
+  // 128 x 128 core (two workgroups per CU, so up to 512 tiles in one round) is faster in
+  // every layout: 11-33% at 128 tiles ([2048,4096,4096], [8192,1024,2048]; A/B, one box);
+  // with a long contraction the 256 x 128 core (gemm_half_tiles).  All cores give the
+  // same bits.
   if (p.M >= 256 && p.N >= 256 && t256 > 128) return launch_bf16_4w<false, InT, OutT>(p, ma, mb, s);
+  if (gemm_half_tiles(p.batch, p.M, p.N, p.K, ma == 1)) return launch_bf16_half<InT, OutT>(p, ma == 1, mb == 1, s);
   return launch_bf16<128, 128, 2, 2, InT, OutT>(p, ma, mb, s);
 }
 
