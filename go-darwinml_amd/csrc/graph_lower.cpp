@@ -3040,8 +3040,9 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
     if (!live[d] || have[d] || outs.count(d) || fusion[d].kind != Fusion::None || n.shape.dims != os.dims) return false;
     for (int w : users[d])
       if (!inset.count(w) || copied[w]) return false;
-    return N[n.in[0]].shape.dtype == GHIP_DTYPE_BFLOAT16 && N[n.in[1]].shape.dtype == GHIP_DTYPE_BFLOAT16 &&
-           (n.shape.dtype == GHIP_DTYPE_BFLOAT16 || n.shape.dtype == GHIP_DTYPE_FLOAT32);
+    const int dt = N[n.in[0]].shape.dtype;
+    return (dt == GHIP_DTYPE_BFLOAT16 || dt == GHIP_DTYPE_FLOAT16) && N[n.in[1]].shape.dtype == dt &&
+           (n.shape.dtype == dt || n.shape.dtype == GHIP_DTYPE_FLOAT32);
   };
   std::vector<int> dots;
   for (int u : mem) {
@@ -3074,7 +3075,7 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   // unfused (the split's fp32 partials are summed by a kernel of their own, which
   // the generated epilogue kernel does not reproduce).
   if (gemm_uses_split(d.B, d.M, d.N, d.K, 2)) return View{};
-  // The bf16 MFMA path's operand conditions, decided here because the fused
+  // The 16-bit MFMA path's operand conditions, decided here because the fused
   // kernel has no generic fallback.
   if (d.B > 65535 || d.M == 0 || d.N == 0 || d.K == 0) return View{};
   if (d.sab < 0 || d.sam < 0 || d.sak < 0 || d.sbb < 0 || d.sbk < 0 || d.sbn < 0) return View{};
@@ -3097,6 +3098,33 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   const bool big = !rs && (ea >= (int64_t{1} << 31) || eb >= (int64_t{1} << 31));
   const char* big_arg = big ? ", true" : "";
 
+  // A VALU-heavy epilogue (transcendentals, long chains) runs faster on an 8-wave
+  // core: with one wave per SIMD a wave issues a VALU instruction every few cycles,
+  // with two the SIMD's VALU stays busy (FusedDense + tanh-GELU: 894 -> 953 TFLOP/s
+  // against the 4-wave core), while the 4-wave MN-contiguous core's main loop is a
+  // few percent faster for light epilogues.
+  int valu_weight = 0;
+  for (int u : mem) {
+    const Node& n = N[u];
+    valu_weight += 1;
+    if (n.kind == Kind::Unary &&
+        (n.sub == GHIP_UNARY_EXP || n.sub == GHIP_UNARY_EXPM1 || n.sub == GHIP_UNARY_LOG ||
+         n.sub == GHIP_UNARY_LOG1P || n.sub == GHIP_UNARY_SIN || n.sub == GHIP_UNARY_COS ||
+         n.sub == GHIP_UNARY_TANH || n.sub == GHIP_UNARY_LOGISTIC || n.sub == GHIP_UNARY_ERF ||
+         n.sub == GHIP_UNARY_SQRT || n.sub == GHIP_UNARY_RSQRT))
+      valu_weight += 6;
+  }
+  const bool heavy_epilogue = valu_weight >= 8;
+  // fp16: such an epilogue on a round of 256 x 256 tiles that is less than 3/4 full costs
+  // more than the elementwise kernel it saves (tanh-GELU, us, unfused / fused:
+  // [2304,4096,4096] 90 / 92, [4096,5120,2048] 117 / 123; full rounds [4096,4096,1024] 52 /
+  // 49, [8192,8192,2048] 301 / 286).
+  const int ab_dt = N[N[dots[0]].in[0]].shape.dtype;
+  const int64_t t256 = d.B * ((d.M + 255) / 256) * ((d.N + 255) / 256);
+  if (ab_dt == GHIP_DTYPE_FLOAT16 && NB == 1 && heavy_epilogue && !rs && d.M >= 256 && d.N >= 256 && t256 > 128 &&
+      4 * t256 < 3 * ((t256 + 255) / 256 * 256))
+    return View{};
+
   // Extra operands: each must fold to one stride per (batch, m, n) group of the
   // output dims [batch (nbatch), lhs free (nlfree), rhs free].
   std::vector<int64_t> gb, gm, gn;
@@ -3111,13 +3139,12 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   };
   std::vector<In> ins;
   std::map<int, std::string> expr;
-  // The GEMM stages each product in the Dot's own dtype (bf16 bits, or fp32), so
+  // The GEMM stages each product in the Dot's own dtype (bf16 bits, fp16 or fp32), so
   // the value read back is exactly what the stand-alone Dot would have stored.
   const int dot_dt = N[dots[0]].shape.dtype;
-  const bool stage_bf16 = dot_dt == GHIP_DTYPE_BFLOAT16;
-  const int CH = stage_bf16 ? 8 : 4;  // outputs per epilogue call (16 staged bytes)
-  for (int k = 0; k < NB; ++k) expr[dots[k]] = stage_bf16 ? (k == 0 ? "bf2f(acc0[e])" : "bf2f(acc1[e])")
-                                                           : (k == 0 ? "acc0[e]" : "acc1[e]");
+  const char* f16 = ab_dt == GHIP_DTYPE_FLOAT16 ? "true" : "false";
+  const int CH = 16 / dtype_size(dot_dt);  // outputs per epilogue call (16 staged bytes)
+  for (int k = 0; k < NB; ++k) expr[dots[k]] = load_expr(dot_dt, k == 0 ? "acc0[e]" : "acc1[e]");
   std::ostringstream body;
   for (size_t ui = 0; ui < mem.size(); ++ui) {
     const int u = mem[ui];
@@ -3158,24 +3185,6 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   // 256 x (2 x 128) tile does the MMA work of one 256 x 256 tile.
   int BM = 128, BN = 128, WM = 2, WN = 2;
   bool four_wave = false;
-  const int64_t t256 = d.B * ((d.M + 255) / 256) * ((d.N + 255) / 256);
-  // A VALU-heavy epilogue (transcendentals, long chains) runs faster on an 8-wave
-  // core: with one wave per SIMD a wave issues a VALU instruction every few cycles,
-  // with two the SIMD's VALU stays busy (FusedDense + tanh-GELU: 894 -> 953 TFLOP/s
-  // against the 4-wave core), while the 4-wave MN-contiguous core's main loop is a
-  // few percent faster for light epilogues.
-  int valu_weight = 0;
-  for (int u : mem) {
-    const Node& n = N[u];
-    valu_weight += 1;
-    if (n.kind == Kind::Unary &&
-        (n.sub == GHIP_UNARY_EXP || n.sub == GHIP_UNARY_EXPM1 || n.sub == GHIP_UNARY_LOG ||
-         n.sub == GHIP_UNARY_LOG1P || n.sub == GHIP_UNARY_SIN || n.sub == GHIP_UNARY_COS ||
-         n.sub == GHIP_UNARY_TANH || n.sub == GHIP_UNARY_LOGISTIC || n.sub == GHIP_UNARY_ERF ||
-         n.sub == GHIP_UNARY_SQRT || n.sub == GHIP_UNARY_RSQRT))
-      valu_weight += 6;
-  }
-  const bool heavy_epilogue = valu_weight >= 8;
   // Otherwise A K-contiguous, B MN-contiguous: the 8-wave 32-deep core.  Other
   // layouts: the 8-wave 64-deep 16x16x32 core, except both operands MN-contiguous
   // with a light epilogue (4-wave 32-deep core).
@@ -3184,7 +3193,9 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   // products: the 4-wave core (128 x 128 waves, one per SIMD, a third fewer LDS
   // reads per MFMA; on the block's residual and SwiGLU epilogues 2.5% faster than
   // the 8-wave core under sustained load).  A VALU-heavy epilogue of one product
-  // (FusedDense + tanh-GELU) stays on the 8-wave core (4% faster there).
+  // (FusedDense + tanh-GELU) stays on the 8-wave core with bf16 operands (4% faster
+  // there), but with fp16 operands takes the 4-wave core (tanh-GELU, us, 8 / 4 waves:
+  // [4096,4096,4096] 132 / 124, [8192,8192,2048] 299 / 286).
   //
   // One product on a grid of at most 128 256 x 256 tiles: the 128 x 128 core (two
   // workgroups per CU), as the precompiled GEMMs do (a 256 x 256 grid that small
@@ -3195,7 +3206,8 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   const int64_t t4 = d.B * ((d.M + 255) / 256) * ((d.N + 256 / NB - 1) / (256 / NB));
   if (rs) {
     if (gemm_small_tiles(d.B, d.M, d.N, 2)) BM = BN = 64;
-  } else if (ma && !mb && d.M >= 256 && d.N >= 256 / NB && (NB == 2 || !heavy_epilogue) && (NB == 2 ? t4 >= 128 : t4 > 128)) {
+  } else if (ma && !mb && d.M >= 256 && d.N >= 256 / NB && (NB == 2 || !heavy_epilogue || ab_dt == GHIP_DTYPE_FLOAT16) &&
+             (NB == 2 ? t4 >= 128 : t4 > 128)) {
     BM = 256, BN = 256 / NB, WM = 2, WN = 2, four_km = true;
   } else if (NB == 1) {
     if (d.M >= 256 && d.N >= 256 && t256 > 128 && ma && !mb) BM = 256, BN = 256, WM = 2, WN = 4, eight_km = true;
@@ -3217,8 +3229,8 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   // tile lies inside the output, so no column bounds checks.
   const bool vec = d.N % CH == 0;
   const std::string CHs = std::to_string(CH);
-  src << "namespace ghip {\nstruct GenEpi {\n  using Stage = " << (stage_bf16 ? "unsigned short" : "float") << ";\n"
-      << "  __device__ __forceinline__ static Stage stage(float v) { return " << (stage_bf16 ? "f2bf(v)" : "v")
+  src << "namespace ghip {\nstruct GenEpi {\n  using Stage = " << stype(dot_dt) << ";\n"
+      << "  __device__ __forceinline__ static Stage stage(float v) { return " << store_expr(dot_dt, "v")
       << "; }\n  struct Pre {";
   for (size_t k = 0; k < ins.size(); ++k) src << " " << stype(ins[k].dt) << " x" << k << "[" << CH << "];";
   src << " };\n  EpiArgs a;\n"
@@ -3265,21 +3277,21 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
       << "  const ghip::GenEpi epi{a};\n";
   if (rs)
     src << "  ghip::gemm_bf16_body_rs<" << BM << ", " << BN << ", " << (ma ? "true" : "false") << ", "
-        << (mb ? "true" : "false") << ", ghip::GenEpi>(p, epi);\n}\n";
+        << (mb ? "true" : "false") << ", ghip::GenEpi, " << f16 << ">(p, epi);\n}\n";
   else if (four_km)
-    src << "  ghip::gemm_bf16_body4km<ghip::GenEpi, false, " << NB << big_arg << ">(p, epi);\n}\n";
+    src << "  ghip::gemm_bf16_body4km<ghip::GenEpi, " << f16 << ", " << NB << big_arg << ">(p, epi);\n}\n";
   else if (eight_km)
-    src << "  ghip::gemm_bf16_body8km<ghip::GenEpi, false, " << NB << big_arg << ">(p, epi);\n}\n";
+    src << "  ghip::gemm_bf16_body8km<ghip::GenEpi, " << f16 << ", " << NB << big_arg << ">(p, epi);\n}\n";
   else if (eight_x)
     src << "  ghip::gemm_bf16_body8x<" << (ma ? "true" : "false") << ", " << (mb ? "true" : "false")
-        << ", ghip::GenEpi, false, " << NB << big_arg << ">(p, epi);\n}\n";
+        << ", ghip::GenEpi, " << f16 << ", " << NB << big_arg << ">(p, epi);\n}\n";
   else if (half)
-    src << "  ghip::gemm_bf16_body4h<" << (ma ? "true" : "false") << ", " << (mb ? "true" : "false") << ", ghip::GenEpi>(p, epi);\n}\n";
+    src << "  ghip::gemm_bf16_body4h<" << (ma ? "true" : "false") << ", " << (mb ? "true" : "false") << ", ghip::GenEpi, " << f16 << ">(p, epi);\n}\n";
   else if (four_wave)
-    src << "  ghip::gemm_bf16_body4mn<ghip::GenEpi, false" << big_arg << ">(p, epi);\n}\n";
+    src << "  ghip::gemm_bf16_body4mn<ghip::GenEpi, " << f16 << big_arg << ">(p, epi);\n}\n";
   else
     src << "  ghip::gemm_bf16_body<" << BM << ", " << BN << ", " << WM << ", " << WN << ", " << (ma ? "true" : "false") << ", "
-        << (mb ? "true" : "false") << ", " << NB << ", ghip::GenEpi, false" << big_arg << ">(p, epi);\n}\n";
+        << (mb ? "true" : "false") << ", " << NB << ", ghip::GenEpi, " << f16 << big_arg << ">(p, epi);\n}\n";
   RtcKernel kern;
   if (rtc_get(be, src.str(), "gemm_epilogue", &kern, err) != GHIP_OK) {
     failed = true;
@@ -3310,9 +3322,9 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   std::ostringstream desc;
   // core: waves and k-depth of the main loop (km32: A in 64-deep, B in 32-deep stages)
   const char* core = four_km ? "4w-km32" : eight_km ? "8w-km32" : eight_x ? "8w-k64" : four_wave ? "4w-mn32" : half ? "4w-k64" : rs ? "staged" : "small";
-  desc << fmt("gemm_batched+epilogue bf16 B=%lld M=%lld N=%lld K=%lld dots=%d tile=%dx%d waves=%d core=%s (%s) ops=%zu "
+  desc << fmt("gemm_batched+epilogue %s B=%lld M=%lld N=%lld K=%lld dots=%d tile=%dx%d waves=%d core=%s (%s) ops=%zu "
               "inputs=%zu [",
-              (long long)d.B, (long long)d.M, (long long)d.N, (long long)d.K, NB, BM, BN * NB, WM * WN, core,
+              ab_dt == GHIP_DTYPE_FLOAT16 ? "f16" : "bf16", (long long)d.B, (long long)d.M, (long long)d.N, (long long)d.K, NB, BM, BN * NB, WM * WN, core,
               d.how.c_str(), mem.size(), ins.size());
   for (size_t i = 0; i < mem.size(); ++i) {
     const Node& n = N[mem[i]];
@@ -3322,9 +3334,9 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   desc << "]";
   add_step(desc.str(), rd, {y.slot}, [=](ExecState& st, GHipError* e) -> int {
     GemmParams p = gp;
-    p.a = st.ptr(lv, GHIP_DTYPE_BFLOAT16);
-    p.b = st.ptr(rv0, GHIP_DTYPE_BFLOAT16);
-    p.b1 = st.ptr(rv1, GHIP_DTYPE_BFLOAT16);
+    p.a = st.ptr(lv, ab_dt);
+    p.b = st.ptr(rv0, ab_dt);
+    p.b1 = st.ptr(rv1, ab_dt);
     p.c = st.ptr(y, odt);
     if (!rs && (reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b) | reinterpret_cast<uintptr_t>(p.b1)) & 15u)
       return set_error(e, GHIP_ERR_STATE, "fused GEMM epilogue: operand base not 16-byte aligned");
