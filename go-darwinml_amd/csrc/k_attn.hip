@@ -299,13 +299,14 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
   // is folded into one FMA per exponent: exp2(s * c - m * c).
   const float c = p.scale_log2;
 
-  // Key mask: bit i of keep[t - t0] is set when key 64 t + i exists and is kept (one
-  // key a lane, read once per workgroup).  A tile without a kept key is neither loaded
-  // nor computed (its weights are exactly zero), one of kept keys alone needs no mask.
-  // As beyond the causal bound, V of a tile left out is not read: NaN or infinities
-  // there do not reach the output.
-  // [8,12,1000,64] f16, padded sequences of 500 to 1000 keys: 57.6 us with every lane
-  // loading its keys' mask bytes in every tile, 36.5 with the bits.
+  // Key mask: bit i of keep[t - t0] is set when key 64 t + i is kept or past Sk (one key
+  // a lane, read once per workgroup); a tile of kept keys alone needs no mask.  Every
+  // tile is computed, with the per-lane mask's term (0 or -inf) added to each score: what
+  // K and V hold at dropped keys (NaN, infinities) reaches the output as it does through
+  // a mask that has a query axis.  f16 [8,12,1000,64], padded sequences of 500 to 1000
+  // keys, us a call: 57.4 with every lane loading its keys' mask bytes in every tile,
+  // 41.8 with the bits (37.2 with the tiles without a kept key left out, which loses
+  // those effects).
   uint64_t* keep = nullptr;
   if constexpr (MK == kKeyMask) {
     __shared__ uint64_t bits_lds[kMaxBitTiles];
@@ -320,7 +321,7 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const uint64_t bits = __builtin_amdgcn_ballot_w64((tw + i) * kBKV + lane < p.Sk && kept[i] != 0);
+        const uint64_t bits = __builtin_amdgcn_ballot_w64((tw + i) * kBKV + lane >= p.Sk || kept[i] != 0);
         if (lane == 0 && tw + i < ntiles) keep[tw + i - t0] = bits;
       }
     }
@@ -330,12 +331,6 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
     const uint64_t v = keep[t - t0];
     return static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)))) |
            static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32)))) << 32;
-  };
-  // First tile at or after t with a key to see (the same for every wave).
-  auto next = [&](int t) {
-    if constexpr (MK == kKeyMask)
-      while (t < ntiles && tile_bits(t) == 0) ++t;
-    return t;
   };
 
   // Per-lane byte offsets of this wave's NDMA K and NDMA V DMA instructions within
@@ -455,18 +450,20 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
     if constexpr (MK == kKeyMask) {
       const uint64_t bits = tile_bits(t);
       if (bits != ~0ull) {
-        const uint32_t w0 = static_cast<uint32_t>(bits) >> (4 * h2), w1 = static_cast<uint32_t>(bits >> 32) >> (4 * h2);
+        // Dropped keys' bits, sign-extended over the bits of -inf.
+        const int d0 = static_cast<int>(~static_cast<uint32_t>(bits) >> (4 * h2));
+        const int d1 = static_cast<int>(~static_cast<uint32_t>(bits >> 32) >> (4 * h2));
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int kv = (v >> 2) * 8 + (v & 3);
-          s0[v] = (w0 >> kv) & 1u ? s0[v] : -INFINITY;
-          s1[v] = (w1 >> kv) & 1u ? s1[v] : -INFINITY;
+          s0[v] += __int_as_float(__builtin_amdgcn_sbfe(d0, kv, 1) & static_cast<int>(0xff800000u));
+          s1[v] += __int_as_float(__builtin_amdgcn_sbfe(d1, kv, 1) & static_cast<int>(0xff800000u));
         }
       }
     }
-    // Only the diagonal tile(s) and a ragged last tile (whose keys past Sk a key mask
-    // drops already) need the element mask: visible iff kv (+32 for s1) < lim.
-    if ((p.causal && key0 + kBKV - 1 > qw) || (MK != kKeyMask && key0 + kBKV > p.Sk)) {
+    // Only the diagonal tile(s) and a ragged last tile need the element mask:
+    // visible iff kv (+32 for s1) < lim.
+    if ((p.causal && key0 + kBKV - 1 > qw) || key0 + kBKV > p.Sk) {
       const int lim = min(p.Sk, p.causal ? qi + 1 : p.Sk) - key0 - 4 * h2;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
@@ -555,13 +552,9 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
       // refilled.
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
-    if constexpr (MK == kKeyMask) {
-      for (int t = next(t0); t < ntiles; t = next(t + 1)) tile(t);
-    } else {
-      for (int t = t0; t < ntiles; t += 2) {
-        tile(t);
-        if (t + 1 < ntiles) tile(t + 1);
-      }
+    for (int t = t0; t < ntiles; t += 2) {
+      tile(t);
+      if (t + 1 < ntiles) tile(t + 1);
     }
   } else {
     // K and V load separately, each under the other half of the tile: V_t during
@@ -571,25 +564,23 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
     constexpr int kWaitOneTile = NDMA | (7 << 4) | (15 << 8);  // vmcnt(NDMA), other counters not waited
     static_assert(NDMA < 16, "vmcnt immediate");
     // (A split with no keys for this query block issues nothing.)
-    const int first = next(t0);
-    if (first < ntiles) {
-      issue_k(first);
-      issue_v(first);
+    if (t0 < ntiles) {
+      issue_k(t0);
+      issue_v(t0);
     }
-    for (int t = first; t < ntiles; t = next(t + 1)) {
-      if (t == first) __builtin_amdgcn_s_waitcnt(kWaitOneTile);  // its K landed (V may be in flight)
+    for (int t = t0; t < ntiles; ++t) {
+      if (t == t0) __builtin_amdgcn_s_waitcnt(kWaitOneTile);  // K_t0 landed (V_t0 may be in flight)
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // K_t landed
       __syncthreads();  // K_t visible; every wave done with P V of tile t-1
-      if (t > first) issue_v(t);
+      if (t > t0) issue_v(t);
       bf16x8_t pb[4];
       const bool sk = skip(t);
       if (!sk) scores(t, pb);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();  // every wave done reading K_t
-      const int tn = next(t + 1);
-      if (tn < ntiles) {
-        issue_k(tn);
-        __builtin_amdgcn_s_waitcnt(kWaitOneTile);  // V_t landed, the next tile's K in flight
+      if (t + 1 < ntiles) {
+        issue_k(t + 1);
+        __builtin_amdgcn_s_waitcnt(kWaitOneTile);  // V_t landed, K_{t+1} in flight
       } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }

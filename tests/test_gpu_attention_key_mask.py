@@ -71,3 +71,24 @@ def test_no_kept_key_is_nan(cuda, Sq):
     keep[1] = False
     got = ops.sdpa_masked(q, k, v, keep, 0.125, False)
     assert torch.isnan(got[1]).all() and not torch.isnan(got[0]).any()
+
+
+@pytest.mark.parametrize("D,dt,causal", [(64, F16, False), (128, BF16, True), (256, F16, False), (64, BF16, True)])
+@pytest.mark.parametrize("where", ["k", "v"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("key", [70, 130, 199])
+def test_non_finite_at_a_dropped_key(cuda, D, dt, causal, where, value, key):
+    """A NaN or infinity at a dropped key has one effect, whatever else its 64-key tile
+    keeps (70: a tile of kept and dropped keys, 130 and 199: tiles without a kept key):
+    the per-lane mask's, which adds -inf to the key's score and multiplies its V by 0."""
+    B, H, Sq, Sk = 2, 2, 200, 200
+    q, k, v = _qkv(B, H, H, Sq, Sk, D, dt, cuda)
+    (k if where == "k" else v)[0, 1, key, 3] = value
+    keep = (torch.arange(Sk, device=cuda) < 66).view(1, 1, 1, Sk).expand(B, 1, 1, Sk).contiguous()
+    print(D, dt, causal, where, value, key, flush=True)
+    got = ops.sdpa_masked(q, k, v, keep, D ** -0.5, causal)
+    full = ops.sdpa_masked(q, k, v, keep.expand(B, 1, Sq, Sk).contiguous(), D ** -0.5, causal)
+    assert torch.equal(torch.isnan(got), torch.isnan(full)) and torch.equal(got.nan_to_num(), full.nan_to_num())
+    assert not torch.isnan(got[1]).any() and not torch.isnan(got[0, 0]).any()
+    if where == "v" and not causal:
+        assert torch.isnan(got[0, 1, :, 3]).all()
