@@ -2708,7 +2708,22 @@ View Lowerer::emit_cluster(int root, int v) {
         }
       return ext;
     };
-    std::set<int> mine = externals(mem);
+    const std::set<int> mine = externals(mem);
+    // The operands are emitted before the joiners are chosen: one that itself needs a
+    // candidate stores it, and only what is not stored by then joins.  (A product whose
+    // split partials this kernel may sum is emitted with the kernel; its operands here.)
+    if (os.size() >= 65536)
+      for (int u : mem)
+        for (int o : N[u].in) {
+          if (!mine.count(o)) continue;
+          if (N[o].kind == Kind::Dot && fusion[o].kind == Fusion::None && !have[o]) {
+            get(N[o].in[0]);
+            get(N[o].in[1]);
+          } else {
+            get(o);
+          }
+          if (failed) return bad();
+        }
     auto at_hand = [&](int o) {
       while (!have[o] && (N[o].kind == Kind::Broadcast || N[o].kind == Kind::Reshape || N[o].kind == Kind::Transpose))
         o = N[o].in[0];

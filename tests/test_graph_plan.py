@@ -556,3 +556,45 @@ def test_decode_step_plan(be):
     assert "sums the split partials of 2 products" in plan and plan.count("sums the split partials of 1 product") == 2
     assert plan.count("sdpa_fwd") == 1 and "key range split" in plan, plan
     assert "strided_copy" not in plan and "epilogue" not in plan, plan
+
+
+def _residual_mlp(f):
+    """x + tanh(x) W, four layers: the product needs tanh(x), which shares x with the sum."""
+    x = f.Parameter("x", make_shape(F32, 4096, 512))
+    for i in range(4):
+        x = f.Add(x, f.DotGeneral(f.Tanh(x), [1], [], f.Parameter(f"w{i}", make_shape(F32, 512, 512)), [0], []))
+    return [x]
+
+
+def _softmax_of_a_sum(f):
+    x, y = (f.Parameter(n, make_shape(BF16, 1024, 2048)) for n in "xy")
+    w = f.Add(x, y)
+    return [f.Mul(f.Mul(x, f.FusedSoftmax(w, 1)), y), w]
+
+
+def _norm_of_a_sum(f):
+    x, y = (f.Parameter(n, make_shape(BF16, 1024, 2048)) for n in "xy")
+    w = f.Add(x, y)
+    h = graphs.rms_norm(f, w, f.Parameter("g", make_shape(BF16, 2048)), 1e-6)
+    return [f.Add(f.Mul(h, x), y), f.Mul(h, w), w]
+
+
+def _reduce_of_a_transpose(f):
+    x, y = (f.Parameter(n, make_shape(BF16, 512, 512)) for n in "xy")
+    e = f.Exp(x)
+    s = f.ReduceSum(f.Transpose(e, 1, 0), 1)
+    return [f.Mul(f.Add(x, f.BroadcastInDim(s, make_shape(BF16, 512, 512), [1])), y), e]
+
+
+@pytest.mark.parametrize("build,clusters,arena", [
+    (_residual_mlp, ["[Unary#10]", "[Binary#0]"] * 4, 3 * 4096 * 512 * 4),
+    (_softmax_of_a_sum, ["[Binary#0]", "[Binary#2,Binary#2]"], 1024 * 2048 * 2),
+    (_norm_of_a_sum, ["[Binary#0]", "[Binary#2,Binary#0,Binary#2] outputs=2"], 1024 * 2048 * 2),
+    (_reduce_of_a_transpose, ["[Unary#4]", "[Binary#0,Binary#2]"], 512 * 2)])
+def test_a_cluster_that_an_operand_needs_is_stored_once(be, build, clusters, arena):
+    """A cluster that one of another cluster's operands reads is stored before that
+    operand; it does not join the other cluster's kernel as a second, unread output."""
+    p = plan_of(be, build)
+    assert [l.split(" inputs=")[1].split(" ", 1)[1] for l in p.splitlines()
+            if l.startswith("fused_elementwise")] == clusters, p
+    assert f"arena {arena} bytes" in p, p
