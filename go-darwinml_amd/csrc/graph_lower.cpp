@@ -2729,6 +2729,43 @@ View Lowerer::emit_cluster(int root, int v) {
         o = N[o].in[0];
       return have[o] || mine.count(o) || N[o].kind == Kind::Param || N[o].kind == Kind::Const || N[o].kind == Kind::Capture;
     };
+    const std::set<int> outs(fn->outputs.begin(), fn->outputs.end());
+    // Whether joining here loses output w the memory of parameter o, should it be donated:
+    // o has readers still to be emitted, and all of them precede w where it is emitted
+    // for its own sake (they belong to outputs before the first that needs w).
+    auto loses_donation = [&](int w, int o) {
+      std::set<int> seen;
+      std::vector<int> work{o}, readers;
+      while (!work.empty()) {
+        const int x = work.back();
+        work.pop_back();
+        for (int r : users[x]) {
+          if (!live[r] || !seen.insert(r).second || std::find(mem.begin(), mem.end(), r) != mem.end() ||
+              std::find(members[w].begin(), members[w].end(), r) != members[w].end())
+            continue;
+          const Kind k = N[r].kind;
+          if (!needed[r] || copied[r] || k == Kind::Reshape || k == Kind::Transpose || k == Kind::Broadcast)
+            work.push_back(r);  // read where its own readers are
+          else if (!have[r] && !(cluster[r] >= 0 && have[cluster[r]]))
+            readers.push_back(r);
+        }
+      }
+      if (readers.empty()) return false;
+      std::set<int> before;
+      for (int out : fn->outputs) {
+        std::set<int> anc{out};
+        work.assign(1, out);
+        while (!work.empty()) {
+          const int x = work.back();
+          work.pop_back();
+          for (int q : N[x].in)
+            if (q >= 0 && anc.insert(q).second) work.push_back(q);
+        }
+        if (anc.count(w)) break;
+        before.insert(anc.begin(), anc.end());
+      }
+      return std::all_of(readers.begin(), readers.end(), [&](int r) { return before.count(r) > 0; });
+    };
     const int n = static_cast<int>(N.size());
     size_t inputs = mine.size();
     for (int w = 0; w < n && roots.size() < 4; ++w) {
@@ -2744,6 +2781,10 @@ View Lowerer::emit_cluster(int root, int v) {
         shares = shares || (mine.count(o) && N[o].shape.dims == os.dims && N[o].kind != Kind::Broadcast);
       }
       if (!ok || !shares || inputs + ext.size() > 12) continue;
+      if (outs.count(w) && std::any_of(ext.begin(), ext.end(), [&](int o) {
+            return N[o].kind == Kind::Param && N[o].shape == N[w].shape && loses_donation(w, o);
+          }))
+        continue;
       roots.push_back(w);
       inputs += ext.size();
       for (int u : members[w])
@@ -2844,18 +2885,20 @@ View Lowerer::emit_cluster(int root, int v) {
   int V = std::max(1, 16 / widest);
   while (V > 1 && (total / V < 65536 || (need_idx && inner % V != 0))) V /= 2;
   const std::string Vs = std::to_string(V);
-  // Slots every read of which is at the output's own element index (linear,
-  // offset 0, same element size): the output may overwrite them in place (a
-  // donated input), so those operands and the output are not declared
-  // __restrict__: with donation they are one buffer.  (A thread's loads of its
-  // vector all precede its store.)
+  // Slots every read of which is at the outputs' own element index (linear, offset 0, an
+  // output's element size): an output may overwrite them in place (a donated input of
+  // its shape and dtype), so those operands and the outputs are not declared
+  // __restrict__: with donation they are one buffer.  (A thread's loads of its vector
+  // all precede its stores, and no other thread reads those elements.)
   std::vector<int> inplace;
   for (auto& in : ins) {
-    bool ok = !in.partial && roots.size() == 1;
+    bool ok = !in.partial;
     for (auto& o2 : ins)
       if (o2.view.slot == in.view.slot)
         ok = ok && !o2.partial && o2.linear && o2.view.offset == 0 &&
-             dtype_size(N[o2.value].shape.dtype) == dtype_size(os.dtype);
+             std::any_of(roots.begin(), roots.end(), [&](int r) {
+               return dtype_size(N[o2.value].shape.dtype) == dtype_size(N[r].shape.dtype);
+             });
     if (ok && std::find(inplace.begin(), inplace.end(), in.view.slot) == inplace.end()) inplace.push_back(in.view.slot);
   }
   auto may_alias = [&](const View& w) { return std::find(inplace.begin(), inplace.end(), w.slot) != inplace.end(); };

@@ -79,6 +79,50 @@ def test_donation_refused_when_the_input_is_read_later(be):
         be.BufferFinalize(b)
 
 
+@pytest.mark.parametrize("shape", [(256, 256), (641, 257)])
+def test_optimizer_state_is_donated(be, shape):
+    """One Adam step with p, m and v donated: p', m' and v' take their memory, also
+    where the clusters of m' and v' share a kernel (they share g); the values are those
+    of a step without donation."""
+    s = make_shape(F32, *shape)
+
+    def adam(f, p, m, v, g):
+        c = lambda x: f.Constant(np.float32(x))
+        m2 = f.Add(f.Mul(m, c(0.5)), f.Mul(g, c(0.5)))
+        v2 = f.Add(f.Mul(v, c(0.75)), f.Mul(f.Mul(g, g), c(0.25)))
+        return [f.Sub(p, f.Div(f.Mul(m2, c(0.125)), f.Add(f.Sqrt(v2), c(1e-8)))), m2, v2]
+
+    ex = _compile(be, "adam", adam, [s] * 4)
+    assert "outputs=2" in ex.Plan()
+    host = [synth.normal(5401 + i, shape) for i in range(4)]
+    host[2] = np.abs(host[2])
+    ins = [be.BufferFromFlatData(0, h, s) for h in host]
+    want = [be.BufferToFlatData(y).copy() for y in ex.Execute(ins, None, 0)]
+    ptrs = [be.BufferData(b) for b in ins]
+    outs = ex.Execute(ins, [True, True, True, False], 0)
+    assert [be.BufferData(y) for y in outs] == ptrs[:3]
+    for y, w in zip(outs, want):
+        assert np.array_equal(be.BufferToFlatData(y), w)
+    m2 = np.float32(0.5) * host[1] + np.float32(0.5) * host[3]
+    assert np.array_equal(want[1].reshape(shape), m2)
+
+
+def test_sharing_a_kernel_keeps_a_donation(be):
+    """b = x + y shares y with c = y * z, but x W is computed after c: b is written after
+    that product, where it takes x's donated memory, not with c."""
+    s = make_shape(F32, 256, 256)
+    ex = _compile(be, "late", lambda f, x, y, z, w: [f.Mul(y, z), f.DotGeneral(x, [1], [], w, [0], []), f.Add(x, y)],
+                  [s] * 4)
+    host = [synth.normal(5501 + i, (256, 256)) for i in range(4)]
+    ins = [be.BufferFromFlatData(0, h, s) for h in host]
+    px = be.BufferData(ins[0])
+    c, d, b = ex.Execute(ins, [True, False, False, False], 0)
+    assert be.BufferData(b) == px
+    assert np.array_equal(be.BufferToFlatData(b).reshape(256, 256), host[0] + host[1])
+    ref = host[0].astype(np.float64) @ host[3].astype(np.float64)
+    assert np.max(np.abs(be.BufferToFlatData(d).reshape(256, 256) - ref)) <= 1e-4 * np.max(np.abs(ref))
+
+
 def test_many_executes_and_finalizes_without_sync(be):
     """A state update (w <- 0.5 w + 1, n <- n + 1) run 200 times, each Execute
     donating the previous state, with no host synchronisation until the end: both
