@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "gomlx_hip.h"
+#include "reduce_dev.h"
 
 struct GHipBackend;
 struct GHipBuilder;
@@ -236,6 +237,27 @@ struct CopyDesc {
 };
 int launch_strided_copy(int elem_bytes, const void* src, void* dst, const CopyDesc& d,
                         hipStream_t s, GHipError* err);
+// Reduce of one strided operand into a contiguous result (k_reduce.hip).  Axes that one
+// stride spans are one axis; V consecutive values (ReduceGeom) are `step` elements apart.
+// ws: the ranges' values (g.C > 1), C * osize accumulators.
+struct ReduceAxes {
+  int orank = 0, rrank = 0;
+  int64_t odims[kMaxRank], ost[kMaxRank];
+  int64_t rdims[kMaxRank], rst[kMaxRank];
+  int64_t step = 0;
+  ReduceDiv odiv[kMaxRank], rdiv[kMaxRank];  // by odims / rdims, where the index fits 31 bits
+  bool o_wide = false, r_wide = false;       // it does not
+  bool line = false;  // one reduced axis; kept: one, columns one before and one after it; unit step
+};
+// The kernels are looked up when the graph is compiled (a launch by function handle costs
+// the host 0.5 us less than one by symbol).
+struct ReduceKernels {
+  hipFunction_t main = nullptr, finish = nullptr;
+};
+int reduce_kernels(int dtype, int op, const ReduceAxes& d, const ReduceGeom& g, bool plan_only, ReduceKernels* k,
+                   GHipError* err);
+int launch_reduce(const ReduceKernels& k, int op, const void* x, void* y, void* ws, const ReduceAxes& d,
+                  const ReduceGeom& g, int acc_bytes, hipStream_t s, GHipError* err);
 // Gather rows with int32 or int64 ids (clamped).
 int launch_gather_rows(const void* table, int64_t V, int64_t row_bytes, const void* ids,
                        int id_dtype, int64_t n, void* out, hipStream_t s, GHipError* err);

@@ -90,6 +90,10 @@ __device__ __forceinline__ long long ipow(long long b, long long e) {
 const char kGemmDevSrc[] =
 #include "gemm_bf16_dev.inc"
     ;
+// Text of reduce_dev.h, in front of generated reductions.
+const char kReduceDevSrc[] =
+#include "reduce_dev.inc"
+    ;
 
 std::string fmt(const char* f, ...) {
   char buf[512];
@@ -2340,25 +2344,74 @@ std::string Lowerer::member_stmt(int u, std::map<int, std::string>& expr, const 
 }
 
 
-// One generated kernel for Reduce R, evaluating its producer cluster (rooted at
-// prod_root, over R's input shape; -1: none) on the fly instead of reading it from
-// HBM, and, when cons_root >= 0, the consumer cluster (over R's output shape) on the
-// reduced value before the one store.  The accumulation order depends on R's shapes,
-// axes and dtype alone, and the reduced value is rounded to R's dtype before the
-// consumers see it, so results do not depend on what is fused.  Three forms:
-//   rows:    the reduced axes are the last ones.  A wave (few outputs: a workgroup of
-//            256 or 1024 threads) per output, V consecutive elements a lane and load.
-//   columns: one block of reduced axes before the last kept axes.  A workgroup takes
-//            TX vectors of V adjacent columns and strides the reduced index with its
-//            other lanes, so every load is coalesced; a butterfly, then LDS, combine.
-//   general: any other axes.  A wave per output (one thread below 64 values), an
-//            element a load.
-// The first two are bound by HBM; where they have too few workgroups to fill the chip
-// and enough data to pay for a second launch (from 2 MB read), the reduced range
-// splits over workgroups, whose partial results a finishing kernel combines in order.
+// Launch shape of a Reduce of x (dims, reduced axes red in order, element size es,
+// accumulator size as) with osize outputs of rsize values.  Three forms (reduce_dev.h):
+//   rows:    the reduced axes are the last ones; also, an element a load, any other axes
+//            of 64 values or more.
+//   columns: one block of reduced axes before the last kept axes.
+//   threads: any other axes.
+// Bound by HBM; where rows and columns have too few workgroups to fill the chip and
+// enough data to pay for a second launch (from 2 MB read), the reduced range splits over
+// workgroups, whose partial results a finishing kernel combines in order.
 // Measured, us, a wave per output with an element a load / here: bf16 [4096,2048] over
 // the rows, product fused 64 / 12.7 (8 ranges, both kernels); over the columns 19 / 5.8;
 // fp32 [256,10] to a scalar 12.7 / 2.0; [256,512] over the rows 5.3 / 4.4.
+static ReduceGeom reduce_geometry(const std::vector<int64_t>& dims, const std::vector<int>& red, int64_t osize,
+                                  int64_t rsize, int es, int as) {
+  const int rx = static_cast<int>(dims.size());
+  const int64_t last = rx ? dims[rx - 1] : 1;
+  int64_t inner = 1;
+  for (int i = red.empty() ? 0 : red.back() + 1; i < rx; ++i) inner *= dims[i];
+  bool block = !red.empty();  // reduced axes adjacent
+  for (size_t k = 1; k < red.size(); ++k) block = block && red[k] == red[k - 1] + 1;
+  const bool rows = block && red.back() == rx - 1 && rsize >= 64;
+  const bool cols = block && !rows && inner >= 8 && osize > 0 && rsize > 0;
+  int V = 1;
+  if (rows || cols) {
+    V = std::max(1, 16 / es);
+    while (V > 1 && (last % V != 0 || (rows ? rsize / V < 64 : inner / V < 8))) V /= 2;
+  }
+  int64_t C = 1, gx = 0, cblocks = 1;
+  int L = 64, NT = 256;
+  const bool split_pays = osize * rsize * es >= (int64_t{1} << 21);
+  if (rows) {
+    if (osize <= 256 && rsize >= 2048 * V) L = 1024;
+    else if (osize <= 1024 && rsize >= 512 * V) L = 256;
+    NT = std::max(256, L);
+    gx = (osize + NT / L - 1) / (NT / L);
+    if (split_pays && osize > 0 && gx < 128) C = std::min<int64_t>(256 / gx, rsize / (int64_t{4} * L * V));
+  } else if (cols) {
+    const int64_t outer = osize / inner, vecs = (inner + V - 1) / V;
+    while (L > 1 && L / 2 >= vecs) L /= 2;
+    // Narrower column blocks until the chip is full, down to a 128-byte line.
+    while (L > 1 && L * V * es > 128 && outer * ((vecs + L - 1) / L) < 512) L /= 2;
+    if (rsize >= 512 && outer * ((vecs + L - 1) / L) < 1024) NT = 1024;
+    while (NT / 64 * L * V * as > 65536) L /= 2;  // the combine step's LDS
+    cblocks = (vecs + L - 1) / L;
+    gx = outer * cblocks;
+    if (split_pays && gx < 128) C = std::min<int64_t>(256 / gx, rsize / (int64_t{4} * (NT / L)));
+  } else {
+    gx = rsize >= 64 ? (osize + 3) / 4 : (osize + 255) / 256;
+  }
+  if (C < 2) C = 1;
+  const int64_t unit = rows ? static_cast<int64_t>(L) * V : cols ? NT / L : 1;
+  const int64_t chunk = C > 1 ? (rsize + C * unit - 1) / (C * unit) * unit : rsize;
+  if (C > 1) C = (rsize + chunk - 1) / chunk;
+  ReduceGeom g;
+  g.osize = osize, g.rsize = rsize, g.inner = inner, g.gx = gx, g.chunk = chunk, g.C = static_cast<int>(C);
+  g.form = cols ? kReduceColumns : rows || rsize >= 64 ? kReduceRows : kReduceThreads;
+  auto log2i = [](int v) { return 31 - __builtin_clz(static_cast<unsigned>(v)); };
+  g.V = V, g.log_l = log2i(L), g.log_nt = log2i(NT), g.cblocks = reduce_div(static_cast<unsigned>(std::max<int64_t>(cblocks, 1)));
+  return g;
+}
+
+// One generated kernel for Reduce R, evaluating its producer cluster (rooted at
+// prod_root, over R's input shape; -1: none) on the fly instead of reading it from
+// HBM, and, when cons_root >= 0, the consumer cluster (over R's output shape) on the
+// reduced value before the one store; with neither, the precompiled kernel.  The
+// accumulation order depends on R's shapes, axes and dtype alone, and the reduced value
+// is rounded to R's dtype before the consumers see it, so results do not depend on what
+// is fused.
 View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
   const Node& rn = N[R];
   const int x = rn.in[0];
@@ -2372,53 +2425,86 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
   for (int i : kept) osize *= xs.dims[i];
   for (int i : red) rsize *= xs.dims[i];
   const int rdt = rs.dtype, xdt = xs.dtype;
-  // ---- form and launch shape
-  const int64_t last = rx ? xs.dims[rx - 1] : 1;
-  int64_t inner = 1;  // kept elements after the last reduced axis
-  for (int i = red.empty() ? 0 : red.back() + 1; i < rx; ++i) inner *= xs.dims[i];
-  bool block = !red.empty();  // reduced axes adjacent
-  for (size_t k = 1; k < red.size(); ++k) block = block && red[k] == red[k - 1] + 1;
-  const bool rows = block && red.back() == rx - 1 && rsize >= 64;
-  const bool cols = block && !rows && inner >= 8 && osize > 0 && rsize > 0;
-  int V = 1;
-  if (rows || cols) {
-    V = std::max(1, 16 / dtype_size(xdt));
-    while (V > 1 && (last % V != 0 || (rows ? rsize / V < 64 : inner / V < 8))) V /= 2;
-  }
-  int64_t C = 1;                     // ranges of the reduced index
-  int L = 64, NT = 256;              // rows: lanes per output
-  int TX = 64;                       // columns: vectors per workgroup
-  int64_t gx = 0, cblocks = 1;
-  const int64_t bytes = osize * rsize * dtype_size(xdt);
-  const bool split_pays = bytes >= (int64_t{1} << 21);
-  if (rows) {
-    if (osize <= 256 && rsize >= 2048 * V) L = 1024;
-    else if (osize <= 1024 && rsize >= 512 * V) L = 256;
-    NT = std::max(256, L);
-    gx = (osize + NT / L - 1) / (NT / L);
-    if (split_pays && osize > 0 && gx < 128) C = std::min<int64_t>(256 / gx, rsize / (int64_t{4} * L * V));
-  } else if (cols) {
-    const int64_t outer = osize / inner, vecs = (inner + V - 1) / V;
-    while (TX > 1 && TX / 2 >= vecs) TX /= 2;
-    // Narrower column blocks until the chip is full, down to a 128-byte line.
-    while (TX > 1 && TX * V * dtype_size(xdt) > 128 && outer * ((vecs + TX - 1) / TX) < 512) TX /= 2;
-    cblocks = (vecs + TX - 1) / TX;
-    gx = outer * cblocks;
-    NT = rsize >= 512 && gx < 1024 ? 1024 : 256;
-    if (split_pays && gx < 128) C = std::min<int64_t>(256 / gx, rsize / (int64_t{4} * (NT / TX)));
-  } else {
-    gx = rsize >= 64 ? (osize + 3) / 4 : (osize + 255) / 256;
-  }
-  if (C < 2) C = 1;
-  const int64_t unit = rows ? static_cast<int64_t>(L) * V : cols ? NT / TX : 1;
-  const int64_t chunk = C > 1 ? (rsize + C * unit - 1) / (C * unit) * unit : rsize;
-  if (C > 1) C = (rsize + chunk - 1) / chunk;
-  if (gx > 0x7fffffffLL) return fail(GHIP_ERR_UNSUPPORTED, "Reduce: too many outputs");
-  const bool wave = !rows && !cols && rsize >= 64;
+  const ReduceGeom g = reduce_geometry(xs.dims, red, osize, rsize, dtype_size(xdt),
+                                       dtype_is_int(rdt) || rdt == GHIP_DTYPE_FLOAT64 ? 8 : 4);
+  if (g.gx > 0x7fffffffLL) return fail(GHIP_ERR_UNSUPPORTED, "Reduce: too many outputs");
+  const int V = g.V;
   // Accumulator type (fp32, fp64 or 64-bit integers).
   std::string acc_t = "float";
   if (rdt == GHIP_DTYPE_FLOAT64) acc_t = "double";
   else if (dtype_is_int(rdt)) acc_t = dtype_is_unsigned(rdt) ? "unsigned long long" : "long long";
+  static const char* names[] = {"sum", "product", "max", "min"};
+  const bool fused = prod_root >= 0 || cons_root >= 0;
+  const int wdt = acc_t == "float" ? GHIP_DTYPE_FLOAT32 : GHIP_DTYPE_INT64;
+  View wsv;  // the ranges' values
+  auto range_slots = [&](const View& y) {
+    std::vector<int> wr{y.slot};
+    if (g.C > 1) {
+      Shape wss;
+      wss.dtype = wdt;
+      wss.dims = {g.C * osize};
+      wsv = fresh(wss);
+      wr.push_back(wsv.slot);
+    }
+    return wr;
+  };
+  auto describe = [&](const Shape& os) {
+    std::string desc = fmt("%sreduce_%s %s -> %s", fused ? "fused_" : "", names[rn.sub], xs.str().c_str(), os.str().c_str());
+    if (prod_root >= 0) desc += " (producer fused)";
+    if (cons_root >= 0) desc += " (consumer fused)";
+    if (g.C > 1) desc += fmt(" (in %d ranges)", g.C);
+    return desc;
+  };
+  if (!fused) {
+    const View xv = get(x);
+    if (failed) return bad();
+    ReduceAxes d;
+    // Adjacent axes that one stride spans fold into one (columns: not across the block).
+    auto fold = [&](const std::vector<int>& axes, int* rank, int64_t* dims, int64_t* st, int from) {
+      for (int i : axes) {
+        if (xs.dims[i] == 1) continue;
+        if (*rank > from && st[*rank - 1] == xs.dims[i] * xv.strides[i]) {
+          dims[*rank - 1] *= xs.dims[i];
+          st[*rank - 1] = xv.strides[i];
+        } else {
+          dims[*rank] = xs.dims[i];
+          st[(*rank)++] = xv.strides[i];
+        }
+      }
+    };
+    auto finish_axes = [](int* rank, int64_t* dims, int64_t* st, ReduceDiv* div, int64_t size) {
+      if (*rank == 0) {
+        dims[0] = 1;
+        st[(*rank)++] = 0;
+      }
+      const bool wide = size >> 31;
+      for (int k = 0; k < *rank && !wide; ++k) div[k] = reduce_div(static_cast<unsigned>(std::max<int64_t>(dims[k], 1)));
+      return wide;
+    };
+    std::vector<int> before, after;
+    for (int i : kept) (g.form == kReduceColumns && i > red.back() ? after : before).push_back(i);
+    fold(before, &d.orank, d.odims, d.ost, 0);
+    const int n_before = d.orank;
+    fold(after, &d.orank, d.odims, d.ost, n_before);
+    const int n_after = d.orank - n_before;
+    fold(red, &d.rrank, d.rdims, d.rst, 0);
+    d.o_wide = finish_axes(&d.orank, d.odims, d.ost, d.odiv, osize);
+    d.r_wide = finish_axes(&d.rrank, d.rdims, d.rst, d.rdiv, rsize);
+    d.step = g.form == kReduceColumns ? d.ost[d.orank - 1] : d.rst[d.rrank - 1];
+    d.line = d.rrank == 1 && n_before <= 1 && n_after <= 1 && (V == 1 || d.step == 1);
+    const View y = fresh(rs);
+    const std::vector<int> wr = range_slots(y);
+    const View ws = wsv;
+    const int op = rn.sub;
+    if (!be->plan_only) hipSetDevice(be->device);
+    ReduceKernels k;
+    if (reduce_kernels(rdt, op, d, g, be->plan_only, &k, err) != GHIP_OK) return bad();
+    add_step(describe(rs), {xv.slot}, wr, [=](ExecState& st, GHipError* e) {
+      return launch_reduce(k, op, st.ptr(xv, rdt), st.ptr(y, rdt), g.C > 1 ? st.ptr(ws, wdt) : nullptr, d, g,
+                           dtype_size(wdt), st.stream, e);
+    });
+    return y;
+  }
   struct In {
     View view;
     int dt;
@@ -2529,116 +2615,68 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
       init = acc_t == "float" ? "__builtin_inff()" : acc_t == "double" ? "__builtin_inf()"
            : acc_t == "long long" ? "9223372036854775807LL" : "18446744073709551615ull";
   }
-  std::string params, args_s;
+  std::string params, args_s, fields;
   for (size_t k = 0; k < ins.size(); ++k) {
     params += "const void* __restrict__ p_in" + std::to_string(k) + ", ";
     args_s += "p_in" + std::to_string(k) + ", ";
+    fields += "  const void* p_in" + std::to_string(k) + ";\n";
   }
-  const std::string ws_t = acc_t + "* __restrict__ p_ws";
-  // Coordinates: 32-bit where the index fits.
-  auto coords = [&](const std::string& idx, const std::vector<int>& axes, const char* name, int64_t size, const char* ind) {
+  const std::string Vs = std::to_string(V);
+  // Coordinates (axes of index idx): 32-bit where the index fits.
+  auto coords = [&](const std::string& idx, const std::vector<int>& axes, const char* name, int64_t size, const char* decl) {
     std::ostringstream s;
     const std::string I = size < (int64_t{1} << 31) ? "unsigned" : "long long";
     if (axes.size() == 1) {
-      s << ind << "const long long " << name << "0 = " << idx << ";\n";
+      s << "    " << decl << name << "0 = " << idx << ";\n";
     } else if (!axes.empty()) {
-      s << ind << I << " q_" << name << " = (" << I << ")(" << idx << ");\n";
+      s << "    " << I << " q_" << name << " = (" << I << ")(" << idx << ");\n";
       for (int k = static_cast<int>(axes.size()) - 1; k >= 0; --k)
-        s << ind << "const long long " << name << k << " = (long long)(q_" << name << " % (" << I << ")" << xs.dims[axes[k]]
+        s << "    " << decl << name << k << " = (long long)(q_" << name << " % (" << I << ")" << xs.dims[axes[k]]
           << "LL); q_" << name << " /= (" << I << ")" << xs.dims[axes[k]] << "LL;\n";
     }
     return s.str();
   };
   std::ostringstream pre;
-  pre << kRtcPrelude << "__device__ __forceinline__ " << acc_t << " comb(" << acc_t << " a, " << acc_t << " b) { return "
-      << ops[rn.sub] << "; }\n"
+  pre << kRtcPrelude << kReduceDevSrc << "typedef " << acc_t << " acc_t;\n"
+      << "struct Comb { __device__ __forceinline__ acc_t operator()(acc_t a, acc_t b) const { return " << ops[rn.sub] << "; } };\n"
+      << "constexpr ghip::ReduceGeom geom = {" << g.osize << "LL, " << g.rsize << "LL, " << g.inner << "LL, " << g.gx << "LL, "
+      << g.chunk << "LL, " << g.C << ", " << g.form << ", " << g.V << ", " << g.log_l << ", " << g.log_nt << ", {" << g.cblocks.d
+      << "u, " << g.cblocks.mul << "u, " << g.cblocks.shift << "}};\n"
       // Output o from its reduced value, which is rounded as the unfused plan stores it.
-      << "__device__ __forceinline__ void finish(long long o, " << acc_t << " acc, " << params << "void* __restrict__ p_out) {\n"
-      << coords("o", kept, "o", osize, "  ") << "  const " << ctype(rdt) << " red = "
+      << "__device__ __forceinline__ void finish(long long o, acc_t acc, " << params << "void* __restrict__ p_out) {\n"
+      << coords("o", kept, "o", osize, "const long long ") << "  const " << ctype(rdt) << " red = "
       << load_expr(rdt, "(" + stype(rdt) + ")(" + store_expr(rdt, "(" + ctype(rdt) + ")acc") + ")") << ";\n"
       << cbody.str() << "  ((" << stype(odt) << "*)p_out)[o] = " << store_expr(odt, outv) << ";\n}\n";
-  auto done = [&](const std::string& o, const std::string& a) {
-    return C > 1 ? "p_ws[(long long)blockIdx.y * " + std::to_string(osize) + "LL + " + o + "] = " + a + ";"
-                 : "finish(" + o + ", " + a + ", " + args_s + "p_out);";
-  };
   std::ostringstream src;
-  src << pre.str() << "extern \"C\" __global__ void __launch_bounds__(" << NT << ") fused_reduce(" << params
-      << "void* __restrict__ p_out, " << ws_t << ") {\n  const int t = threadIdx.x;\n";
-  const std::string accs = "  " + acc_t + " acc[" + std::to_string(V) + "];\n#pragma unroll\n  for (int e = 0; e < " +
-                           std::to_string(V) + "; ++e) acc[e] = " + init + ";\n";
-  const std::string range = "  const long long r_end = " +
-      (C > 1 ? "((long long)blockIdx.y + 1) * " + std::to_string(chunk) + "LL < " + std::to_string(rsize) +
-                   "LL ? ((long long)blockIdx.y + 1) * " + std::to_string(chunk) + "LL : " + std::to_string(rsize) + "LL"
-             : std::to_string(rsize) + "LL") + ";\n";
-  const std::string start = C > 1 ? "(long long)blockIdx.y * " + std::to_string(chunk) + "LL + " : "";
-  auto step = [&]() {
-    std::ostringstream s;
-    s << coords("r", red, "r", rsize, "      ") << loads.str() << "#pragma unroll\n      for (int e = 0; e < " << V << "; ++e) {\n"
-      << pbody.str() << "      acc[e] = comb(acc[e], (" << acc_t << ")(" << val << "));\n      }\n    }\n";
-    return s.str();
-  };
-  if (rows) {
-    src << "  const int lane = t % " << L << ";\n  const long long o = (long long)blockIdx.x * " << NT / L << " + t / " << L << ";\n";
-    if (L == 64) src << "  if (o >= " << osize << "LL) return;\n";
-    src << coords("o", kept, "o", osize, "  ") << accs << range << "#pragma unroll 4\n  for (long long r = " << start << "lane * " << V
-        << "; r < r_end; r += " << L * V << ") {\n"
-        << step() << "  " << acc_t << " a = acc[0];\n#pragma unroll\n  for (int e = 1; e < " << V << "; ++e) a = comb(a, acc[e]);\n"
-        << "#pragma unroll\n  for (int off = 32; off >= 1; off >>= 1) a = comb(a, __shfl_xor(a, off, 64));\n";
-    if (L > 64)
-      src << "  __shared__ " << acc_t << " part[" << L / 64 << "];\n  if (t % 64 == 0) part[t / 64] = a;\n  __syncthreads();\n"
-          << "  if (t != 0) return;\n  for (int w = 1; w < " << L / 64 << "; ++w) a = comb(a, part[w]);\n";
-    else
-      src << "  if (lane != 0) return;\n";
-    src << "  " << done("o", "a") << "\n}\n";
-  } else if (cols) {
-    const int TY = NT / TX, NW = NT / 64;
-    // Kept index of the vector's first column: axes before the reduced block, then inner.
-    src << "  const int tx = t % " << TX << ", ty = t / " << TX << ";\n  const long long ou = blockIdx.x / " << cblocks
-        << ", col = ((long long)(blockIdx.x % " << cblocks << ") * " << TX << " + tx) * " << V << ";\n"
-        << "  const bool ok = col < " << inner << "LL;\n  const long long o = ou * " << inner << "LL + (ok ? col : 0);\n"
-        << coords("o", kept, "o", osize, "  ") << accs << range << "#pragma unroll 4\n  for (long long r = " << start << "ty; r < r_end; r += "
-        << TY << ") {\n" << step();
-    const int W = std::max(TX, 1);
-    if (TX < 64)
-      src << "#pragma unroll\n  for (int off = " << TX << "; off <= 32; off <<= 1)\n#pragma unroll\n    for (int e = 0; e < " << V
-          << "; ++e) acc[e] = comb(acc[e], __shfl_xor(acc[e], off, 64));\n";
-    src << "  __shared__ " << acc_t << " part[" << NW << "][" << W * V << "];\n  if (t % 64 < " << TX << ")\n#pragma unroll\n    for (int e = 0; e < "
-        << V << "; ++e) part[t / 64][tx * " << V << " + e] = acc[e];\n  __syncthreads();\n"
-        << "  for (int c = t; c < " << W * V << "; c += " << NT << ") {\n    const long long oc = (long long)(blockIdx.x % " << cblocks << ") * "
-        << TX * V << " + c;\n    if (oc >= " << inner << "LL) return;\n    " << acc_t << " a = part[0][c];\n    for (int w = 1; w < " << NW
-        << "; ++w) a = comb(a, part[w][c]);\n    const long long of = ou * " << inner << "LL + oc;\n    " << done("of", "a") << "\n  }\n}\n";
-  } else {
-    if (wave) src << "  const long long o = (long long)blockIdx.x * 4 + t / 64;\n  const int lane = t % 64;\n";
-    else src << "  const long long o = (long long)blockIdx.x * 256 + t;\n";
-    src << "  if (o >= " << osize << "LL) return;\n" << coords("o", kept, "o", osize, "  ") << accs << "  for (long long r = "
-        << (wave ? "lane" : "0") << "; r < " << rsize << "LL; r += " << (wave ? 64 : 1) << ") {\n"
-        << step() << "  " << acc_t << " a = acc[0];\n";
-    if (wave)
-      src << "#pragma unroll\n  for (int off = 32; off >= 1; off >>= 1) a = comb(a, __shfl_xor(a, off, 64));\n  if (lane != 0) return;\n";
-    src << "  " << done("o", "a") << "\n}\n";
-  }
+  src << pre.str() << "struct Src {\n" << fields;
+  for (size_t k = 0; k < kept.size(); ++k) src << "  long long o" << k << ";\n";
+  src << "  __device__ __forceinline__ void at(long long o) {\n" << coords("o", kept, "o", osize, "")
+      << "  }\n  __device__ __forceinline__ void at(long long ou, long long col) { at(ou * geom.inner + col); }\n"
+      << "  __device__ __forceinline__ void get(long long r, acc_t (&v)[" << Vs << "]) const {\n"
+      << coords("r", red, "r", rsize, "const long long ") << loads.str() << "#pragma unroll\n      for (int e = 0; e < " << Vs << "; ++e) {\n"
+      << pbody.str() << "      v[e] = (acc_t)(" << val << ");\n      }\n  }\n};\n"
+      << "struct Dst {\n" << fields << "  void* p_out;\n  acc_t* p_ws;\n"
+      << "  __device__ __forceinline__ void put(long long o, acc_t a) const {\n    "
+      << (g.C > 1 ? "p_ws[blockIdx.y * geom.osize + o] = a;" : "finish(o, a, " + args_s + "p_out);") << "\n  }\n};\n"
+      << "extern \"C\" __global__ void __launch_bounds__(" << (1 << g.log_nt) << ") fused_reduce(" << params
+      << "void* __restrict__ p_out, acc_t* __restrict__ p_ws) {\n  __shared__ acc_t part[ghip::reduce_lds(geom)];\n"
+      << "  Src src{" << args_s << "};\n  const Dst dst{" << args_s << "p_out, p_ws};\n"
+      << "  ghip::reduce_body<" << g.form << ", " << Vs << ">(geom, (acc_t)" << init << ", Comb{}, src, dst, part);\n}\n";
   RtcKernel kern, fin;
   if (rtc_get(be, src.str(), "fused_reduce", &kern, err) != GHIP_OK) return bad();
-  if (C > 1) {
+  if (g.C > 1) {
     std::ostringstream fs;
-    fs << pre.str() << "extern \"C\" __global__ void __launch_bounds__(256) reduce_finish(" << params << "void* __restrict__ p_out, "
-       << ws_t << ") {\n  const long long o = (long long)blockIdx.x * 256 + threadIdx.x;\n  if (o >= " << osize << "LL) return;\n  "
-       << acc_t << " a = p_ws[o];\n#pragma unroll 16\n  for (int c = 1; c < " << C << "; ++c) a = comb(a, p_ws[o + c * " << osize
-       << "LL]);\n  finish(o, a, " << args_s << "p_out);\n}\n";
+    fs << pre.str() << "extern \"C\" __global__ void __launch_bounds__(256) reduce_finish(" << params
+       << "void* __restrict__ p_out, const acc_t* __restrict__ p_ws) {\n"
+       << "  const long long o = (long long)blockIdx.x * 256 + threadIdx.x;\n"
+       << "  if (o < geom.osize) finish(o, ghip::reduce_ranges(geom, p_ws, o, Comb{}), " << args_s << "p_out);\n}\n";
     if (rtc_get(be, fs.str(), "reduce_finish", &fin, err) != GHIP_OK) return bad();
   }
   const Shape& os = N[out_v].shape;
   View y = fresh(os);
-  View wsv;
-  std::vector<int> rd, wr{y.slot};
-  const int wdt = acc_t == "float" ? GHIP_DTYPE_FLOAT32 : GHIP_DTYPE_INT64;
-  if (C > 1) {
-    Shape wss;
-    wss.dtype = wdt;
-    wss.dims = {C * osize};
-    wsv = fresh(wss);
-    wr.push_back(wsv.slot);
-  }
+  std::vector<int> rd;
+  const std::vector<int> wr = range_slots(y);
+  const View ws = wsv;
   std::vector<View> in_views;
   std::vector<int> in_dt;
   for (auto& in : ins) {
@@ -2646,25 +2684,19 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
     in_views.push_back(in.view);
     in_dt.push_back(in.dt);
   }
-  static const char* names[] = {"sum", "product", "max", "min"};
-  const bool fused = prod_root >= 0 || cons_root >= 0;
-  std::string desc = fmt("%sreduce_%s %s -> %s", fused ? "fused_" : "", names[rn.sub], xs.str().c_str(), os.str().c_str());
-  if (prod_root >= 0) desc += " (producer fused)";
-  if (cons_root >= 0) desc += " (consumer fused)";
-  if (C > 1) desc += fmt(" (in %lld ranges)", (long long)C);
-  add_step(desc, rd, wr, [=](ExecState& st, GHipError* e) -> int {
+  add_step(describe(os), rd, wr, [=](ExecState& st, GHipError* e) -> int {
     if (osize == 0) return GHIP_OK;
     std::vector<void*> ptrs(in_views.size());
     std::vector<void*> args;
     for (size_t k = 0; k < in_views.size(); ++k) ptrs[k] = st.ptr(in_views[k], in_dt[k]);
     void* outp = st.ptr(y, odt);
-    void* wsp = C > 1 ? st.ptr(wsv, wdt) : nullptr;
+    void* wsp = g.C > 1 ? st.ptr(ws, wdt) : nullptr;
     for (size_t k = 0; k < ptrs.size(); ++k) args.push_back(&ptrs[k]);
     args.push_back(&outp);
     args.push_back(&wsp);
-    hipError_t h = hipModuleLaunchKernel(kern.func, static_cast<unsigned>(gx), static_cast<unsigned>(C), 1, NT, 1, 1, 0,
+    hipError_t h = hipModuleLaunchKernel(kern.func, static_cast<unsigned>(g.gx), static_cast<unsigned>(g.C), 1, 1u << g.log_nt, 1, 1, 0,
                                          st.stream, args.data(), nullptr);
-    if (h == hipSuccess && C > 1)
+    if (h == hipSuccess && g.C > 1)
       h = hipModuleLaunchKernel(fin.func, static_cast<unsigned>((osize + 255) / 256), 1, 1, 256, 1, 1, 0, st.stream,
                                 args.data(), nullptr);
     if (h != hipSuccess) return check_hip(h, e, "generated reduce kernel launch");

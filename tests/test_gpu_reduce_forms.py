@@ -85,3 +85,42 @@ def test_split_reduce_says_so(be):
         ex = b.Compile()
         assert "ranges)" in ex.Plan()
         ex.Finalize()
+
+
+VIEWS = [  # (operand shape, permutation, last-axis slice stride, reduced axes of the view)
+    ((40, 96, 130), (0, 1, 2), 1, [2]), ((40, 96, 130), (2, 0, 1), 1, [2]), ((40, 96, 130), (1, 2, 0), 2, [0]),
+    ((40, 96, 128), (0, 1, 2), 2, [1]), ((5, 6, 7, 72), (2, 0, 3, 1), 1, [1, 3]), ((5, 6, 7, 72), (1, 3, 0, 2), 1, [0, 2]),
+    ((4, 3, 2, 5, 64), (0, 2, 1, 3, 4), 1, [2, 3]), ((9, 70, 8), (0, 1, 2), 1, [1]), ((2, 3, 4096), (1, 0, 2), 1, [1, 2]),
+]
+
+
+@pytest.mark.parametrize("shape,perm,stride,axes", VIEWS)
+@pytest.mark.parametrize("op", ["ReduceSum", "ReduceProduct", "ReduceMax", "ReduceMin"])
+@pytest.mark.parametrize("dt,npt", [(dtypes.Int8, np.int8), (dtypes.Uint8, np.uint8), (dtypes.Int16, np.int16),
+                                    (dtypes.Uint16, np.uint16), (dtypes.Uint32, np.uint32), (dtypes.Int64, np.int64),
+                                    (dtypes.Uint64, np.uint64), (dtypes.Float64, np.float64), (F32, np.float32)])
+def test_strided_operands(be, shape, perm, stride, axes, op, dt, npt):
+    """Every dtype and operation over transposed and strided views, small whole numbers:
+    exact (sums and products of the integer types wrap)."""
+    u = synth.uniform_f32(9101, shape, 0, 1)
+    signed = np.issubdtype(npt, np.signedinteger) or npt in (np.float32, np.float64)
+    if op == "ReduceProduct":  # mostly ones
+        x = np.where(u < 0.03, 2, np.where((u > 0.97) & signed, -1, 1)).astype(npt)
+    else:
+        x = (np.floor(u * 100) - (50 if signed else 0)).astype(npt)
+    print(shape, perm, stride, axes, op, dt, flush=True)
+    b = be.Builder("strided")
+    f = b.Main()
+    v = f.Transpose(f.Parameter("x", make_shape(dt, *shape)), *perm)
+    dims = [shape[p] for p in perm]
+    if stride > 1:
+        v = f.Slice(v, [0] * len(dims), dims, [1] * (len(dims) - 1) + [stride])
+    f.Return([getattr(f, op)(v, *axes)])
+    ex = b.Compile()
+    (y,) = ex.Execute([be.BufferFromFlatData(0, x, make_shape(dt, *shape))])
+    got = be.BufferToFlatData(y).reshape(be.BufferShape(y).dims)
+    ex.Finalize()
+    view = x.transpose(perm)[..., ::stride]
+    fn = {"ReduceSum": np.sum, "ReduceProduct": np.prod, "ReduceMax": np.max, "ReduceMin": np.min}[op]
+    want = fn(view, axis=tuple(axes), **({"dtype": npt} if op in ("ReduceSum", "ReduceProduct") else {}))
+    assert np.array_equal(got, want)

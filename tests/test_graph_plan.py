@@ -598,3 +598,17 @@ def test_a_cluster_that_an_operand_needs_is_stored_once(be, build, clusters, are
     assert [l.split(" inputs=")[1].split(" ", 1)[1] for l in p.splitlines()
             if l.startswith("fused_elementwise")] == clusters, p
     assert f"arena {arena} bytes" in p, p
+
+
+def test_plain_reduces_compile_no_kernel(be, monkeypatch, tmp_path):
+    """A Reduce without a fused cluster runs a precompiled kernel, whatever its shape,
+    axes and operand strides: compiling it generates none."""
+    monkeypatch.setenv("GHIP_RTC_DUMP", str(tmp_path))
+    for i in range(20):
+        def build(f):
+            x = f.Parameter("x", make_shape([F32, BF16, dtypes.Int8][i % 3], 3 + i, 40 + i, 64))
+            return [f.ReduceMax(x, 1), f.ReduceSum(x, 2), f.ReduceSum(x), f.ReduceMin(x, 0, 2),
+                    f.ReduceProduct(f.Transpose(x, 2, 0, 1), 1)]
+        p = plan_of(be, build)
+        assert p.count("reduce_") == 5 and "fused" not in p, p
+    assert not list(tmp_path.iterdir())
