@@ -2349,7 +2349,7 @@ std::string Lowerer::member_stmt(int u, std::map<int, std::string>& expr, const 
 //   rows:    the reduced axes are the last ones; also, an element a load, any other axes
 //            of 64 values or more.
 //   columns: one block of reduced axes before the last kept axes.
-//   threads: any other axes.
+//   threads: any other axes; also columns of few bytes (below).
 // Bound by HBM; where rows and columns have too few workgroups to fill the chip and
 // enough data to pay for a second launch (from 2 MB read), the reduced range splits over
 // workgroups, whose partial results a finishing kernel combines in order.
@@ -2366,13 +2366,15 @@ static ReduceGeom reduce_geometry(const std::vector<int64_t>& dims, const std::v
   for (size_t k = 1; k < red.size(); ++k) block = block && red[k] == red[k - 1] + 1;
   const bool rows = block && red.back() == rx - 1 && rsize >= 64;
   const bool cols = block && !rows && inner >= 8 && osize > 0 && rsize > 0;
-  int V = 1;
-  if (rows || cols) {
-    V = std::max(1, 16 / es);
-    while (V > 1 && (last % V != 0 || (rows ? rsize / V < 64 : inner / V < 8))) V /= 2;
-  }
+  auto widest = [&](auto narrow) {  // elements a load: up to 16 bytes, within a row of the last axis
+    int v = std::max(1, 16 / es);
+    while (v > 1 && (last % v != 0 || narrow(v))) v /= 2;
+    return v;
+  };
+  int V = rows ? widest([&](int v) { return rsize / v < 64; }) : cols ? widest([&](int v) { return inner / v < 8; }) : 1;
   int64_t C = 1, gx = 0, cblocks = 1;
   int L = 64, NT = 256;
+  bool threads = !rows && !cols && rsize < 64;
   const bool split_pays = osize * rsize * es >= (int64_t{1} << 21);
   if (rows) {
     if (osize <= 256 && rsize >= 2048 * V) L = 1024;
@@ -2390,16 +2392,26 @@ static ReduceGeom reduce_geometry(const std::vector<int64_t>& dims, const std::v
     cblocks = (vecs + L - 1) / L;
     gx = outer * cblocks;
     if (split_pays && gx < 128) C = std::min<int64_t>(256 / gx, rsize / (int64_t{4} * (NT / L)));
-  } else {
-    gx = rsize >= 64 ? (osize + 3) / 4 : (osize + 255) / 256;
+    // Many workgroups of little data each: a workgroup's combine steps cost 0.6 ns of the
+    // launch (1.2 from V = 8), more than a thread per V outputs (two bytes or more a lane,
+    // still 65536 threads) loses by its serial range.  us, columns / threads: bf16
+    // [65536,8,8] 38.6 / 7.1, [32768,20,64] 38.9 / 21.8, [8192,8,64] 11.2 / 6.7, fp32
+    // [32768,8,64] 23.1 / 15.2, but bf16 [8192,60,8] 7.5 / 9.8, [32768,60,64] 39.7 / 56.8,
+    // fp32 [8192,20,64] 9.4 / 11.4, [4096,8,512] 13.1 / 15.1.
+    if (rsize < 64 && rsize * L * V * es < std::min<int64_t>(4096, gx / (V >= 8 ? 6 : 12))) {
+      threads = true;
+      V = widest([&](int v) { return osize / v < 65536; });
+    }
   }
+  if (threads) gx = (osize / V + 255) / 256;
+  else if (!rows && !cols) gx = (osize + 3) / 4;
   if (C < 2) C = 1;
   const int64_t unit = rows ? static_cast<int64_t>(L) * V : cols ? NT / L : 1;
   const int64_t chunk = C > 1 ? (rsize + C * unit - 1) / (C * unit) * unit : rsize;
   if (C > 1) C = (rsize + chunk - 1) / chunk;
   ReduceGeom g;
   g.osize = osize, g.rsize = rsize, g.inner = inner, g.gx = gx, g.chunk = chunk, g.C = static_cast<int>(C);
-  g.form = cols ? kReduceColumns : rows || rsize >= 64 ? kReduceRows : kReduceThreads;
+  g.form = threads ? kReduceThreads : cols ? kReduceColumns : kReduceRows;
   auto log2i = [](int v) { return 31 - __builtin_clz(static_cast<unsigned>(v)); };
   g.V = V, g.log_l = log2i(L), g.log_nt = log2i(NT), g.cblocks = reduce_div(static_cast<unsigned>(std::max<int64_t>(cblocks, 1)));
   return g;
@@ -2453,7 +2465,8 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
     if (prod_root >= 0) desc += " (producer fused)";
     if (cons_root >= 0) desc += " (consumer fused)";
     if (g.C > 1) desc += fmt(" (in %d ranges)", g.C);
-    return desc;
+    static const char* forms[] = {"rows", "columns", "threads"};
+    return desc + fmt(" [%s, %d wide, grid %u x %u x %d]", forms[g.form], g.V, reduce_grid_x(g), reduce_grid_y(g), 1 << g.log_nt);
   };
   if (!fused) {
     const View xv = get(x);
@@ -2490,7 +2503,7 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
     fold(red, &d.rrank, d.rdims, d.rst, 0);
     d.o_wide = finish_axes(&d.orank, d.odims, d.ost, d.odiv, osize);
     d.r_wide = finish_axes(&d.rrank, d.rdims, d.rst, d.rdiv, rsize);
-    d.step = g.form == kReduceColumns ? d.ost[d.orank - 1] : d.rst[d.rrank - 1];
+    d.step = g.form == kReduceRows ? d.rst[d.rrank - 1] : d.ost[d.orank - 1];
     d.line = d.rrank == 1 && n_before <= 1 && n_after <= 1 && (V == 1 || d.step == 1);
     const View y = fresh(rs);
     const std::vector<int> wr = range_slots(y);
@@ -2643,10 +2656,11 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
       << g.chunk << "LL, " << g.C << ", " << g.form << ", " << g.V << ", " << g.log_l << ", " << g.log_nt << ", {" << g.cblocks.d
       << "u, " << g.cblocks.mul << "u, " << g.cblocks.shift << "}};\n"
       // Output o from its reduced value, which is rounded as the unfused plan stores it.
-      << "__device__ __forceinline__ void finish(long long o, acc_t acc, " << params << "void* __restrict__ p_out) {\n"
+      << "__device__ __forceinline__ " << stype(odt) << " finish(long long o, acc_t acc, "
+      << params.substr(0, params.size() - 2) << ") {\n"
       << coords("o", kept, "o", osize, "const long long ") << "  const " << ctype(rdt) << " red = "
       << load_expr(rdt, "(" + stype(rdt) + ")(" + store_expr(rdt, "(" + ctype(rdt) + ")acc") + ")") << ";\n"
-      << cbody.str() << "  ((" << stype(odt) << "*)p_out)[o] = " << store_expr(odt, outv) << ";\n}\n";
+      << cbody.str() << "  return " << store_expr(odt, outv) << ";\n}\n";
   std::ostringstream src;
   src << pre.str() << "struct Src {\n" << fields;
   for (size_t k = 0; k < kept.size(); ++k) src << "  long long o" << k << ";\n";
@@ -2657,11 +2671,16 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
       << pbody.str() << "      v[e] = (acc_t)(" << val << ");\n      }\n  }\n};\n"
       << "struct Dst {\n" << fields << "  void* p_out;\n  acc_t* p_ws;\n"
       << "  __device__ __forceinline__ void put(long long o, acc_t a) const {\n    "
-      << (g.C > 1 ? "p_ws[blockIdx.y * geom.osize + o] = a;" : "finish(o, a, " + args_s + "p_out);") << "\n  }\n};\n"
+      << (g.C > 1 ? "p_ws[blockIdx.y * geom.osize + o] = a;"
+                  : "((" + stype(odt) + "*)p_out)[o] = finish(o, a, " + args_s.substr(0, args_s.size() - 2) + ");")
+      << "\n  }\n  __device__ __forceinline__ void put(long long o, const acc_t (&a)[" << Vs << "]) const {\n"
+      << "    struct __attribute__((packed)) W { " << stype(odt) << " x[" << Vs << "]; } w;\n#pragma unroll\n    for (int e = 0; e < " << Vs
+      << "; ++e) w.x[e] = finish(o + e, a[e], " << args_s.substr(0, args_s.size() - 2) << ");\n    *(W*)((" << stype(odt)
+      << "*)p_out + o) = w;\n  }\n};\n"
       << "extern \"C\" __global__ void __launch_bounds__(" << (1 << g.log_nt) << ") fused_reduce(" << params
       << "void* __restrict__ p_out, acc_t* __restrict__ p_ws) {\n  __shared__ acc_t part[ghip::reduce_lds(geom)];\n"
       << "  Src src{" << args_s << "};\n  const Dst dst{" << args_s << "p_out, p_ws};\n"
-      << "  ghip::reduce_body<" << g.form << ", " << Vs << ">(geom, (acc_t)" << init << ", Comb{}, src, dst, part);\n}\n";
+      << "  ghip::reduce_body<" << g.form << ", " << Vs << ", ghip::reduce_unroll(" << Vs << ")>(geom, (acc_t)" << init << ", Comb{}, src, dst, part);\n}\n";
   RtcKernel kern, fin;
   if (rtc_get(be, src.str(), "fused_reduce", &kern, err) != GHIP_OK) return bad();
   if (g.C > 1) {
@@ -2669,7 +2688,8 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
     fs << pre.str() << "extern \"C\" __global__ void __launch_bounds__(256) reduce_finish(" << params
        << "void* __restrict__ p_out, const acc_t* __restrict__ p_ws) {\n"
        << "  const long long o = (long long)blockIdx.x * 256 + threadIdx.x;\n"
-       << "  if (o < geom.osize) finish(o, ghip::reduce_ranges(geom, p_ws, o, Comb{}), " << args_s << "p_out);\n}\n";
+       << "  if (o < geom.osize) ((" << stype(odt) << "*)p_out)[o] = finish(o, ghip::reduce_ranges(geom, p_ws, o, Comb{}), "
+       << args_s.substr(0, args_s.size() - 2) << ");\n}\n";
     if (rtc_get(be, fs.str(), "reduce_finish", &fin, err) != GHIP_OK) return bad();
   }
   const Shape& os = N[out_v].shape;
@@ -2694,7 +2714,7 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
     for (size_t k = 0; k < ptrs.size(); ++k) args.push_back(&ptrs[k]);
     args.push_back(&outp);
     args.push_back(&wsp);
-    hipError_t h = hipModuleLaunchKernel(kern.func, static_cast<unsigned>(g.gx), static_cast<unsigned>(g.C), 1, 1u << g.log_nt, 1, 1, 0,
+    hipError_t h = hipModuleLaunchKernel(kern.func, reduce_grid_x(g), reduce_grid_y(g), 1, 1u << g.log_nt, 1, 1, 0,
                                          st.stream, args.data(), nullptr);
     if (h == hipSuccess && g.C > 1)
       h = hipModuleLaunchKernel(fin.func, static_cast<unsigned>((osize + 255) / 256), 1, 1, 256, 1, 1, 0, st.stream,

@@ -4,213 +4,41 @@
 // Bound by HBM; forms and accumulation order: reduce_dev.h, reduce_geometry.  us a call, a
 // kernel generated with the sizes as literals / here: bf16 [4096,2048] over the rows 7.7 /
 // 7.5, over the columns 5.4 / 5.6; fp32 [8192,8192] over the rows 41.0 / 44.5, over the
-// columns 39.3 / 39.3; many short rows pay for the arguments, [65536,64] over the columns 6.6 / 9.2, and axes
-// that do not fold for their divisions, [6,40,500] over 0 and 2 7.2 / 14.1.
+// columns 39.3 / 39.3; many short rows pay for the arguments, [65536,64] over the columns
+// 6.4 / 10.0 (17.5 a wave per output by the earlier kernel), and axes that do not fold for
+// their divisions, [6,40,500] over 0 and 2 7.2 / 15.9 (earlier 28).
 // Accumulator: fp32 for fp32 / bf16 / f16, fp64 for fp64, 64-bit integers for integers.
-#include <limits>
-
-#include "common.h"
-#include "graph.h"
-#include "reduce_dev.h"
+#include "reduce_kernels.h"
 
 namespace ghip {
-namespace {
-
-template <typename T> struct Acc { using type = float; };
-template <> struct Acc<double> { using type = double; };
-template <> struct Acc<int8_t> { using type = long long; };
-template <> struct Acc<int16_t> { using type = long long; };
-template <> struct Acc<int32_t> { using type = long long; };
-template <> struct Acc<int64_t> { using type = long long; };
-template <> struct Acc<uint8_t> { using type = unsigned long long; };
-template <> struct Acc<uint16_t> { using type = unsigned long long; };
-template <> struct Acc<uint32_t> { using type = unsigned long long; };
-template <> struct Acc<uint64_t> { using type = unsigned long long; };
-
-template <typename T> __device__ __forceinline__ typename Acc<T>::type widen(T x) { return x; }
-__device__ __forceinline__ float widen(bf16_t x) { return bf16_to_f32(x.bits); }
-template <typename T> __device__ __forceinline__ void narrow(T* p, typename Acc<T>::type v) { *p = static_cast<T>(v); }
-__device__ __forceinline__ void narrow(bf16_t* p, float v) { p->bits = f32_to_bf16(v); }
-
-template <int OP, typename A>
-__device__ __forceinline__ A init_of() {
-  if constexpr (OP == GHIP_REDUCE_SUM) return A(0);
-  else if constexpr (OP == GHIP_REDUCE_PRODUCT) return A(1);
-  else if constexpr (std::is_floating_point<A>::value) return OP == GHIP_REDUCE_MAX ? -A(INFINITY) : A(INFINITY);
-  else return OP == GHIP_REDUCE_MAX ? std::numeric_limits<A>::lowest() : std::numeric_limits<A>::max();
-}
-template <int OP>
-struct Combine {
-  template <typename A>
-  __device__ __forceinline__ A operator()(A a, A b) const {
-    if constexpr (OP == GHIP_REDUCE_SUM) return a + b;
-    else if constexpr (OP == GHIP_REDUCE_PRODUCT) return a * b;
-    else if constexpr (OP == GHIP_REDUCE_MAX) return (a > b || a != a) ? a : b;  // NaN propagates
-    else return (a < b || a != a) ? a : b;
-  }
-};
-
-// V consecutive values from p, UNIT: next to each other (one load at element alignment),
-// else `step` elements apart.
-template <typename T, int V, bool UNIT>
-__device__ __forceinline__ void load_values(const T* p, int64_t step, typename Acc<T>::type (&v)[V]) {
-  if constexpr (UNIT) {
-    struct __attribute__((packed)) W { T x[V]; };
-    const W w = *reinterpret_cast<const W*>(p);
-#pragma unroll
-    for (int e = 0; e < V; ++e) v[e] = widen(w.x[e]);
-  } else {
-#pragma unroll
-    for (int e = 0; e < V; ++e) v[e] = widen(p[e * step]);
-  }
-}
-
-// An operand of one reduced axis and one kept axis (columns: one before, one after it)
-// whose vectors lie together.
-template <typename T, int V>
-struct LineOperand {
-  const T* x;
-  int64_t s_out, s_in, s_red;
-  const T* row;
-  __device__ __forceinline__ void at(long long o) { row = x + o * s_out; }
-  __device__ __forceinline__ void at(long long ou, long long col) { row = x + ou * s_out + col * s_in; }
-  __device__ __forceinline__ void get(long long r, typename Acc<T>::type (&v)[V]) const {
-    load_values<T, V, true>(row + r * s_red, 1, v);
-  }
-};
-
-// Any axes.
-template <typename T, int V, bool UNIT>
-struct AxesOperand {
-  const T* x;
-  const ReduceAxes& d;
-  long long inner;
-  const T* row;
-  __device__ __forceinline__ static long long offset(long long i, bool wide, int rank, const ReduceDiv* div,
-                                                     const int64_t* dims, const int64_t* st) {
-    long long off = 0;
-#pragma unroll
-    for (int k = kMaxRank - 1; k > 0; --k)
-      if (k < rank) {
-        const long long q = wide ? i / dims[k] : reduce_quot(static_cast<unsigned>(i), div[k]);
-        off += (i - q * dims[k]) * st[k];
-        i = q;
-      }
-    return off + i * st[0];
-  }
-  __device__ __forceinline__ void at(long long o) { row = x + offset(o, d.o_wide, d.orank, d.odiv, d.odims, d.ost); }
-  __device__ __forceinline__ void at(long long ou, long long col) { at(ou * inner + col); }
-  __device__ __forceinline__ void get(long long r, typename Acc<T>::type (&v)[V]) const {
-    load_values<T, V, UNIT>(row + offset(r, d.r_wide, d.rrank, d.rdiv, d.rdims, d.rst), d.step, v);
-  }
-};
-template <typename T>
-struct Result {
-  T* y;
-  typename Acc<T>::type* ws;
-  const ReduceGeom& g;
-  __device__ __forceinline__ void put(long long o, typename Acc<T>::type a) const {
-    if (g.C > 1) ws[blockIdx.y * g.osize + o] = a;
-    else narrow(y + o, a);
-  }
-};
-
-template <typename T, int V, int FORM, int OP>
-__global__ __launch_bounds__(1024) void reduce_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t s_out,
-                                                      int64_t s_red, int64_t s_in, typename Acc<T>::type* __restrict__ ws,
-                                                      ReduceGeom g) {
-  using A = typename Acc<T>::type;
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  reduce_body<FORM, V>(g, init_of<OP, A>(), Combine<OP>{}, LineOperand<T, V>{x, s_out, s_in, s_red, x},
-                       Result<T>{y, ws, g}, reinterpret_cast<A*>(lds));
-}
-// Any axes: fewer calls, so the operation is an argument.
-template <typename T, int V, int FORM>
-__global__ __launch_bounds__(1024) void reduce_axes_kernel(const T* __restrict__ x, T* __restrict__ y,
-                                                           typename Acc<T>::type* __restrict__ ws, ReduceAxes d, ReduceGeom g,
-                                                           int op) {
-  using A = typename Acc<T>::type;
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  const A init = op == GHIP_REDUCE_SUM ? init_of<GHIP_REDUCE_SUM, A>() : op == GHIP_REDUCE_PRODUCT ? init_of<GHIP_REDUCE_PRODUCT, A>()
-               : op == GHIP_REDUCE_MAX ? init_of<GHIP_REDUCE_MAX, A>() : init_of<GHIP_REDUCE_MIN, A>();
-  auto comb = [op](A a, A b) {
-    switch (op) {
-      case GHIP_REDUCE_SUM: return Combine<GHIP_REDUCE_SUM>{}(a, b);
-      case GHIP_REDUCE_PRODUCT: return Combine<GHIP_REDUCE_PRODUCT>{}(a, b);
-      case GHIP_REDUCE_MAX: return Combine<GHIP_REDUCE_MAX>{}(a, b);
-      default: return Combine<GHIP_REDUCE_MIN>{}(a, b);
-    }
-  };
-  auto body = [&](auto unit) {
-    reduce_body<FORM, V>(g, init, comb, AxesOperand<T, V, decltype(unit)::value>{x, d, g.inner, x}, Result<T>{y, ws, g},
-                         reinterpret_cast<A*>(lds));
-  };
-  if constexpr (V == 1) body(std::true_type{});
-  else if (d.step == 1) body(std::true_type{});
-  else body(std::false_type{});
-}
-template <typename T, int OP>
-__global__ __launch_bounds__(256) void reduce_finish_kernel(T* __restrict__ y, const typename Acc<T>::type* __restrict__ ws,
-                                                            ReduceGeom g) {
-  const long long o = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-  if (o < g.osize) narrow(y + o, reduce_ranges(g, ws, o, Combine<OP>{}));
-}
-
-// go(form, V) with both as compile-time constants.
-template <typename T, typename F>
-void with_form(const ReduceGeom& g, F go) {
-  constexpr int VMAX = 16 / sizeof(T);
-  auto width = [&](auto form) {
-    if (g.V == 1) go(form, std::integral_constant<int, 1>{});
-    else if (g.V == 2) go(form, std::integral_constant<int, 2>{});
-    else if (g.V == 4) { if constexpr (VMAX >= 4) go(form, std::integral_constant<int, 4>{}); }
-    else if (g.V == 8) { if constexpr (VMAX >= 8) go(form, std::integral_constant<int, 8>{}); }
-    else if constexpr (VMAX >= 16) go(form, std::integral_constant<int, 16>{});
-  };
-  if (g.form == kReduceRows) width(std::integral_constant<int, kReduceRows>{});
-  else if (g.form == kReduceColumns) width(std::integral_constant<int, kReduceColumns>{});
-  else go(std::integral_constant<int, kReduceThreads>{}, std::integral_constant<int, 1>{});
-}
-
-// The kernels of a Reduce: over the operand, and over the ranges' values.
-template <typename T, int OP>
-void kernels_of(const ReduceAxes& d, const ReduceGeom& g, const void** main, const void** finish) {
-  with_form<T>(g, [&](auto form, auto v) {
-    constexpr int F = decltype(form)::value, V = decltype(v)::value;
-    *main = d.line ? reinterpret_cast<const void*>(&reduce_kernel<T, V, F, OP>)
-                   : reinterpret_cast<const void*>(&reduce_axes_kernel<T, V, F>);
-  });
-  *finish = reinterpret_cast<const void*>(&reduce_finish_kernel<T, OP>);
-}
-template <typename T>
-void kernels_of(int op, const ReduceAxes& d, const ReduceGeom& g, const void** main, const void** finish) {
-  switch (op) {
-    case GHIP_REDUCE_SUM: return kernels_of<T, GHIP_REDUCE_SUM>(d, g, main, finish);
-    case GHIP_REDUCE_PRODUCT: return kernels_of<T, GHIP_REDUCE_PRODUCT>(d, g, main, finish);
-    case GHIP_REDUCE_MAX: return kernels_of<T, GHIP_REDUCE_MAX>(d, g, main, finish);
-    default: return kernels_of<T, GHIP_REDUCE_MIN>(d, g, main, finish);
-  }
-}
-
-}  // namespace
+namespace reduce {
+extern template void kernels_of<int8_t>(int, const ReduceAxes&, const ReduceGeom&, const void**, const void**);
+extern template void kernels_of<int16_t>(int, const ReduceAxes&, const ReduceGeom&, const void**, const void**);
+extern template void kernels_of<int32_t>(int, const ReduceAxes&, const ReduceGeom&, const void**, const void**);
+extern template void kernels_of<int64_t>(int, const ReduceAxes&, const ReduceGeom&, const void**, const void**);
+extern template void kernels_of<uint8_t>(int, const ReduceAxes&, const ReduceGeom&, const void**, const void**);
+extern template void kernels_of<uint16_t>(int, const ReduceAxes&, const ReduceGeom&, const void**, const void**);
+extern template void kernels_of<uint32_t>(int, const ReduceAxes&, const ReduceGeom&, const void**, const void**);
+extern template void kernels_of<uint64_t>(int, const ReduceAxes&, const ReduceGeom&, const void**, const void**);
+}  // namespace reduce
 
 int reduce_kernels(int dtype, int op, const ReduceAxes& d, const ReduceGeom& g, bool plan_only, ReduceKernels* k,
                    GHipError* err) {
   const void* main = nullptr;
   const void* finish = nullptr;
   switch (dtype) {
-    case GHIP_DTYPE_FLOAT32: kernels_of<float>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_BFLOAT16: kernels_of<bf16_t>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_FLOAT16: kernels_of<_Float16>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_FLOAT64: kernels_of<double>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_INT8: kernels_of<int8_t>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_INT16: kernels_of<int16_t>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_INT32: kernels_of<int32_t>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_INT64: kernels_of<int64_t>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_UINT8: kernels_of<uint8_t>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_UINT16: kernels_of<uint16_t>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_UINT32: kernels_of<uint32_t>(op, d, g, &main, &finish); break;
-    case GHIP_DTYPE_UINT64: kernels_of<uint64_t>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_FLOAT32: reduce::kernels_of<float>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_BFLOAT16: reduce::kernels_of<bf16_t>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_FLOAT16: reduce::kernels_of<_Float16>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_FLOAT64: reduce::kernels_of<double>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_INT8: reduce::kernels_of<int8_t>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_INT16: reduce::kernels_of<int16_t>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_INT32: reduce::kernels_of<int32_t>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_INT64: reduce::kernels_of<int64_t>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_UINT8: reduce::kernels_of<uint8_t>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_UINT16: reduce::kernels_of<uint16_t>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_UINT32: reduce::kernels_of<uint32_t>(op, d, g, &main, &finish); break;
+    case GHIP_DTYPE_UINT64: reduce::kernels_of<uint64_t>(op, d, g, &main, &finish); break;
     default: return set_error(err, GHIP_ERR_UNSUPPORTED, "reduce: dtype %d", dtype);
   }
   if (plan_only) return GHIP_OK;
@@ -229,7 +57,7 @@ int launch_reduce(const ReduceKernels& k, int op, const void* x, void* y, void* 
   void* line_args[] = {&x, &y, &s_out, &s_red, &s_in, &ws, &geom};
   void* axes_args[] = {&x, &y, &ws, &axes, &geom, &op};
   const unsigned nt = 1u << g.log_nt, lds = static_cast<unsigned>(reduce_lds(g) * acc_bytes);
-  hipError_t h = hipModuleLaunchKernel(k.main, static_cast<unsigned>(g.gx), static_cast<unsigned>(g.C), 1, nt, 1, 1, lds, s,
+  hipError_t h = hipModuleLaunchKernel(k.main, reduce_grid_x(g), reduce_grid_y(g), 1, nt, 1, 1, lds, s,
                                        d.line ? line_args : axes_args, nullptr);
   if (h == hipSuccess && g.C > 1) {
     void* fin_args[] = {&y, &ws, &geom};

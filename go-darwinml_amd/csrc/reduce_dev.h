@@ -12,7 +12,7 @@ namespace ghip {
 //   columns: a workgroup takes L vectors of V adjacent columns and strides the reduced
 //            index with its other lanes, so every load is coalesced; a butterfly over
 //            the lanes of one column, then LDS.
-//   threads: a thread per output.
+//   threads: a thread per output, or per V adjacent outputs.
 enum ReduceForm { kReduceRows = 0, kReduceColumns = 1, kReduceThreads = 2 };
 
 // n / d for n < 2^31 by a multiply: q = (mulhi(n, mul) + n) >> shift.
@@ -39,20 +39,33 @@ struct ReduceGeom {
   int log_nt;              // threads per workgroup
   ReduceDiv cblocks;       // columns: workgroups side by side
 };
+// Workgroups in x: HIP takes fewer than 2^32 work-items per dimension, so a grid of more
+// workgroups goes on in y.
+constexpr long long kReduceGridX = 1 << 21;
+constexpr unsigned reduce_grid_x(const ReduceGeom& g) { return static_cast<unsigned>(g.gx < kReduceGridX ? g.gx : kReduceGridX); }
+constexpr unsigned reduce_grid_y(const ReduceGeom& g) {
+  return g.C > 1 ? static_cast<unsigned>(g.C) : static_cast<unsigned>((g.gx + kReduceGridX - 1) / kReduceGridX);
+}
 // Accumulators the combine step keeps in LDS.
 constexpr int reduce_lds(const ReduceGeom& g) {
   return g.form == kReduceRows ? 1 << g.log_l >> 6 : g.form == kReduceColumns ? (g.V << g.log_nt >> 6) << g.log_l : 1;
 }
 
 #if defined(__HIP__) || defined(__HIPCC_RTC__)
+// Loads in flight a lane: at least 64 bytes of 16-byte vectors, eight narrower ones.
+constexpr int reduce_unroll(int v) { return v <= 2 ? 8 : 4; }
+
 __device__ __forceinline__ unsigned reduce_quot(unsigned n, const ReduceDiv& d) { return (__umulhi(n, d.mul) + n) >> d.shift; }
 
 // src.at(o) / src.at(ou, col): the kept index (columns: before / after the reduced axes)
 // whose values src.get(r, v) then gives, V of them from reduced index r (rows) or column
-// col (columns).  dst.put(o, a): output o's value (of one range).
-template <int FORM, int V, class A, class Comb, class Src, class Dst>
+// col (columns).  dst.put(o, a): output o's value (of one range);
+// dst.put(o, acc): outputs o .. o + V - 1.
+template <int FORM, int V, int U, class A, class Comb, class Src, class Dst>
 __device__ __forceinline__ void reduce_body(const ReduceGeom& g, A init, Comb comb, Src src, Dst dst, A* part) {
   const int t = threadIdx.x;
+  const unsigned blk = g.gx <= kReduceGridX ? blockIdx.x : blockIdx.y * static_cast<unsigned>(kReduceGridX) + blockIdx.x;
+  if (blk >= g.gx) return;
   A acc[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) acc[e] = init;
@@ -61,9 +74,8 @@ __device__ __forceinline__ void reduce_body(const ReduceGeom& g, A init, Comb co
   // Every 2^log-th reduced index from r, U loads in flight (by hand: the trip count
   // differs between lanes, for which the compiler tests it after every load).
   auto sweep = [&](long long r, int log) {
-    constexpr int U = V <= 2 ? 8 : 4, LU = V <= 2 ? 3 : 2;
     long long n = r < r_end ? ((r_end - r - 1) >> log) + 1 : 0;
-    for (; n >= U; n -= U, r += 1ll << (log + LU)) {
+    for (; n >= U; n -= U, r += static_cast<long long>(U) << log) {
       A v[U][V];
 #pragma unroll
       for (int u = 0; u < U; ++u) src.get(r + (static_cast<long long>(u) << log), v[u]);
@@ -82,7 +94,7 @@ __device__ __forceinline__ void reduce_body(const ReduceGeom& g, A init, Comb co
   };
   if constexpr (FORM == kReduceRows) {
     const int lane = t & ((1 << g.log_l) - 1);
-    const long long o = (static_cast<long long>(blockIdx.x) << (g.log_nt - g.log_l)) +
+    const long long o = (static_cast<long long>(blk) << (g.log_nt - g.log_l)) +
                         __builtin_amdgcn_readfirstlane(t >> g.log_l);  // the same for a whole wave
     if (g.log_l == 6 && o >= g.osize) return;  // whole waves; wider groups are one output a workgroup
     src.at(o);
@@ -103,8 +115,8 @@ __device__ __forceinline__ void reduce_body(const ReduceGeom& g, A init, Comb co
     dst.put(o, a);
   } else if constexpr (FORM == kReduceColumns) {
     const int TX = 1 << g.log_l, tx = t & (TX - 1), ty = t >> g.log_l, W = V << g.log_l;
-    const unsigned ou = reduce_quot(blockIdx.x, g.cblocks);
-    const long long col0 = static_cast<long long>(blockIdx.x - ou * g.cblocks.d) * W;
+    const unsigned ou = reduce_quot(blk, g.cblocks);
+    const long long col0 = static_cast<long long>(blk - ou * g.cblocks.d) * W;
     const long long col = col0 + tx * V;
     src.at(ou, col < g.inner ? col : 0);
     sweep(start + ty, g.log_nt - g.log_l);
@@ -122,11 +134,11 @@ __device__ __forceinline__ void reduce_body(const ReduceGeom& g, A init, Comb co
       dst.put(ou * g.inner + col0 + c, a);
     }
   } else {
-    const long long o = (static_cast<long long>(blockIdx.x) << g.log_nt) + t;
+    const long long o = ((static_cast<long long>(blk) << g.log_nt) + t) * V;
     if (o >= g.osize) return;
     src.at(o);
     sweep(0, 0);
-    dst.put(o, acc[0]);
+    dst.put(o, acc);
   }
 }
 

@@ -22,6 +22,8 @@ CASES = [
     ((64, 8), [0]), ((2000, 64), [0]), ((7, 50, 24), [1]), ((3, 129, 9), [1]),    # columns
     ((4096, 2048), [0]), ((2, 70000, 8), [1]), ((513, 130), [0]), ((6, 5, 4, 40), [1, 2]),
     ((6, 40, 5), [0, 2]), ((70, 3), [0]), ((9, 7, 3), [1]),                       # general, wave and thread
+    ((8193, 2, 8), [1]), ((8200, 3, 24), [1]), ((70001, 5, 9), [1]), ((16384, 7, 20), [1]),  # threads, 1 to 4 wide
+    ((70000, 63, 8), [1]), ((33000, 2, 3, 64), [1, 2]),
     ((0, 8), [0]), ((8, 0), [1]),                                                 # nothing to reduce
 ]
 
@@ -75,6 +77,29 @@ def test_reduce_forms(be, shape, axes, dt, monkeypatch):
     monkeypatch.setenv("GHIP_REDUCE_FUSION", "0")
     plain, _ = _run(be, shape, axes, dt, "ReduceSum", feed, True)
     assert "producer fused" in plan and np.array_equal(fused, plain, equal_nan=True)
+
+
+def test_grid_beyond_x(be):
+    """More workgroups than a grid takes in x: they go on in y (int8; rows and columns,
+    fused with their operand)."""
+    for dims, axis in [((1 << 24, 64), 1), ((1 << 22, 64, 8), 1)]:
+        b = be.Builder("grid")
+        f = b.Main()
+        S = make_shape(dtypes.Int8, *dims)
+        r = f.Parameter("r", make_shape(dtypes.Int8, *dims[1:]))
+        i = f.ConvertDType(f.Rem(f.Iota(make_shape(dtypes.Int32, *dims), 0), f.Constant(np.int32(101))), dtypes.Int8)
+        f.Return([f.ReduceMax(f.Add(i, f.BroadcastInDim(r, S, list(range(1, len(dims))))), axis), f.ReduceMax(i, axis)])
+        ex = b.Compile()
+        print(dims, ex.Plan(), flush=True)
+        row = (np.arange(np.prod(dims[1:])) % 13).astype(np.int8).reshape(dims[1:])
+        got = ex.Execute([be.BufferFromFlatData(0, row, make_shape(dtypes.Int8, *dims[1:]))])
+        base = (np.arange(dims[0]) % 101).astype(np.int8)
+        tail = row.max(0)
+        want = [base[:, None] + tail.reshape(1, -1), np.broadcast_to(base[:, None], (dims[0], tail.size))]
+        for y, w in zip(got, want):
+            assert np.array_equal(be.BufferToFlatData(y).reshape(dims[0], -1), w)
+            be.BufferFinalize(y)
+        ex.Finalize()
 
 
 def test_split_reduce_says_so(be):

@@ -612,3 +612,19 @@ def test_plain_reduces_compile_no_kernel(be, monkeypatch, tmp_path):
         p = plan_of(be, build)
         assert p.count("reduce_") == 5 and "fused" not in p, p
     assert not list(tmp_path.iterdir())
+
+
+def test_reduce_launch_shapes(be):
+    """Reduces of many short ranges take a thread per output vector, not a workgroup per
+    outer index, and no grid reaches 2^32 work-items in x (HIP's limit)."""
+    def step(dt, dims, axis):
+        p = plan_of(be, lambda f: [f.ReduceMax(f.Parameter("x", make_shape(dt, *dims)), axis)])
+        form, _, _, _, x, _, y, _, nt = p[p.index(" [", p.index("->") + 20) + 2:].split("]")[0].replace(",", "").split()
+        assert int(x) * int(nt) < 2 ** 32 and int(y) < 65536, p
+        return form, int(x) * int(y) * int(nt)
+    assert step(dtypes.Int8, (1 << 24, 2, 8), 1) == ("threads", 1 << 24)
+    assert step(BF16, (65536, 8, 64), 1) == ("threads", 65536 * 64 // 8)
+    assert step(F32, (1 << 20, 2, 8), 1) == ("threads", (1 << 20) * 8 // 4)
+    assert step(F32, (8192, 20, 64), 1)[0] == "columns"
+    assert step(F32, (1 << 28, 64), 1) == ("rows", (1 << 28) * 64)      # beyond x: goes on in y
+    assert step(dtypes.Int8, (1 << 25, 64, 8), 1) == ("columns", (1 << 25) * 256)
