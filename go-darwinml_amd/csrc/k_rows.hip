@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "rows_dispatch.h"
 
 namespace ghip {
 
@@ -854,9 +855,10 @@ static hipError_t launch_rows(const RowParams& p, hipStream_t s) {
   }
   // Rows of any width and alignment, and wide softmax rows (sixteen waves a row), held
   // whole in registers too (x read from HBM once).  vecs: blocks of 16 bytes the row may
-  // touch.  Norms stop at four vectors a lane: wider ones are not met.
+  // touch.  Norms stop at four vectors a lane; rows beyond that (16K fp32, 32K 16-bit
+  // elements) take the several-pass kernel below.
   if constexpr (OP != kMaskedSoftmax) {
-    const int64_t vecs = (p.n + 2 * VEC - 2) / VEC;
+    const int64_t vecs = row_blocks(p.n, VEC, static_cast<int>(reinterpret_cast<uintptr_t>(p.x) / sizeof(T) % VEC));
     auto go = [&](auto nv, auto wpr) { return launch_reg<T, OP, decltype(nv)::value, decltype(wpr)::value, true>(p, s); };
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;

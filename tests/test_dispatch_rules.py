@@ -1,0 +1,23 @@
+"""Host rules of the kernels' dispatch, compiled on the CPU: static_asserts over the
+headers that hold them."""
+import os
+import subprocess
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "go-darwinml_amd", "csrc")
+
+
+def _check(tmp_path, header, asserts):
+    src = tmp_path / "rules.cpp"
+    src.write_text(f'#include "{header}"\nusing namespace ghip;\n' +
+                   "".join(f'static_assert({a}, "");\n' for a in asserts))
+    r = subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-I", CSRC, str(src)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+
+
+def test_row_blocks(tmp_path):
+    """Blocks of 16 bytes a row touches: 1024 threads hold 16 of them each in fp32 (8 in 16
+    bits), so an aligned row of 65536 elements fits, and no row that touches more."""
+    _check(tmp_path, "rows_dispatch.h", [
+        "row_blocks(65536, 4, 0) == 16384", "row_blocks(65536, 8, 0) == 8192",
+        "row_blocks(65536, 4, 3) == 16385", "row_blocks(65533, 4, 0) == 16384", "row_blocks(65534, 4, 0) == 16385",
+        "row_blocks(1, 4, 3) == 1", "row_blocks(2, 4, 3) == 2", "row_blocks(4, 4, 1) == 2", "row_blocks(9, 8, 0) == 2"])
