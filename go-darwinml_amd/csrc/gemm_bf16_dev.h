@@ -105,6 +105,9 @@ __host__ __device__ inline int gemm_fast_ktiles(bool k_contig, int64_t MN, int64
 }
 
 #if !defined(__HIPCC_RTC__)
+}  // namespace ghip
+#include "gemm_rules.h"
+namespace ghip {
 // Contraction split for products whose grid leaves most of the chip idle.  s
 // ranges of kc = K / s contraction steps (kc a multiple of 64) run as s slices of
 // one grid, each writing its fp32 partial product; a second kernel sums the s
@@ -152,16 +155,6 @@ inline GemmSplit gemm_k_split(int64_t batch, int64_t M, int64_t N, int64_t K, in
   }
   return r;
 }
-// Grids of at most this many 128 x 128 tiles run 64 x 64 tiles of the register-staged
-// core instead (any layout): four times the workgroups, each with four k-tiles of
-// loads in flight.  Graph-replayed, us, 128 x 128 DMA core / 64 x 64: bf16 [256,512,256]
-// 5.8 / 4.3, [512,512,512] 8.0 / 5.4, [1024,1024,1024] 12.6 / 8.1, [1024,2048,1024] (128
-// tiles) 12.8 / 11.3, but 14.2 / 14.8 at 144 tiles and 14.6 / 18.8 at 256; fp32, bound
-// by a CU's MFMA rate, [256,512,256] 20.9 / 8.2, [1024,1024,256] 21.8 / 9.4,
-// [1536,2048,512] (192 tiles) 40.2 / 32.4, 270 / 277 at 224 tiles.
-inline bool gemm_small_tiles(int64_t batch, int64_t M, int64_t N, int es) {
-  return batch * ((M + 127) / 128) * ((N + 127) / 128) <= (es == 4 ? 192 : 128);
-}
 // 16-bit products for 256 x 128 tiles (gemm_bf16_body4h): grids that are one round of
 // them but more than one 128 x 128 tile per CU, with a contraction long enough to pay for
 // a prologue and an epilogue that no second workgroup hides.  Graph-replayed, us, 128 x
@@ -176,12 +169,6 @@ inline bool gemm_half_tiles(int64_t batch, int64_t M, int64_t N, int64_t K, bool
   const int64_t t128 = batch * ((M + 127) / 128) * ((N + 127) / 128);
   const int64_t half = batch * ((M + 255) / 256) * ((N + 127) / 128);
   return M >= 256 && t128 > 256 && half <= 256 && (gemm_half_whole(M, N, K) ? K >= 2048 : a_k && K >= 4096);
-}
-// fp32 grids of at most 128 tiles of 64 x 64: 32 x 32 tiles with the contraction spread
-// over a workgroup's waves.  us, 64 x 64 / 32 x 32: [256,512,256] 8.1 / 4.9, [256,256,512]
-// 13.0 / 6.5, [512,1024,1024] (128 tiles) 23.7 / 16.7, but 24.7 / 27.0 at 256.
-inline bool gemm_f32_tiny(int64_t batch, int64_t M, int64_t N) {
-  return batch * ((M + 63) / 64) * ((N + 63) / 64) <= 128;
 }
 // Whether a product that gemm_k_split would split runs as its split: not where small
 // tiles, unsplit, are modelled at less than 0.8 of the split's cost.  Their cost: one

@@ -3201,6 +3201,8 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
     mb = rs_majorness(d.sbn, d.sbk, d.N, d.K);
   }
   if (ma < 0 || mb < 0) return View{};
+  const int rs_tile = rs ? gemm_staged_tile(d.B, d.M, d.N, d.K, 2) : 0;
+  if (rs_tile == 16) return View{};  // the stand-alone product runs the 16 x 16 kernel
   const int64_t ea = ((d.M - 1) * d.sam + (d.K - 1) * d.sak + 1) * 2;
   const int64_t eb = ((d.N - 1) * d.sbn + (d.K - 1) * d.sbk + 1) * 2;
   if (!gemm_rows_fit(d.sam, d.sak, 2) || !gemm_rows_fit(d.sbn, d.sbk, 2)) return View{};
@@ -3315,7 +3317,7 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   bool eight_km = false, eight_x = false, four_km = false, half = false;
   const int64_t t4 = d.B * ((d.M + 255) / 256) * ((d.N + 256 / NB - 1) / (256 / NB));
   if (rs) {
-    if (gemm_small_tiles(d.B, d.M, d.N, 2)) BM = BN = 64;
+    BM = BN = rs_tile;
   } else if (ma && !mb && d.M >= 256 && d.N >= 256 / NB && (NB == 2 || !heavy_epilogue || ab_dt == GHIP_DTYPE_FLOAT16) &&
              (NB == 2 ? t4 >= 128 : t4 > 128)) {
     BM = 256, BN = 256 / NB, WM = 2, WN = 2, four_km = true;

@@ -159,10 +159,11 @@ static int64_t slice_bytes(int64_t rows, int64_t s_row, int64_t K, int64_t s_k, 
 
 template <typename InT, typename OutT>
 static hipError_t launch_rs(const GemmParams& p, hipStream_t s) {
+  const int t = gemm_staged_tile(p.batch, p.M, p.N, p.K, sizeof(InT));
+  if (t == 16) return launch_generic<InT, OutT>(p, s);
   if constexpr (sizeof(InT) == 4)
-    if (gemm_f32_tiny(p.batch, p.M, p.N)) return launch_rs_tile<32, InT, OutT>(p, s);
-  return gemm_small_tiles(p.batch, p.M, p.N, sizeof(InT)) ? launch_rs_tile<64, InT, OutT>(p, s)
-                                                          : launch_rs_tile<128, InT, OutT>(p, s);
+    if (t == 32) return launch_rs_tile<32, InT, OutT>(p, s);
+  return t == 64 ? launch_rs_tile<64, InT, OutT>(p, s) : launch_rs_tile<128, InT, OutT>(p, s);
 }
 
 // Workspace of a split contraction (16-byte aligned, large enough: checked by the

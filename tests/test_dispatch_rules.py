@@ -21,3 +21,14 @@ def test_row_blocks(tmp_path):
         "row_blocks(65536, 4, 0) == 16384", "row_blocks(65536, 8, 0) == 8192",
         "row_blocks(65536, 4, 3) == 16385", "row_blocks(65533, 4, 0) == 16384", "row_blocks(65534, 4, 0) == 16385",
         "row_blocks(1, 4, 3) == 1", "row_blocks(2, 4, 3) == 2", "row_blocks(4, 4, 1) == 2", "row_blocks(9, 8, 0) == 2"])
+
+
+def test_staged_tiles(tmp_path):
+    """Batches of small ragged products take tiles of their size, not 128 x 128 ones."""
+    _check(tmp_path, "gemm_rules.h", [
+        "gemm_staged_tile(512, 33, 33, 33, 2) == 64", "gemm_staged_tile(512, 63, 63, 1001, 2) == 64",
+        "gemm_staged_tile(4096, 5, 5, 7, 2) == 16", "gemm_staged_tile(65536, 5, 5, 7, 2) == 64",
+        "gemm_staged_tile(4096, 17, 17, 1001, 4) == 32", "gemm_staged_tile(4096, 33, 33, 65, 4) == 64",
+        "gemm_staged_tile(512, 100, 100, 65, 2) == 128", "gemm_staged_tile(1, 1999, 1999, 1001, 2) == 128",
+        "gemm_staged_tile(1, 1000, 776, 1531, 2) == 64", "gemm_staged_tile(1, 256, 10, 512, 4) == 32",
+        "gemm_staged_tile(200, 5, 5, 300, 2) == 64"])

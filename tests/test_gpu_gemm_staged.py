@@ -22,7 +22,8 @@ BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
 # or less (32 and 64 deep), fewer columns than a 16-byte chunk, a contraction of one
 # chunk, several edge tiles; and a grid of 128 x 128 tiles.
 SHAPES = [(1, 1, 1, 1), (1, 63, 65, 31), (2, 65, 63, 33), (1, 64, 10, 512), (1, 256, 512, 10), (1, 10, 3, 257),
-          (3, 1, 129, 63), (1, 129, 1, 65), (1, 100, 7, 129), (1, 31, 33, 1531), (1, 2049, 2055, 67)]
+          (3, 1, 129, 63), (1, 129, 1, 65), (1, 100, 7, 129), (1, 31, 33, 1531), (1, 2049, 2055, 67),
+          (700, 5, 7, 9), (700, 33, 31, 33), (300, 17, 19, 65), (150, 101, 67, 65)]  # tiles by M, N and the batch
 
 
 def _operand(r, c, off, trans, dt, seed, cuda):
