@@ -148,6 +148,18 @@ static bool reshape_strides(const std::vector<int64_t>& od, const std::vector<in
   return true;
 }
 
+// Compile-time image of the run-time checks ghip_gemm_batched makes before it takes the
+// LDS-DMA MFMA path: vec elements are 16 bytes (slot bases are 256-byte aligned, so a
+// view's base is 16-byte aligned iff its element offset is a multiple of vec).
+static int mfma_majorness(int64_t offset, int64_t s_b, int64_t s_mn, int64_t s_k, int64_t MN, int64_t K,
+                          int64_t batch, int vec = 8) {
+  if (offset % vec != 0) return -1;
+  const bool b_ok = batch == 1 || s_b % vec == 0;
+  if (s_k == 1 && K % vec == 0 && (MN == 1 || s_mn % vec == 0) && b_ok) return 1;
+  if (s_mn == 1 && MN % vec == 0 && (K == 1 || s_k % vec == 0) && b_ok) return 0;
+  return -1;
+}
+
 struct Lowerer {
   GHipBackend* be;
   GHipFunction* fn;
@@ -1843,7 +1855,8 @@ struct Lowerer {
     const int64_t M = d.M, N_ = d.N, K = d.K, sam = d.sam, sak = d.sak, sbk = d.sbk, sbn = d.sbn;
     // Products that split their contraction run one after another, sharing one
     // workspace in the arena.
-    const int64_t ws_bytes = split_ws_bytes(dt, odt, 1, M, N_, K);
+    int64_t ws_bytes = split_ws_bytes(dt, d);
+    for (auto& pl : plans) ws_bytes = std::min(ws_bytes, split_ws_bytes(dt, pl));
     const View wsv = gemm_workspace_view(ws_bytes, &wr);
     add_step(fmt("gemm_grouped %s G=%d M=%lld N=%lld K=%lld (products sharing a; a strides m=%lld k=%lld, b strides "
                  "k=%lld n=%lld%s)",
@@ -1883,7 +1896,7 @@ struct Lowerer {
     const int dt = N[n.in[0]].shape.dtype, odt = n.shape.dtype;
     const int64_t scb = M * N_, scm = N_;
     std::vector<int> wr{y.slot};
-    const int64_t ws_bytes = split_ws_bytes(dt, odt, B, M, N_, K);
+    const int64_t ws_bytes = split_ws_bytes(dt, d);
     const View wsv = gemm_workspace_view(ws_bytes, &wr);
     add_step(fmt("gemm_batched %s B=%lld M=%lld N=%lld K=%lld (%s; a strides b=%lld m=%lld k=%lld, b strides b=%lld k=%lld n=%lld%s)",
                  dtype_name(dt), (long long)B, (long long)M, (long long)N_, (long long)K, d.how.c_str(), (long long)sab,
@@ -1908,10 +1921,22 @@ struct Lowerer {
     wr->push_back(w.slot);
     return w;
   }
-  // Workspace bytes of a GEMM step (0 unless it runs as its contraction split).
-  static int64_t split_ws_bytes(int dt, int odt, int64_t B, int64_t M, int64_t N_, int64_t K) {
-    return gemm_uses_split(B, M, N_, K, dt == GHIP_DTYPE_FLOAT32 ? 4 : 2)
-               ? ghip_gemm_workspace_bytes(dt, odt, B, M, N_, K) : 0;
+  // Workspace bytes of a GEMM step: 0 unless it runs as its contraction split, which only
+  // operands that the LDS DMA can address do (the image of the run-time checks).
+  static int64_t split_ws_bytes(int dt, const DotPlan& d) {
+    const int64_t es = dt == GHIP_DTYPE_FLOAT32 ? 4 : 2;
+    if ((dt != GHIP_DTYPE_FLOAT32 && dt != GHIP_DTYPE_BFLOAT16 && dt != GHIP_DTYPE_FLOAT16) ||
+        !gemm_uses_split(d.B, d.M, d.N, d.K, static_cast<int>(es)))
+      return 0;
+    if (d.sam < 0 || d.sak < 0 || d.sbk < 0 || d.sbn < 0) return 0;
+    const int vec = static_cast<int>(16 / es);
+    if (mfma_majorness(d.lv.offset, d.sab, d.sam, d.sak, d.M, d.K, d.B, vec) < 0 ||
+        mfma_majorness(d.rv.offset, d.sbb, d.sbn, d.sbk, d.N, d.K, d.B, vec) < 0)
+      return 0;
+    if (!gemm_rows_fit(d.sam, d.sak, es) || !gemm_rows_fit(d.sbn, d.sbk, es)) return 0;
+    const int64_t ea = ((d.M - 1) * d.sam + (d.K - 1) * d.sak + 1) * es, eb = ((d.N - 1) * d.sbn + (d.K - 1) * d.sbk + 1) * es;
+    if (ea >= (int64_t{1} << 31) || eb >= (int64_t{1} << 31)) return 0;
+    return ghip_gemm_workspace_bytes(dt, dt, d.B, d.M, d.N, d.K);
   }
   static std::string split_note(int64_t ws_bytes, int64_t B, int64_t M, int64_t N_, int64_t K, int dt) {
     if (ws_bytes <= 0) return "";
@@ -3078,18 +3103,6 @@ View Lowerer::emit_cluster(int root, int v) {
   return ys[0];
 }
 
-// Compile-time image of the run-time checks ghip_gemm_batched makes before it
-// takes the bf16 MFMA path (slot bases are 256-byte aligned, so a view's base is
-// 16-byte aligned iff its element offset is a multiple of 8).
-static int mfma_majorness(int64_t offset, int64_t s_b, int64_t s_mn, int64_t s_k, int64_t MN, int64_t K,
-                          int64_t batch) {
-  if (offset % 8 != 0) return -1;
-  const bool b_ok = batch == 1 || s_b % 8 == 0;
-  if (s_k == 1 && K % 8 == 0 && (MN == 1 || s_mn % 8 == 0) && b_ok) return 1;
-  if (s_mn == 1 && MN % 8 == 0 && (K == 1 || s_k % 8 == 0) && b_ok) return 0;
-  return -1;
-}
-
 // A DotGeneral o that only the elementwise cluster being emitted reads (its
 // members: inset), with 16-bit operands on the MFMA path, batch 1, o's shape the
 // cluster's, and a contraction that splits: emits the GEMM step that writes o's
@@ -3109,15 +3122,8 @@ bool Lowerer::emit_split_partials(int o, const Shape& os, const std::set<int>& i
   DotPlan d;
   if (!plan_dot(o, false, &d)) return false;
   if (d.B != 1 || d.M <= 0 || d.N <= 0 || d.K <= 0) return false;
-  const int64_t wsb = ghip_gemm_workspace_bytes(dt, odt, 1, d.M, d.N, d.K);
-  if (wsb <= 0 || !gemm_uses_split(1, d.M, d.N, d.K, 2) || d.sam < 0 || d.sak < 0 || d.sbk < 0 || d.sbn < 0) return false;
-  if (mfma_majorness(d.lv.offset, 0, d.sam, d.sak, d.M, d.K, 1) < 0 ||
-      mfma_majorness(d.rv.offset, 0, d.sbn, d.sbk, d.N, d.K, 1) < 0)
-    return false;
-  if (!gemm_rows_fit(d.sam, d.sak, 2) || !gemm_rows_fit(d.sbn, d.sbk, 2)) return false;
-  const int64_t ea = ((d.M - 1) * d.sam + (d.K - 1) * d.sak + 1) * 2;
-  const int64_t eb = ((d.N - 1) * d.sbn + (d.K - 1) * d.sbk + 1) * 2;
-  if (ea >= (int64_t{1} << 31) || eb >= (int64_t{1} << 31)) return false;
+  const int64_t wsb = split_ws_bytes(dt, d);
+  if (wsb <= 0) return false;
   const int S = gemm_k_split(1, d.M, d.N, d.K, 2).s;
   Shape wss;
   wss.dtype = GHIP_DTYPE_FLOAT32;
@@ -3184,7 +3190,7 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
   // A product the stand-alone GEMM step would run with its contraction split stays
   // unfused (the split's fp32 partials are summed by a kernel of their own, which
   // the generated epilogue kernel does not reproduce).
-  if (gemm_uses_split(d.B, d.M, d.N, d.K, 2)) return View{};
+  if (split_ws_bytes(N[N[dots[0]].in[0]].shape.dtype, d) > 0) return View{};
   // The 16-bit MFMA path's operand conditions, decided here because the fused
   // kernel has no generic fallback.
   if (d.B > 65535 || d.M == 0 || d.N == 0 || d.K == 0) return View{};

@@ -83,7 +83,7 @@ def test_values_past_the_edges_do_not_leak(cuda):
 
 
 @pytest.mark.parametrize("M,N,K", [(1000, 776, 1531), (65, 10, 33), (7, 129, 64), (256, 512, 256), (300, 2049, 40),
-                                   (2049, 2051, 65)])
+                                   (2049, 2051, 65), (16, 4097, 4096), (100, 1001, 4096)])
 @pytest.mark.parametrize("act", [ActivationType.NONE, ActivationType.GELU])
 def test_staged_epilogue_equals_unfused(cuda, M, N, K, act):
     x = synth.to_bf16_bits(synth.normal(7301, (M, K)))

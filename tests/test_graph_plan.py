@@ -628,3 +628,22 @@ def test_reduce_launch_shapes(be):
     assert step(F32, (8192, 20, 64), 1)[0] == "columns"
     assert step(F32, (1 << 28, 64), 1) == ("rows", (1 << 28) * 64)      # beyond x: goes on in y
     assert step(dtypes.Int8, (1 << 25, 64, 8), 1) == ("columns", (1 << 25) * 256)
+
+
+@pytest.mark.parametrize("dt", [BF16, dtypes.Float16])
+@pytest.mark.parametrize("M,K,N", [(16, 4096, 4097), (100, 4096, 1001), (256, 2048, 1003)])
+def test_split_needs_operands_the_dma_can_address(be, dt, M, K, N):
+    """A long contraction of few tiles whose operand rows are not whole 16-byte chunks never
+    runs as a split: no workspace, no note of one, and the staged core carries its epilogue;
+    the same sizes with aligned rows still split."""
+    def dense(n):
+        def build(f):
+            x, w, b = (f.Parameter(k, make_shape(dt, *s)) for k, s in (("x", (M, K)), ("w", (K, n)), ("b", (n,))))
+            return [f.Tanh(f.Add(f.DotGeneral(x, [1], [], w, [0], []), f.BroadcastInDim(b, make_shape(dt, M, n), [1])))]
+        return plan_of(be, build)
+    p = dense(N)
+    assert "core=staged" in p and "split" not in p and "arena 0 bytes" in p, p
+    assert "contraction split" in dense((N + 15) // 16 * 16)
+    f32 = plan_of(be, lambda f: [f.DotGeneral(f.Parameter("x", make_shape(F32, M, K)), [1], [],
+                                              f.Parameter("w", make_shape(F32, K, N)), [0], [])])
+    assert "split" not in f32 and "arena 0 bytes" in f32, f32
