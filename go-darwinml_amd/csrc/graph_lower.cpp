@@ -2705,7 +2705,7 @@ View Lowerer::emit_reduce_fused(int R, int prod_root, int cons_root) {
       << "extern \"C\" __global__ void __launch_bounds__(" << (1 << g.log_nt) << ") fused_reduce(" << params
       << "void* __restrict__ p_out, acc_t* __restrict__ p_ws) {\n  __shared__ acc_t part[ghip::reduce_lds(geom)];\n"
       << "  Src src{" << args_s << "};\n  const Dst dst{" << args_s << "p_out, p_ws};\n"
-      << "  ghip::reduce_body<" << g.form << ", " << Vs << ", ghip::reduce_unroll(" << Vs << ")>(geom, (acc_t)" << init << ", Comb{}, src, dst, part);\n}\n";
+      << "  ghip::reduce_body<" << g.form << ", " << Vs << ", ghip::reduce_unroll(geom)>(geom, (acc_t)" << init << ", Comb{}, src, dst, part);\n}\n";
   RtcKernel kern, fin;
   if (rtc_get(be, src.str(), "fused_reduce", &kern, err) != GHIP_OK) return bad();
   if (g.C > 1) {

@@ -2,11 +2,11 @@
 // Precompiled over dtype, vector width and form, with sizes and strides as arguments, so
 // compiling a graph costs nothing for them (a kernel generated per shape: ~0.25 s each).
 // Bound by HBM; forms and accumulation order: reduce_dev.h, reduce_geometry.  us a call, a
-// kernel generated with the sizes as literals / here: bf16 [4096,2048] over the rows 7.7 /
-// 7.5, over the columns 5.4 / 5.6; fp32 [8192,8192] over the rows 41.0 / 44.5, over the
-// columns 39.3 / 39.3; many short rows pay for the arguments, [65536,64] over the columns
-// 6.4 / 10.0 (17.5 a wave per output by the earlier kernel), and axes that do not fold for
-// their divisions, [6,40,500] over 0 and 2 7.2 / 15.9 (earlier 28).
+// kernel generated with the sizes as literals / here: bf16 [4096,2048] over the rows 8.0 /
+// 7.9, over the columns 5.5 / 5.7; fp32 [8192,8192] over the rows 40.6 / 43.0, over the
+// columns 39.1 / 39.3; many short rows pay for the arguments, [65536,64] over the columns
+// 6.6 / 9.9 (17.5 a wave per output by the earlier kernel), and axes that do not fold for
+// their divisions, [6,40,500] over 0 and 2 7.2 / 15.8 (earlier 28).
 // Accumulator: fp32 for fp32 / bf16 / f16, fp64 for fp64, 64-bit integers for integers.
 #include "reduce_kernels.h"
 

@@ -52,8 +52,15 @@ constexpr int reduce_lds(const ReduceGeom& g) {
 }
 
 #if defined(__HIP__) || defined(__HIPCC_RTC__)
-// Loads in flight a lane: at least 64 bytes of 16-byte vectors, eight narrower ones.
+// Loads in flight a lane: eight, of wide vectors four.  Kernels generated for one geometry
+// take its own number of loads where that is less.
 constexpr int reduce_unroll(int v) { return v <= 2 ? 8 : 4; }
+constexpr int reduce_unroll(const ReduceGeom& g) {
+  const long long lanes = g.form == kReduceRows ? static_cast<long long>(g.V) << g.log_l
+                        : g.form == kReduceColumns ? 1ll << (g.log_nt - g.log_l) : 1;
+  const long long n = (g.chunk + lanes - 1) / lanes;
+  return n < 1 ? 1 : n < reduce_unroll(g.V) ? static_cast<int>(n) : reduce_unroll(g.V);
+}
 
 __device__ __forceinline__ unsigned reduce_quot(unsigned n, const ReduceDiv& d) { return (__umulhi(n, d.mul) + n) >> d.shift; }
 
@@ -84,8 +91,25 @@ __device__ __forceinline__ void reduce_body(const ReduceGeom& g, A init, Comb co
 #pragma unroll
         for (int e = 0; e < V; ++e) acc[e] = comb(acc[e], v[u][e]);
     }
-#pragma unroll 1
-    for (; n > 0; --n, r += 1ll << log) {
+    constexpr int H = U > 3 ? U / 2 : 1;
+    for (; n >= H; n -= H, r += static_cast<long long>(H) << log) {
+      A v[H][V];
+#pragma unroll
+      for (int u = 0; u < H; ++u) src.get(r + (static_cast<long long>(u) << log), v[u]);
+#pragma unroll
+      for (int u = 0; u < H; ++u)
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc[e] = comb(acc[e], v[u][e]);
+    }
+    if (n > 1) {  // the rest in flight together, the first one again past the end
+      A v[H][V];
+#pragma unroll
+      for (int u = 0; u < H; ++u) src.get(r + (u < n ? static_cast<long long>(u) << log : 0), v[u]);
+#pragma unroll
+      for (int u = 0; u < H; ++u)
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc[e] = u < n ? comb(acc[e], v[u][e]) : acc[e];
+    } else if (n == 1) {
       A v[V];
       src.get(r, v);
 #pragma unroll

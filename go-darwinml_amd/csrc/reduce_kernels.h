@@ -122,6 +122,9 @@ __global__ __launch_bounds__(1024) void reduce_kernel(const T* __restrict__ x, T
                                                       ReduceGeom g) {
   using A = typename Acc<T>::type;
   extern __shared__ __attribute__((aligned(16))) char lds[];
+  // The arguments at once: fetched where they are first used they are a chain of waits.
+  asm volatile("" ::"s"(g.osize), "s"(g.rsize), "s"(g.inner), "s"(g.gx), "s"(g.chunk), "s"(g.C), "s"(g.log_l), "s"(g.log_nt),
+               "s"(g.cblocks.d), "s"(g.cblocks.mul), "s"(g.cblocks.shift), "s"(s_in));
   reduce_body<FORM, V, reduce_unroll(V)>(g, init_of<OP, A>(), Combine<OP>{}, LineOperand<T, V>{x, s_out, s_in, s_red, x},
                        Result<T>{y, ws, g}, reinterpret_cast<A*>(lds));
 }
