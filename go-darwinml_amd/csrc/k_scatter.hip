@@ -196,11 +196,17 @@ __global__ void __launch_bounds__(256) scatter_rows_kernel(const U* __restrict__
   for (; c < d.D; c += LPR) combine<A>(o + c, widen<U, A>(u[c]), mode);
 }
 
-// Wider rows: a wave takes 64 rows x 64 columns, stages them in LDS (each lane its own
-// column, so no barrier) and combines the rows of one index before its one atomic per
-// column.  Token frequencies fall as 1 / rank, so without that the atomics on the first
-// table rows serialise (~40 ns each on one address) and bound the launch: fp32
-// [32000,256] += [256,50,256] rows at such ids 34 us with an atomic per row (an element a thread: 33), 16 here.
+// Wider rows: a wave takes R = 64 rows (32 with 64-bit accumulators) x 64 columns, stages
+// them in LDS (each lane its own column, so no barrier) and combines the rows of one index
+// before its one atomic per column.  Token frequencies fall as 1 / rank, so without that
+// the atomics on the first table rows serialise (~40 ns each on one address) and bound the
+// launch; indices without repeats pay for the wave's serial chain over its rows instead.
+// CW of a workgroup's waves lie side by side over the columns, the others take further
+// rows.  us with the table's copy, a wave per row / here, ids at such frequencies and
+// uniform ones: fp32 131072 rows of 32 215 / 61, 24.7 / 20.4; of 256 341 / 132, 111 / 122;
+// 32768 rows of 32 57.7 / 19.7, 9.6 / 16.2; fp64 32768 rows of 64 68.6 / 34.0, 16.7 / 19.5.
+// Up to 4096 rows the wave per row: fp64 of 64, 4096 rows 12.7 / 11.4, 8.8 / 11.8, 512 rows
+// 8.8 / 11.5, 8.8 / 11.2.
 template <typename A>
 __device__ __forceinline__ A combine_local(A a, A b, int mode) {
   if (mode == GHIP_SCATTER_SUM) {
@@ -214,19 +220,23 @@ __device__ __forceinline__ A combine_local(A a, A b, int mode) {
   if constexpr (std::is_floating_point_v<A>) return mode == GHIP_SCATTER_MAX ? max_nan(a, b) : min_nan(a, b);
   else return (mode == GHIP_SCATTER_MAX) == (a > b) ? a : b;
 }
-template <typename U, typename A>
+template <typename A>
+constexpr int kScatterRows = sizeof(A) == 8 ? 32 : 64;  // rows a wave: 64 KiB of LDS a workgroup
+template <typename U, typename A, int CW>
 __global__ void __launch_bounds__(256) scatter_groups_kernel(const U* __restrict__ upd, const void* __restrict__ idx,
                                                              A* acc, RowScatter d, int mode) {
-  __shared__ A stage[4][64][64];
+  constexpr int R = kScatterRows<A>;
+  __shared__ A stage[4][R][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t col = (static_cast<int64_t>(blockIdx.y) * 4 + w) * 64 + lane;
-  if (col - lane >= d.D) return;  // whole wave; the kernel has no barrier
+  const int64_t col = (static_cast<int64_t>(blockIdx.y) * CW + w % CW) * 64 + lane;
+  const int64_t row0 = (static_cast<int64_t>(blockIdx.x) * (4 / CW) + (CW == 4 ? 0 : __builtin_amdgcn_readfirstlane(w / CW))) * R;
+  if (col - lane >= d.D || (CW < 4 && row0 >= d.rows)) return;  // whole wave; the kernel has no barrier
   int64_t uo;
-  const int id = static_cast<int>(scatter_row(d, idx, static_cast<int64_t>(blockIdx.x) * 64 + lane, &uo));
+  const int id = static_cast<int>(scatter_row(d, idx, lane < R ? row0 + lane : d.rows, &uo));
   const U* u = upd + (col < d.D ? col : 0);
   A(*st)[64] = stage[w];
 #pragma unroll
-  for (int k0 = 0; k0 < 64; k0 += 16) {  // 16 rows' loads in flight
+  for (int k0 = 0; k0 < R; k0 += 16) {  // 16 rows' loads in flight
     U v[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
@@ -305,10 +315,17 @@ static void launch_scatter_t(const void* upd, const void* idx, void* acc, const 
     hipLaunchKernelGGL((scatter_rows_kernel<U, A, L>), dim3(static_cast<unsigned>((r.rows + 256 / L - 1) / (256 / L))),
                        dim3(256), 0, s, u, idx, a, r, mode);
   };
-  if (r.D >= 32 && r.V < (int64_t{1} << 31) && r.D <= 65535 * 256)
-    hipLaunchKernelGGL((scatter_groups_kernel<U, A>),
-                       dim3(static_cast<unsigned>((r.rows + 63) / 64), static_cast<unsigned>((r.D + 255) / 256)), dim3(256), 0,
-                       s, u, idx, a, r, mode);
+  auto groups = [&](auto cw) {
+    constexpr int CW = decltype(cw)::value, R = kScatterRows<A> * (4 / CW);
+    hipLaunchKernelGGL((scatter_groups_kernel<U, A, CW>),
+                       dim3(static_cast<unsigned>((r.rows + R - 1) / R), static_cast<unsigned>((r.D + 64 * CW - 1) / (64 * CW))),
+                       dim3(256), 0, s, u, idx, a, r, mode);
+  };
+  if (r.D >= 32 && r.rows > 4096 && r.V < (int64_t{1} << 31) && r.D <= 65535 * 64) {
+    if (r.D <= 64) groups(std::integral_constant<int, 1>{});
+    else if (r.D <= 128) groups(std::integral_constant<int, 2>{});
+    else groups(std::integral_constant<int, 4>{});
+  }
   else if (r.D >= 32) go(std::integral_constant<int, 64>{});
   else if (r.D >= 8) go(std::integral_constant<int, 16>{});
   else go(std::integral_constant<int, 4>{});

@@ -95,3 +95,22 @@ def test_fill(cuda, dt, n):
     out = torch.zeros(n + 16, device=cuda, dtype=dt)
     ops.copy(src.expand(n), out[:n])
     assert torch.all(out[:n] == src) and torch.all(out[n:] == 0)
+
+
+# Widths around the columns a workgroup takes (64, 128, 256) and row counts around the
+# rows a wave and a workgroup take, above the 4096 rows from which indices are combined.
+@pytest.mark.parametrize("D", [32, 63, 64, 65, 128, 129, 257])
+@pytest.mark.parametrize("rows", [4096, 4097, 4160, 5000])
+@pytest.mark.parametrize("mode", ["ScatterSum", "ScatterMax"])
+@pytest.mark.parametrize("dt,npt", [(F32, np.float32), (dtypes.Float64, np.float64), (I32, np.int32)])
+def test_combined_rows(be, D, rows, mode, dt, npt):
+    """Whole numbers, so sums are exact in any order; most rows name a few indices."""
+    V = 40
+    ids = np.minimum(synth.uniform_int(9501, (rows, 1), -2, V + 2), synth.uniform_int(9502, (rows, 1), -2, V + 2))
+    table = synth.uniform_int(9503, (V, D), -50, 50).astype(npt)
+    upd = synth.uniform_int(9504, (rows, 1, D), -50, 50).astype(npt)
+    print(D, rows, mode, dt, flush=True)
+    got, _ = _scatter(be, mode, dt, table, ids, upd, False)
+    want, ok = table.copy(), (ids[:, 0] >= 0) & (ids[:, 0] < V)
+    (np.add if mode == "ScatterSum" else np.maximum).at(want, ids[ok, 0], upd[ok, 0])
+    assert np.array_equal(got, want)
