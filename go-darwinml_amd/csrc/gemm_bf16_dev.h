@@ -155,21 +155,6 @@ inline GemmSplit gemm_k_split(int64_t batch, int64_t M, int64_t N, int64_t K, in
   }
   return r;
 }
-// 16-bit products for 256 x 128 tiles (gemm_bf16_body4h): grids that are one round of
-// them but more than one 128 x 128 tile per CU, with a contraction long enough to pay for
-// a prologue and an epilogue that no second workgroup hides.  Graph-replayed, us, 128 x
-// 128 core / 256 x 128: [4096,2048,8192] 127 / 108, [2304,2304,4096] 55.3 / 48.0,
-// [2048,3072,4096] 55 / 49, [4096,2048,2048] 35.0 / 33.0, but [2,2048,2048,1024] 20.4 /
-// 20.7; at 256 tiles of 128 x 128 [2048,2048,2048] 27.5 / 28.5; where 256 x 256 tiles are
-// more than 128 their cores win ([4096,4096,4096] 97 / 112).  Ragged tiles pay for the
-// masks of their loads, more so on an MN-contiguous A: [3080,2056,4096] 60.2 / 56.2, A
-// MN-contiguous 65.0 / 64.0 ([2056,2184,4096] 58.6 / 60.6), [3080,2056,2048] 33.5 / 34.6.
-inline bool gemm_half_whole(int64_t M, int64_t N, int64_t K) { return M % 256 == 0 && N % 128 == 0 && K % 64 == 0; }
-inline bool gemm_half_tiles(int64_t batch, int64_t M, int64_t N, int64_t K, bool a_k) {
-  const int64_t t128 = batch * ((M + 127) / 128) * ((N + 127) / 128);
-  const int64_t half = batch * ((M + 255) / 256) * ((N + 127) / 128);
-  return M >= 256 && t128 > 256 && half <= 256 && (gemm_half_whole(M, N, K) ? K >= 2048 : a_k && K >= 4096);
-}
 // Whether a product that gemm_k_split would split runs as its split: not where small
 // tiles, unsplit, are modelled at less than 0.8 of the split's cost.  Their cost: one
 // round of 256 tiles ~2.4 us + 4.6 ns a contraction step, two rounds ~4 + 8.3 (fp32
@@ -1642,8 +1627,9 @@ __device__ __forceinline__ void gemm_bf16_body4km(const GemmParams& p, const Epi
 // this wave's reads of stage kt % 3 have completed: wait for tile kt+1 (issued two
 // tiles earlier), barrier, refill the stage with tile kt+3 (12 DMA instructions over
 // the remaining 24 MFMAs) and read step 0 of tile kt+1.  Bit-identical to the other
-// cores (same MFMA, same k order per accumulator).
-template <bool A_K, bool B_K, class Epi, bool F16 = false>
+// cores (same MFMA, same k order per accumulator).  EDGE: ragged tiles too, which
+// gemm_half_tiles admits with a K-contiguous A alone.
+template <bool A_K, bool B_K, class Epi, bool F16 = false, bool EDGE = A_K>
 __device__ __forceinline__ void gemm_bf16_body4h(const GemmParams& p, const Epi& epi) {
   constexpr int BM = 256, BN = 128, WM = 2, WN = 2, BK = kBK;
   constexpr int NW = WM * WN, NS = 3;
@@ -1810,8 +1796,12 @@ __device__ __forceinline__ void gemm_bf16_body4h(const GemmParams& p, const Epi&
       if (kt + 2 < KT) tile(kt + 2, IntC<2>{}, BoolC<false>{});
     }
   };
-  if (mn_full && (p.K % BK) == 0) run(BoolC<true>{});
-  else run(BoolC<false>{});
+  if constexpr (EDGE) {
+    if (mn_full && (p.K % BK) == 0) run(BoolC<true>{});
+    else run(BoolC<false>{});
+  } else {
+    run(BoolC<true>{});
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   mfma_drain_a(acc);
   tile_epilogue<BM, BN, WM, WN, 1>(p, epi, smem, acc, bb, m0, n0, mn_full, lane, wm, wn);

@@ -20,6 +20,21 @@ constexpr bool gemm_small_tiles(int64_t batch, int64_t M, int64_t N, int es) {
 constexpr bool gemm_f32_tiny(int64_t batch, int64_t M, int64_t N) {
   return batch * ((M + 63) / 64) * ((N + 63) / 64) <= 128;
 }
+// 16-bit products for 256 x 128 tiles (gemm_bf16_body4h): grids that are one round of
+// them but more than one 128 x 128 tile per CU, with a contraction long enough to pay for
+// a prologue and an epilogue that no second workgroup hides.  Graph-replayed, us, 128 x
+// 128 core / 256 x 128: [4096,2048,8192] 127 / 108, [2304,2304,4096] 55.3 / 48.0,
+// [2048,3072,4096] 55 / 49, [4096,2048,2048] 35.0 / 33.0, but [2,2048,2048,1024] 20.4 /
+// 20.7; at 256 tiles of 128 x 128 [2048,2048,2048] 27.5 / 28.5; where 256 x 256 tiles are
+// more than 128 their cores win ([4096,4096,4096] 97 / 112).  Ragged tiles pay for the
+// masks of their loads, more so on an MN-contiguous A: [3080,2056,4096] 60.2 / 56.2, A
+// MN-contiguous 65.0 / 64.0 ([2056,2184,4096] 58.6 / 60.6), [3080,2056,2048] 33.5 / 34.6.
+constexpr bool gemm_half_whole(int64_t M, int64_t N, int64_t K) { return M % 256 == 0 && N % 128 == 0 && K % 64 == 0; }
+constexpr bool gemm_half_tiles(int64_t batch, int64_t M, int64_t N, int64_t K, bool a_k) {
+  const int64_t t128 = batch * ((M + 127) / 128) * ((N + 127) / 128);
+  const int64_t half = batch * ((M + 255) / 256) * ((N + 127) / 128);
+  return M >= 256 && t128 > 256 && half <= 256 && (gemm_half_whole(M, N, K) ? K >= 2048 : a_k && K >= 4096);
+}
 // Tiles of a product that only the register-staged cores can address: 64 x 64 (fp32
 // 32 x 32) for grids of few tiles, else the size whose grid is modelled fastest, since a
 // tile's cost hardly depends on how much of it lies inside the output: ns a tile of a full

@@ -3404,7 +3404,7 @@ View Lowerer::emit_gemm_epilogue(int v, const std::vector<int>& mem, bool* fused
     src << "  ghip::gemm_bf16_body8x<" << (ma ? "true" : "false") << ", " << (mb ? "true" : "false")
         << ", ghip::GenEpi, " << f16 << ", " << NB << big_arg << ">(p, epi);\n}\n";
   else if (half)
-    src << "  ghip::gemm_bf16_body4h<" << (ma ? "true" : "false") << ", " << (mb ? "true" : "false") << ", ghip::GenEpi, " << f16 << ">(p, epi);\n}\n";
+    src << "  ghip::gemm_bf16_body4h<" << (ma ? "true" : "false") << ", " << (mb ? "true" : "false") << ", ghip::GenEpi, " << f16 << ", false>(p, epi);\n}\n";
   else if (four_wave)
     src << "  ghip::gemm_bf16_body4mn<ghip::GenEpi, " << f16 << big_arg << ">(p, epi);\n}\n";
   else

@@ -32,3 +32,13 @@ def test_staged_tiles(tmp_path):
         "gemm_staged_tile(512, 100, 100, 65, 2) == 128", "gemm_staged_tile(1, 1999, 1999, 1001, 2) == 128",
         "gemm_staged_tile(1, 1000, 776, 1531, 2) == 64", "gemm_staged_tile(1, 256, 10, 512, 4) == 32",
         "gemm_staged_tile(200, 5, 5, 300, 2) == 64"])
+
+
+def test_half_tiles(tmp_path):
+    """The shapes that test the 256 x 128 core run on it: whole tiles in any layout, ragged
+    ones with a K-contiguous A alone."""
+    whole = [(1, 2048, 4096, 2048), (1, 256, 32768, 2048)]
+    ragged = [(1, 2056, 2184, 4104), (1, 4096, 1288, 4160), (2, 2048, 1152, 4232)]
+    tiles = "gemm_half_tiles({}, {}, {}, {}, {})".format
+    _check(tmp_path, "gemm_rules.h", [tiles(*s, a) for s in whole for a in ("true", "false")] +
+           [tiles(*s, "true") for s in ragged] + ["!" + tiles(*s, "false") for s in ragged])

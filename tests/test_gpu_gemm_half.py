@@ -1,6 +1,6 @@
-"""The 256 x 128 GEMM core (grids that 256 x 256 tiles leave half empty): edge tiles of
-rows and columns, contractions of whole and partial k-tiles, each operand layout, against
-the fp64 oracle on rows and columns at tile edges, and a fused epilogue against the
+"""The 256 x 128 GEMM core (grids that 256 x 256 tiles leave half empty): whole tiles in
+each operand layout and, with a K-contiguous A (others run the 128 x 128 core there),
+edge tiles of rows and columns and contractions of partial k-tiles, against the fp64 oracle on rows and columns at tile edges, and a fused epilogue against the
 unfused plan, bit for bit.  Tolerances: one rounding of a 16-bit output (half a unit in
 the last place, 2^-9 of a value in bf16 and 2^-12 in f16, values up to ~5 times the
 result's RMS), and for fp32 results the sum of K products of 16-bit operands, exact in
