@@ -528,18 +528,59 @@ struct Lowerer {
     const Kind k = N[v].kind;
     return is_elementwise(k);
   }
+  // Vector-ALU time of an elementwise node where no memory traffic hides it (the epilogue
+  // of a GEMM): us over 16M elements with 16-bit results, measured on products with such
+  // an epilogue (log1p 50, pow 88, rem 19; tanh, exp, logistic, log and sqrt nothing seen).
+  double valu_cost(int v) const {
+    const Node& n = N[v];
+    const bool wide = dtype_size(n.shape.dtype) == 8;  // fp64 and 64-bit integers: library routines
+    if (n.kind == Kind::Unary) switch (n.sub) {
+        case GHIP_UNARY_LOG1P: return 50;
+        case GHIP_UNARY_ERF: return wide ? 50 : 11;
+        case GHIP_UNARY_SIN: case GHIP_UNARY_COS: return wide ? 50 : 7;
+        case GHIP_UNARY_EXPM1: return wide ? 50 : 5;
+        case GHIP_UNARY_TANH: case GHIP_UNARY_EXP: case GHIP_UNARY_LOGISTIC: case GHIP_UNARY_LOG:
+        case GHIP_UNARY_SQRT: case GHIP_UNARY_RSQRT: return wide ? 50 : 0.5;
+      }
+    if (n.kind == Kind::Binary) switch (n.sub) {
+        case GHIP_BINARY_POW: case GHIP_BINARY_ATAN2: return 88;
+        case GHIP_BINARY_REM: return wide ? 88 : 19;
+        case GHIP_BINARY_DIV: return wide ? 50 : 9;
+      }
+    return 0.3;
+  }
+  // Whether a cluster that reads v may run in the epilogue of a GEMM: a product with 16-bit
+  // operands is read in the elementwise nodes of v's shape around its readers.
+  bool near_product(int v) const {
+    std::set<int> seen(users[v].begin(), users[v].end());
+    std::vector<int> work(seen.begin(), seen.end());
+    while (!work.empty()) {
+      const int w = work.back();
+      work.pop_back();
+      if (seen.size() > 64) return true;
+      for (int o : N[w].in) {
+        if (o < 0 || N[o].shape.dims != N[v].shape.dims) continue;
+        if (N[o].kind == Kind::Dot && dtype_size(N[N[o].in[0]].shape.dtype) == 2) return true;
+        if (o != v && is_elementwise(N[o].kind) && seen.insert(o).second) work.push_back(o);
+      }
+      for (int u : users[w])
+        if (is_elementwise(N[u].kind) && N[u].shape.dims == N[v].shape.dims && seen.insert(u).second) work.push_back(u);
+    }
+    return false;
+  }
   // Values that the clusters reading v load in its place when v is evaluated inside
   // them: v's operands, through the elementwise nodes that only v (or copied nodes)
-  // read.  False: not worth it, or too many nodes.
-  bool copy_leaves(int v, std::set<int>* leaves, int* nodes, const std::set<int>& outs) {
+  // read, whose cost adds up.  False: not worth it, or too many nodes.
+  bool copy_leaves(int v, std::set<int>* leaves, int* nodes, double* cost, const std::set<int>& outs) {
     if (++*nodes > 8) return false;
+    *cost += valu_cost(v);
     for (int p : N[v].in) {
       double c;
       if (p < 0 || scalar_const(p, &c)) continue;
       bool inside = clusterable(p) && !outs.count(p) && N[p].shape.dims == N[v].shape.dims;
       for (int w : users[p]) inside = inside && (w == v || copied[w]);
       if (inside || copied[p]) {
-        if (!copy_leaves(p, leaves, nodes, outs)) return false;
+        if (!copy_leaves(p, leaves, nodes, cost, outs)) return false;
         continue;
       }
       // A value that reaches only v is stored for v's sake alone, and a DotGeneral or
@@ -558,7 +599,12 @@ struct Lowerer {
   // reads it evaluates it itself (in registers, the same rounding: the same bits), so
   // it is neither stored nor read.  silu(x Wg) * (x Wu) and its gradient, bf16
   // [4096, 8192]: logistic, silu and the product were kernels of 20, 31 and 31 us and
-  // are one of 31.
+  // are one of 31.  The kernel and the traffic saved are worth ~22 us on 16M elements of
+  // 16 bits; evaluating the value in every reader must cost less (bf16 [4096,4096], two /
+  // four products with it in the epilogue, us, stored / copied: tanh 72 / 55, 126 / 109,
+  // sin 78 / 67, 134 / 135, erf 78 / 75, 135 / 150, log1p 96 / 124, 153 / 247, pow 115 /
+  // 229, 171 / 459).  Values of 32 bits whose readers stay elementwise kernels hide it
+  // under their traffic (pow, four readers, 507 / 423).
   void find_copied() {
     const int n = static_cast<int>(N.size());
     copied.assign(n, 0);
@@ -572,7 +618,10 @@ struct Lowerer {
       }
       std::set<int> leaves;
       int nodes = 0;
-      if (ok && several && copy_leaves(v, &leaves, &nodes, outs) && leaves.size() <= 1) copied[v] = 1;
+      double cost = 0;
+      if (!ok || !several || !copy_leaves(v, &leaves, &nodes, &cost, outs) || leaves.size() > 1) continue;
+      const double readers = static_cast<double>(std::set<int>(users[v].begin(), users[v].end()).size());
+      if (readers * cost <= 22 || (dtype_size(N[v].shape.dtype) == 4 && !near_product(v))) copied[v] = 1;
     }
   }
   void build_clusters() {

@@ -647,3 +647,26 @@ def test_split_needs_operands_the_dma_can_address(be, dt, M, K, N):
     f32 = plan_of(be, lambda f: [f.DotGeneral(f.Parameter("x", make_shape(F32, M, K)), [1], [],
                                               f.Parameter("w", make_shape(F32, K, N)), [0], [])])
     assert "split" not in f32 and "arena 0 bytes" in f32, f32
+
+
+@pytest.mark.parametrize("op,readers,copies", [
+    ("Tanh", 2, True), ("Tanh", 8, True), ("Sin", 2, True), ("Sin", 4, False), ("Erf", 2, True), ("Erf", 4, False), ("Log1p", 2, False),
+    ("Pow", 2, False), ("Tanh", 50, False)])
+def test_costly_values_are_stored_once(be, op, readers, copies):
+    """A value that several GEMM epilogues read is evaluated in each only where that costs
+    less than storing it once; an fp32 one between elementwise kernels always is."""
+    def value(f, x):
+        return f.Pow(f.Abs(x), x) if op == "Pow" else getattr(f, op)(x)
+    def products(f):
+        a, x = f.Parameter("a", make_shape(BF16, 512, 64)), f.Parameter("x", make_shape(BF16, 512, 512))
+        v = value(f, x)
+        return [f.Mul(f.DotGeneral(a, [1], [], f.Parameter(f"w{i}", make_shape(BF16, 64, 512)), [0], []), v)
+                for i in range(readers)]
+    p = plan_of(be, products)
+    assert ("fused_elementwise" not in p) == copies, p
+    def elementwise(f):
+        x = f.Parameter("x", make_shape(F32, 512, 512))
+        v = value(f, x)
+        return [f.ReduceSum(f.Mul(v, f.Parameter(f"y{i}", make_shape(F32, 512, 512))), 1) for i in range(readers)]
+    p = plan_of(be, elementwise)
+    assert p.count("(producer fused)") == readers and "fused_elementwise" not in p, p
