@@ -871,8 +871,9 @@ struct RsTile {
 };
 
 // The k loop of a register-staged core: the KF whole tiles with PD of them in flight
-// in registers ahead of two LDS stages, one barrier a tile, then the edge tiles (one
-// or two) as they come; compute(stage) runs a staged tile's MFMAs.
+// in registers ahead of two LDS stages, one barrier a tile, then the edge tiles as they
+// come (one or two; every tile where an operand of ragged width repeats along K, s_k = 0);
+// compute(stage) runs a staged tile's MFMAs.
 template <int PD, class TA, class TB, class E, class F>
 __device__ __forceinline__ void rs_main_loop(const TA& ta, const TB& tb, const E* A, const E* B, int64_t K, int KT,
                                              int KF, E* sa, E* sb, int sa_elems, int sb_elems, F compute) {

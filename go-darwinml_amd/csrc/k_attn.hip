@@ -304,7 +304,7 @@ __global__ __launch_bounds__(256, DP >= 256 ? 1 : (MK == kNoMask || MK == kKeyMa
   // tile is computed, with the per-lane mask's term (0 or -inf) added to each score: what
   // K and V hold at dropped keys (NaN, infinities) reaches the output as it does through
   // a mask that has a query axis.  f16 [8,12,1000,64], padded sequences of 500 to 1000
-  // keys, us a call: 57.4 with every lane loading its keys' mask bytes in every tile,
+  // keys, us a call (one card): 57.4 with every lane loading its keys' mask bytes in every tile,
   // 41.8 with the bits (37.2 with the tiles without a kept key left out, which loses
   // those effects).
   uint64_t* keep = nullptr;
